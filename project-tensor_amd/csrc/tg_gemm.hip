@@ -6,12 +6,13 @@
 // Block tile 128x128xBK, 256 threads = 4 wavefronts in a 2x2 grid, each wave a
 // 64x64 sub-tile = 2x2 MFMA 32x32 tiles:
 //   fp16 / bf16: v_mfma_f32_32x32x16_{f16,bf16}, BK = 32
-//   fp32:        v_mfma_f32_32x32x2_f32,        BK = 16
+//   fp32 (small products): v_mfma_f32_32x32x2_f32, BK = 16; the others: tg_gemm_rs.hip
 // Both operands are staged through LDS in k-contiguous layout (As[m][k], Bs[n][k]);
 // an operand whose global layout is contiguous along m/n is transposed while it is
 // written to LDS.  The next k-tile is fetched into registers while the current one
 // is multiplied.  Accumulation is fp32; the epilogue applies alpha/beta and converts.
 #include "tg_common.h"
+#include "tg_gemm_rs.h"
 
 #include <algorithm>
 #include <vector>
@@ -1253,7 +1254,10 @@ int gemm_dispatch(const char* who, int dtype_ab, int dtype_c, int trans_a, int t
     if (dtype_c == TG_F32) TG_GEMM_CALL(tg_bf16, float);
     if (dtype_c == TG_BF16) TG_GEMM_CALL(tg_bf16, tg_bf16);
   } else if (dtype_ab == TG_F32 && dtype_c == TG_F32) {
-    TG_GEMM_CALL(float, float);
+    if (!tg_gemm_rs_serves(M, N, K, batch)) TG_GEMM_CALL(float, float);
+    return tg_gemm_rs(tg_gemm_rs_plan(M, N, K, batch, false), trans_a, trans_b, M, N, K, alpha,
+                      (const float*)A, lda, stride_a, (const float*)B, ldb, stride_b, beta,
+                      (float*)C, ldc, stride_c, batch, bias, s);
   }
 #undef TG_GEMM_CALL
   tg_set_error("%s: unsupported dtype combination ab=%d c=%d", who, dtype_ab, dtype_c);
@@ -1262,38 +1266,45 @@ int gemm_dispatch(const char* who, int dtype_ab, int dtype_c, int trans_a, int t
 }  // namespace
 
 namespace {
-// Finishing pass of the weight-gradient entry: dW[i] (+)= sum_s parts[s][i] over the
-// M*N elements (when K was split), then db[c] (+)= sum_s bparts[s][c].  A thread owns 4
-// adjacent elements and adds the S partials in order with 4 rows of loads in flight,
-// so the result does not depend on scheduling.
+// Finishing pass of a K split: out[i] = alpha * sum_s parts[s][i] (+ bias[i % N])
+// (+ beta * out[i]) over the M*N elements (when K was split), then db[c] (+)= sum_s
+// bparts[s][c].  A thread owns 4 adjacent elements and adds the S partials in order with
+// 4 rows of loads in flight, so the result does not depend on scheduling.  Partial rows
+// are split_stride(M*N) elements apart: a multiple of 4, so the loads are aligned.
 constexpr int kFinBlock = 256;
+int64_t split_stride(int64_t n) { return (n + 3) / 4 * 4; }
 
 template <typename TO>
-__device__ __forceinline__ void fin_store(void* out, int64_t i, const float a[4], int acc) {
+__device__ __forceinline__ void fin_store(void* out, int64_t i, int64_t n, const float a[4],
+                                          float alpha, float beta, const float* bias, int64_t N) {
   TO* o = reinterpret_cast<TO*>(out) + i;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float v = a[j];
-    if (acc) v += tg_to_float(o[j]);
+    if (i + j >= n) return;
+    float v = alpha * a[j];
+    if (bias) v += bias[(i + j) % N];
+    if (beta != 0.f) v += beta * tg_to_float(o[j]);
     o[j] = tg_from_float<TO>(v);
   }
 }
 
-__global__ __launch_bounds__(kFinBlock) void k_wgrad_finish(
-    const float* __restrict__ parts, int S, int64_t MN, void* dW, int dtw, int accw,
-    const float* __restrict__ bparts, int64_t N, void* db, int dtb, int accb) {
+__global__ __launch_bounds__(kFinBlock) void k_split_finish(
+    const float* __restrict__ parts, int S, int64_t MN, int64_t N, float alpha, float beta,
+    const float* __restrict__ bias, void* out_w, int dtw, const float* __restrict__ bparts,
+    int64_t nb, void* db, int dtb, int accb) {
   const int64_t q = (int64_t)blockIdx.x * kFinBlock + threadIdx.x;
-  const int64_t qw = MN / 4;
+  const int64_t qw = (MN + 3) / 4;
   const float* in;
-  int64_t stride, i;
+  int64_t stride, i, n;
   void* out;
-  int dt, acc;
+  int dt;
   if (q < qw) {
-    in = parts, stride = MN, i = q * 4, out = dW, dt = dtw, acc = accw;
+    in = parts, stride = qw * 4, i = q * 4, n = MN, out = out_w, dt = dtw;
   } else {
     i = (q - qw) * 4;
-    if (db == nullptr || i >= N) return;
-    in = bparts, stride = N, out = db, dt = dtb, acc = accb;
+    if (i >= nb) return;
+    in = bparts, stride = nb, n = nb, out = db, dt = dtb;
+    alpha = 1.f, beta = accb ? 1.f : 0.f, bias = nullptr;
   }
   float a[4] = {0.f, 0.f, 0.f, 0.f};
   int r = 0;
@@ -1316,16 +1327,27 @@ __global__ __launch_bounds__(kFinBlock) void k_wgrad_finish(
     a[2] += v.z;
     a[3] += v.w;
   }
-  if (dt == TG_F32) fin_store<float>(out, i, a, acc);
-  else if (dt == TG_F16) fin_store<tg_half>(out, i, a, acc);
-  else fin_store<tg_bf16>(out, i, a, acc);
+  if (dt == TG_F32) fin_store<float>(out, i, n, a, alpha, beta, bias, N);
+  else if (dt == TG_F16) fin_store<tg_half>(out, i, n, a, alpha, beta, bias, N);
+  else fin_store<tg_bf16>(out, i, n, a, alpha, beta, bias, N);
 }
 
-// K split of a weight gradient whose output has too few 128x128 tiles for two per CU
+int split_finish(const char* who, const float* parts, int64_t S, int64_t MN, int64_t N,
+                 float alpha, float beta, const float* bias, void* out, int dt,
+                 const float* bparts, int64_t nb, void* db, int dtb, int accb, hipStream_t s) {
+  const int64_t groups = (MN + 3) / 4 + (nb + 3) / 4;
+  if (groups == 0) return TG_OK;
+  k_split_finish<<<(unsigned)((groups + kFinBlock - 1) / kFinBlock), kFinBlock, 0, s>>>(
+      parts, (int)S, MN, N, alpha, beta, bias, out, dt, bparts, nb, db, dtb, accb);
+  return tg_check_launch(who);
+}
+
+// K split of a 16-bit product whose output has too few 128x128 tiles for two per CU
 // (qkv/out projections [1024, 1024] and FC weights [1024, 4096] over 8192 tokens), or
-// whose K is very long: returns s with K % s == 0 and (K / s) % 64 == 0, or 1.
-int64_t wgrad_split(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N % 4 != 0) return 1;  // the finish reads 4-element groups
+// whose K is very long (the tied head's input gradient over a 32000-word vocabulary: 676
+// -> 563 us in two halves): returns s with K % s == 0 and (K / s) % 64 == 0, or 1.
+int64_t split16(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0) return 1;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   const int64_t cus = tg_num_cus();
   int64_t want;
@@ -1339,28 +1361,85 @@ int64_t wgrad_split(int64_t M, int64_t N, int64_t K) {
 
 size_t al256(size_t n) { return (n + 255) & ~size_t{255}; }
 
+// The K split of a 2-D product, and the bytes of its fp32 partial sums.
+struct SplitPlan {
+  TgRsPlan rs;       // fp32 operands
+  int64_t S, kc;     // batch entry s multiplies k in [s*kc, min(K, (s+1)*kc))
+  size_t bytes;
+};
+
+SplitPlan split_plan(int dtype_ab, int64_t M, int64_t N, int64_t K) {
+  SplitPlan p{};
+  p.S = 1, p.kc = K;
+  if (dtype_ab == TG_F32) {
+    if (!tg_gemm_rs_serves(M, N, K, 1)) return p;
+    p.rs = tg_gemm_rs_plan(M, N, K, 1, true);
+    p.S = p.rs.S, p.kc = p.rs.kc;
+  } else if (dtype_ab != TG_F64) {
+    p.S = split16(M, N, K);
+    p.kc = K / p.S;
+  }
+  if (p.S > 1) p.bytes = al256((size_t)(p.S * split_stride(M * N)) * sizeof(float));
+  return p;
+}
+
 struct WgradPlan {
-  int64_t split;
-  size_t parts, bparts, red;  // byte offsets-to-be: sizes of the three workspace regions
+  SplitPlan sp;
+  size_t bparts, red;  // sizes of the workspace regions behind the partial sums
 };
 
 WgradPlan wgrad_plan(int dtype_ab, int64_t M, int64_t N, int64_t K, bool has_b) {
-  WgradPlan p{1, 0, 0, 0};
-  if (dtype_ab != TG_F64) p.split = wgrad_split(M, N, K);
-  if (p.split > 1) p.parts = al256((size_t)(p.split * M * N) * sizeof(float));
+  WgradPlan p{split_plan(dtype_ab, M, N, K), 0, 0};
   if (has_b) {
-    p.bparts = al256((size_t)(p.split * N) * sizeof(float));
+    p.bparts = al256((size_t)(p.sp.S * N) * sizeof(float));
     p.red = al256(tg_reduce_rows_workspace(K, N));
   }
   return p;
 }
 }  // namespace
 
+TG_EXPORT size_t tg_matmul_workspace(int dtype_ab, int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return split_plan(dtype_ab, M, N, K).bytes;
+}
+
+TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int64_t M, int64_t N,
+                        int64_t K, float alpha, const void* A, int64_t lda, const void* B,
+                        int64_t ldb, const float* bias, float beta, void* C, int64_t ldc,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+  const char* who = "tg_matmul";
+  if (M > 0 && N > 0 && K > 0 && ldc == N) {  // (the split finish writes a dense C)
+    const SplitPlan p = split_plan(dtype_ab, M, N, K);
+    if (p.S > 1 && workspace_bytes >= p.bytes) {
+      TG_REQUIRE(A && B && C, "%s: null operand", who);
+      TG_REQUIRE(lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N), "%s: bad leading dim", who);
+      TG_REQUIRE(dtype_c == TG_F32 || (dtype_c == dtype_ab && dtype_ab != TG_F32),
+                 "%s: unsupported dtype combination ab=%d c=%d", who, dtype_ab, dtype_c);
+      TG_REQUIRE(workspace, "%s: null workspace", who);
+      float* parts = static_cast<float*>(workspace);
+      const int64_t sa = trans_a ? p.kc * lda : p.kc, sb = trans_b ? p.kc : p.kc * ldb;
+      const int64_t sc = split_stride(M * N);
+      hipStream_t s = tg_stream(stream);
+      const int rc =
+          dtype_ab == TG_F32
+              ? tg_gemm_rs(p.rs, trans_a, trans_b, M, N, K, 1.f, (const float*)A, lda, sa,
+                           (const float*)B, ldb, sb, 0.f, parts, N, sc, p.S, nullptr, s)
+              : gemm_dispatch(who, dtype_ab, TG_F32, trans_a, trans_b, M, N, p.kc, 1.f, A, lda, sa,
+                              B, ldb, sb, 0.f, parts, N, sc, p.S, nullptr, stream);
+      if (rc != TG_OK) return rc;
+      return split_finish(who, parts, p.S, M * N, N, alpha, beta, bias, C, dtype_c, nullptr, 0,
+                          nullptr, 0, 0, s);
+    }
+  }
+  return gemm_dispatch(who, dtype_ab, dtype_c, trans_a, trans_b, M, N, K, alpha, A, lda, 0, B, ldb,
+                       0, beta, C, ldc, 0, 1, bias, stream);
+}
+
 TG_EXPORT size_t tg_gemm_wgrad_workspace(int dtype_ab, int64_t M, int64_t N, int64_t K,
                                          int with_bias) {
   if (N <= 0 || M < 0 || K < 0) return 0;
   const WgradPlan p = wgrad_plan(dtype_ab, M, N, K, with_bias != 0);
-  return p.parts + p.bparts + p.red;
+  return p.sp.bytes + p.bparts + p.red;
 }
 
 TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const void* X,
@@ -1383,25 +1462,28 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
              "tg_gemm_wgrad: fp64 operands take fp64 gradients");
   if (K > 0) TG_REQUIRE(X && G, "tg_gemm_wgrad: null operand");
   WgradPlan p = wgrad_plan(dtype_ab, M, N, K, db != nullptr);
-  if (ldw != N) p.split = 1;  // the split finish writes a dense dW
-  TG_REQUIRE(workspace_bytes >= p.parts + p.bparts + p.red && (workspace || !p.parts),
-             "tg_gemm_wgrad: workspace of %zu bytes, need %zu", workspace_bytes,
-             p.parts + p.bparts + p.red);
+  const size_t need = p.sp.bytes + p.bparts + p.red;
+  TG_REQUIRE(workspace_bytes >= need && (workspace || !p.sp.bytes),
+             "tg_gemm_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, need);
   char* ws = static_cast<char*>(workspace);
   float* parts = reinterpret_cast<float*>(ws);
-  float* bparts = reinterpret_cast<float*>(ws + p.parts);
-  void* red = ws + p.parts + p.bparts;
+  float* bparts = reinterpret_cast<float*>(ws + p.sp.bytes);
+  void* red = ws + p.sp.bytes + p.bparts;
+  if (ldw != N && p.sp.S > 1) {  // the split finish writes a dense dW
+    p.sp.S = 1, p.sp.kc = K;
+    p.sp.rs = tg_gemm_rs_plan(M, N, K, 1, false);
+  }
   hipStream_t s = tg_stream(stream);
-  const int64_t S = p.split, kc = K / S;
+  const int64_t S = p.sp.S, kc = p.sp.kc, sc = split_stride(M * N);
   const float bw = acc_w ? 1.f : 0.f;
-  const bool fused = db && K > 0 && (dtype_ab == TG_F16 || dtype_ab == TG_BF16) &&
+  const bool fused = db && K > 0 && N % 4 == 0 && (dtype_ab == TG_F16 || dtype_ab == TG_BF16) &&
                      v3_ok(2, 1, 0, M, N, kc, X, ldx, kc * ldx, G, ldg, kc * ldg);
   int rc;
   if (fused) {
 #define TG_WG(T)                                                                              \
   if (S > 1)                                                                                  \
     rc = launch<T, float>(1, 0, M, N, kc, 1.f, X, ldx, kc * ldx, G, ldg, kc * ldg, 0.f, parts, \
-                          N, M * N, S, s, nullptr, bparts);                                   \
+                          N, sc, S, s, nullptr, bparts);                                      \
   else if (dtype_w == TG_F32)                                                                 \
     rc = launch<T, float>(1, 0, M, N, K, 1.f, X, ldx, 0, G, ldg, 0, bw, dW, ldw, 0, 1, s,       \
                           nullptr, bparts);                                                   \
@@ -1411,24 +1493,22 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
     if (dtype_ab == TG_F16) { TG_WG(tg_half); } else { TG_WG(tg_bf16); }
 #undef TG_WG
     if (rc != TG_OK) return rc;
+  } else if (S > 1 && dtype_ab == TG_F32) {
+    rc = tg_gemm_rs(p.sp.rs, 1, 0, M, N, K, 1.f, (const float*)X, ldx, kc * ldx, (const float*)G,
+                    ldg, kc * ldg, 0.f, parts, N, sc, S, nullptr, s);
+    if (rc != TG_OK) return rc;
   } else if (S > 1) {
     rc = gemm_dispatch("tg_gemm_wgrad", dtype_ab, TG_F32, 1, 0, M, N, kc, 1.f, X, ldx, kc * ldx,
-                       G, ldg, kc * ldg, 0.f, parts, N, M * N, S, nullptr, stream);
+                       G, ldg, kc * ldg, 0.f, parts, N, sc, S, nullptr, stream);
     if (rc != TG_OK) return rc;
   } else {
     rc = gemm_dispatch("tg_gemm_wgrad", dtype_ab, dtype_w, 1, 0, M, N, K, 1.f, X, ldx, 0, G, ldg,
                        0, bw, dW, ldw, 0, 1, nullptr, stream);
     if (rc != TG_OK) return rc;
   }
-  const int64_t MN = S > 1 ? M * N : 0;
-  const int64_t nb = fused ? N : 0;
-  if (MN + nb > 0) {
-    const int64_t groups = (MN + nb) / 4;
-    k_wgrad_finish<<<(unsigned)((groups + kFinBlock - 1) / kFinBlock), kFinBlock, 0, s>>>(
-        parts, (int)S, MN, dW, dtype_w, acc_w, bparts, N, fused ? db : nullptr, dtype_b, acc_b);
-    rc = tg_check_launch("tg_gemm_wgrad");
-    if (rc != TG_OK) return rc;
-  }
+  rc = split_finish("tg_gemm_wgrad", parts, S, S > 1 ? M * N : 0, N, 1.f, bw, nullptr, dW, dtype_w,
+                    bparts, fused ? N : 0, db, dtype_b, acc_b, s);
+  if (rc != TG_OK) return rc;
   if (db && !fused)
     return tg_reduce_rows(dtype_ab, G, dtype_b, db, K, N, acc_b, red, p.red, stream);
   return TG_OK;

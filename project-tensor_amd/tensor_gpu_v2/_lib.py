@@ -93,6 +93,9 @@ SIGNATURES = {
                        _i64, _i64, _f32, _vp, _i64, _i64, _i64, _vp]),
     "tg_gemm_bias": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64,
                             _vp, _vp, _i64, _vp]),
+    "tg_matmul_workspace": (_sz, [_i32, _i64, _i64, _i64]),
+    "tg_matmul": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64,
+                         _vp, _f32, _vp, _i64, _vp, _sz, _vp]),
     "tg_gemm_wgrad_workspace": (_sz, [_i32, _i64, _i64, _i64, _i32]),
     "tg_gemm_wgrad": (_i32, [_i32, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _i32, _vp, _i64, _i32,
                              _i32, _vp, _i32, _vp, _sz, _vp]),
@@ -340,7 +343,7 @@ def gemm_epilogue(epi, a, b, x, out, bias=None, beta=0.0):
         _dev(bias, "bias")
         if bias.dtype != torch.float32 or bias.numel() != N:
             raise ValueError("gemm_epilogue: bias must be fp32 [N]")
-    if _split_k(M, N, K, a.device) > 1:
+    if _matmul_ws(dtype_code(a), M, N, K):
         # the plain product would run K-split (another summation order): not fused, so
         # a fused result always equals the separate kernels' bit for bit
         return False
@@ -1200,10 +1203,14 @@ def _gemm_bias_launch(a, b, bias, out, trans_b):
     an initialised device)."""
     M, K = a.shape
     N = out.shape[1]
-    _check("tg_gemm_bias", (_lib or load()).tg_gemm_bias(
-        _TORCH_TO_CODE[a.dtype], _TORCH_TO_CODE[out.dtype], 0, 1 if trans_b else 0, M, N, K,
-        1.0, a.data_ptr(), K, b.data_ptr(), b.shape[1], bias.data_ptr(), out.data_ptr(), N,
-        stream_handle()))
+    code = _TORCH_TO_CODE[a.dtype]
+    # (16-bit forwards run unsplit: their fused-epilogue forms do)
+    nb = _matmul_ws(code, M, N, K) if code == F32 else 0
+    ws = workspace(nb, out.device) if nb else None
+    _check("tg_matmul", (_lib or load()).tg_matmul(
+        code, _TORCH_TO_CODE[out.dtype], 0, 1 if trans_b else 0, M, N, K, 1.0, a.data_ptr(), K,
+        b.data_ptr(), b.shape[1], bias.data_ptr(), 0.0, out.data_ptr(), N,
+        ws.data_ptr() if nb else None, nb, stream_handle()))
     return out
 
 
@@ -1329,42 +1336,27 @@ def wgrad_group(xs, gs, dws, acc_ws, dbs=None, acc_bs=None):
         _ptr_array(dws), na, accw, _TORCH_TO_CODE[dbt] if with_b else 0,
         _ptr_array(dbs) if with_b else None, accb, ptr(ws), ws.numel(), stream_handle()))
 
-_CUS = {}
+
+_MATMUL_WS = {}
 
 
-def _num_cus(device):
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    if idx not in _CUS:
-        _CUS[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
-    return _CUS[idx]
-
-
-def _split_k(M, N, K, device):
-    """K-split factor for GEMMs whose output has too few 128x128 tiles for two per CU
-    (e.g. weight gradients [1024, 1024] or [1024, 4096] over 8192 tokens; measured on
-    the MI355X: [1024, 4096] 102 -> 86 us with two K halves).  Returns 1 or s with
-    K % s == 0 and (K/s) % 64 == 0."""
-    tiles = ((M + 127) // 128) * ((N + 127) // 128)
-    cus = _num_cus(device)
-    if K >= 16384 and tiles < 4 * cus:
-        # very long K (the tied head's input gradient over a 32000-word vocabulary:
-        # 676 -> 563 us in two halves)
-        want = 2
-    elif tiles >= 2 * cus or K < 2048:
-        return 1
-    else:
-        want = min(-(-2 * cus // tiles), K // 1024)
-    for s_ in range(want, 1, -1):
-        if K % s_ == 0 and (K // s_) % 64 == 0:
-            return s_
-    return 1
+def _matmul_ws(code, M, N, K):
+    """Workspace bytes of tg_matmul for this dtype code and shape (0: the product runs
+    without a K split), kept by shape: training loops repeat them."""
+    key = (code, M, N, K)
+    nb = _MATMUL_WS.get(key)
+    if nb is None:
+        if len(_MATMUL_WS) > 4096:
+            _MATMUL_WS.clear()
+        nb = _MATMUL_WS[key] = load().tg_matmul_workspace(code, M, N, K)
+    return nb
 
 
 def matmul2d(a, b, out=None, trans_a=False, trans_b=False, alpha=1.0, beta=0.0, out_dtype=None):
     """out (= or +=) op(a) @ op(b) for 2-D contiguous a, b.
 
-    Output shapes with few tiles and a long K run as a K-split batched GEMM into
-    fp32 partials followed by the deterministic column-sum kernel."""
+    Output shapes with few tiles and a long K run K-split into fp32 partials, added in a
+    fixed order by a finishing launch (tg_matmul)."""
     _dev(a, "a")
     _dev(b, "b")
     M = a.shape[1] if trans_a else a.shape[0]
@@ -1380,17 +1372,20 @@ def matmul2d(a, b, out=None, trans_a=False, trans_b=False, alpha=1.0, beta=0.0, 
     if tuple(out.shape) != (M, N):
         raise ValueError(f"matmul2d: out shape {tuple(out.shape)} != {(M, N)}")
     lda, ldb = a.shape[1], b.shape[1]
-    s_ = (_split_k(M, N, K, a.device)
-          if (alpha == 1.0 and beta in (0.0, 1.0) and a.dtype != torch.float64) else 1)
-    if s_ > 1:
-        kc = K // s_
-        parts = torch.empty(s_, M, N, dtype=torch.float32, device=a.device)
-        sa = kc * M if trans_a else kc
-        sb = kc if trans_b else kc * N
-        gemm(a, b, parts, trans_a, trans_b, 1.0, 0.0, M, N, kc, lda, ldb, N, sa, sb, M * N, s_)
-        reduce_rows(parts.view(s_, M * N), out.view(M * N), beta == 1.0)
-        return out
-    return gemm(a, b, out, trans_a, trans_b, alpha, beta, M, N, K, lda, ldb, N)
+    code = dtype_code(a)
+    if code == F64:
+        return gemm(a, b, out, trans_a, trans_b, alpha, beta, M, N, K, lda, ldb, N)
+    if a.dtype != b.dtype:
+        raise TypeError(f"gemm: A and B dtypes differ ({a.dtype} vs {b.dtype})")
+    if out.dtype not in (torch.float32, a.dtype):
+        raise TypeError(f"gemm: C must be float32 or {a.dtype}, got {out.dtype}")
+    ensure_device(out.device.index)
+    nb = _matmul_ws(code, M, N, K)
+    ws = workspace(nb, out.device) if nb else None
+    _check("tg_matmul", load().tg_matmul(
+        code, dtype_code(out), int(bool(trans_a)), int(bool(trans_b)), M, N, K, float(alpha),
+        ptr(a), lda, ptr(b), ldb, None, float(beta), ptr(out), N, ptr(ws), nb, stream_handle()))
+    return out
 
 
 # ---------------------------------------------------------------- attention

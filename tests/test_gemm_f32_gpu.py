@@ -1,0 +1,117 @@
+"""fp32 products on the split-operand GEMM (tg_matmul, tg_gemm, tg_gemm_wgrad) against
+float64, at the edges of its tiles, K splits and kernels, and the operand values that its
+bf16 split cannot hold (which it computes again on the fp32 matrix cores)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def L():
+    from tensor_gpu_v2 import _lib
+    return _lib
+
+
+def _mk(g, r, c, ld=None):
+    t = torch.randn(r, ld or c, generator=g, device="cuda")
+    return t[:, :c] if ld else t
+
+
+def _check(c, a, b, what, extra=0.0):
+    """|c - a@b| within the worst case of the summation, elementwise: six MFMAs of 16
+    products each (and their finishing sums), one rounding of at most 2^-23 of
+    sum |a||b| per MFMA, and 2^-22 for the products the split leaves out."""
+    K = a.shape[1]
+    n = 6 * (K // 16 + 1) + 40
+    mag = a.double().abs() @ b.double().abs() + extra
+    err = (c.double() - (a.double() @ b.double() + extra)).abs()
+    assert bool((err <= (n * 2.0 ** -23 + 2.0 ** -22) * mag + 1e-44).all()), \
+        f"{what}: {(err / mag.clamp_min(1e-300)).max().item():.2e}"
+
+
+SHAPES = [(1, 1, 1), (5, 7, 9), (31, 33, 8), (32, 256, 784), (33, 257, 785), (64, 64, 4561),
+          (129, 65, 31), (300, 260, 97), (1000, 1000, 1000), (257, 129, 4099),
+          (4099, 4100, 33), (2050, 2100, 64), (7, 3000, 513)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_matmul_f32(cuda, M, N, K, ta, tb):
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+    a = _mk(g, K, M) if ta else _mk(g, M, K)
+    b = _mk(g, N, K) if tb else _mk(g, K, N)
+    A, B = (a.t() if ta else a), (b.t() if tb else b)
+    c = L().matmul2d(a, b, trans_a=ta, trans_b=tb)
+    _check(c, A, B, "matmul2d")
+    # unsplit, batched with a broadcast operand, accumulating
+    c2 = torch.ones(2, M, N, device="cuda")
+    L().gemm(a, b, c2, ta, tb, 1.0, 1.0, M, N, K, a.shape[1], b.shape[1], N, 0, 0, M * N, 2)
+    assert torch.equal(c2[0], c2[1])
+    _check(c2[1], A, B, "gemm", 1.0)
+    bias = torch.randn(N, generator=g, device="cuda")
+    if not ta:
+        y = torch.empty(M, N, device="cuda")
+        L().gemm_bias(a, b, bias, y, trans_b=tb)
+        assert torch.allclose(y, c + bias, rtol=1e-6, atol=1e-6 * float(c.abs().max()) + 1e-6)
+
+
+@pytest.mark.parametrize("K,M,N", [(4561, 64, 64), (130, 33, 257), (8932, 130, 70), (77, 5, 3)])
+def test_wgrad_f32(cuda, K, M, N):
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, gr = _mk(g, K, M), _mk(g, K, N)
+    dw, db = torch.ones(M, N, device="cuda"), torch.ones(N, device="cuda")
+    L().wgrad(x, gr, dw, True, db, True)
+    _check(dw, x.t(), gr, "wgrad", 1.0)
+    assert torch.allclose(db.double(), gr.double().sum(0) + 1.0, rtol=0, atol=1e-5 * K ** 0.5)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 80, 100), (600, 700, 300), (2100, 4200, 40)])
+def test_matmul_f32_misaligned_rows(cuda, M, N, K):
+    """Operands one element off 16-byte alignment with odd leading dimensions."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    buf = torch.randn(M * (K + 3) + 1, generator=g, device="cuda")[1:].view(M, K + 3)
+    b = torch.randn(K, N + 5, generator=g, device="cuda")
+    c = torch.empty(M, N, device="cuda")
+    L().gemm(buf, b, c, False, False, 1.0, 0.0, M, N, K, K + 3, N + 5, N)
+    _check(c, buf[:, :K], b[:, :N], "misaligned")
+
+
+@pytest.mark.parametrize("M,N,K", [(40, 50, 100), (700, 800, 300), (4099, 4100, 33)])
+@pytest.mark.parametrize("kind", ["inf", "nan", "tiny", "tiny_row", "huge", "overflow", "denormal"])
+def test_matmul_f32_values_outside_the_split(cuda, M, N, K, kind):
+    g = torch.Generator(device="cuda").manual_seed(11)
+    a, b = _mk(g, M, K), _mk(g, K, N)
+    if kind == "inf":
+        a[M // 2, K // 3] = float("inf")
+        b[0, N - 1] = -float("inf")
+        b[:, 3] = 0.0
+    elif kind == "nan":
+        a[M - 1, K - 1] = float("nan")
+    elif kind == "tiny":
+        a *= 1e-36
+    elif kind == "tiny_row":
+        a[M // 2] *= 1e-35
+    elif kind == "huge":
+        a[1, 2] = 3.4e38
+        b[2] *= 1e-30
+    elif kind == "overflow":
+        a[3] *= 1e30
+        b *= 1e30
+    elif kind == "denormal":
+        a[5] = 1e-40
+        b *= 1e10
+    c = L().matmul2d(a, b)
+    want = (a.double() @ b.double())
+    got, ref = c.double(), want.float().double()  # (float64 holds the products exactly enough)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) or kind == "overflow"
+    fin = torch.isfinite(ref) & (want.abs() < 1e38)
+    inf = torch.isinf(ref) & (want.abs() > 1e39)
+    if kind != "overflow":
+        assert torch.equal(got[inf], ref[inf])
+    else:
+        assert bool((~torch.isfinite(got[inf])).all())
+    mag = a.double().abs() @ b.double().abs()
+    err = (got - want).abs()
+    ok = err[fin] <= (6 * (K // 16 + 1) + K) * 2.0 ** -23 * mag[fin] + K * 1.5e-45
+    assert bool(ok.all()), f"{kind}: {(err[fin] / mag[fin]).max().item():.2e}"
