@@ -332,9 +332,11 @@ int tg_gemm_bias(int dtype_ab, int dtype_c, int trans_a, int trans_b, int64_t M,
 /* One 2-D product C = alpha*op(A)@op(B) (+ bias[n]) + beta*C: tg_gemm / tg_gemm_bias,
  * with K split over workgroups where the output alone has too few tiles to fill the
  * device (the fp32 partial sums go to the workspace and one finishing launch adds them in
- * a fixed order).  bias may be NULL.  workspace: tg_matmul_workspace(dtype_ab, M, N, K)
- * bytes, 16-byte aligned; with fewer (NULL, 0) the product runs without a split. */
-size_t tg_matmul_workspace(int dtype_ab, int64_t M, int64_t N, int64_t K);
+ * a fixed order), and 16-bit operands whose rows are no multiple of 8 elements first
+ * copied into the workspace with aligned rows.  bias may be NULL.  workspace:
+ * tg_matmul_workspace bytes, 16-byte aligned; with fewer (NULL, 0) the product runs
+ * without a split and without the copies. */
+size_t tg_matmul_workspace(int dtype_ab, int trans_a, int trans_b, int64_t M, int64_t N, int64_t K);
 int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int64_t M, int64_t N, int64_t K,
               float alpha, const void* A, int64_t lda, const void* B, int64_t ldb,
               const float* bias, float beta, void* C, int64_t ldc, void* workspace,

@@ -3,11 +3,15 @@
 // serving the matmul forward and its backward dA = dC @ B^T, dB = A^T @ dC
 // (reference: Tensor.__matmul__ and its closure, _core.py:999-1068).
 //
-// Block tile 128x128xBK, 256 threads = 4 wavefronts in a 2x2 grid, each wave a
-// 64x64 sub-tile = 2x2 MFMA 32x32 tiles:
-//   fp16 / bf16: v_mfma_f32_32x32x16_{f16,bf16}, BK = 32
-//   fp32 (small products): v_mfma_f32_32x32x2_f32, BK = 16; the others: tg_gemm_rs.hip
-// Both operands are staged through LDS in k-contiguous layout (As[m][k], Bs[n][k]);
+// fp16 / bf16 operands with 16-byte aligned rows: the DMA-staged kernels (v3_tile below);
+// rows of other lengths are first copied into aligned ones (tg_matmul).  fp32 past the
+// small products: tg_gemm_rs.hip.
+//
+// Small fp32 products, and 16-bit ones without a workspace to realign their rows (k_gemm):
+// block tile 128x128xBK, 256 threads = 4 wavefronts in a 2x2 grid, each wave a 64x64
+// sub-tile = 2x2 MFMA 32x32 tiles (16-bit: v_mfma_f32_32x32x16_{f16,bf16}, BK = 32; fp32:
+// v_mfma_f32_32x32x2_f32, BK = 16).  Both
+// operands are staged through LDS in k-contiguous layout (As[m][k], Bs[n][k]);
 // an operand whose global layout is contiguous along m/n is transposed while it is
 // written to LDS.  The next k-tile is fetched into registers while the current one
 // is multiplied.  Accumulation is fp32; the epilogue applies alpha/beta and converts.
@@ -15,6 +19,8 @@
 #include "tg_gemm_rs.h"
 
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -170,7 +176,8 @@ struct TileLoader {
 };
 
 template <typename T, typename TC, bool TA, bool TB, bool VEC>
-__global__ __launch_bounds__(kThreads) void k_gemm(int64_t M, int64_t N, int64_t K, float alpha,
+__global__ __launch_bounds__(kThreads) void k_gemm(int64_t M, int64_t N, int64_t K, int64_t ktot,
+                                                   float alpha,
                                                    const T* __restrict__ A, int64_t lda,
                                                    int64_t sa, const T* __restrict__ B,
                                                    int64_t ldb, int64_t sb, float beta,
@@ -189,6 +196,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm(int64_t M, int64_t N, int64_t
   A += bz * sa;
   B += bz * sb;
   C += bz * sc;
+  K = K < ktot - bz * K ? K : ktot - bz * K;  // (a K split's last chunk)
   const int64_t m0 = (int64_t)blockIdx.y * BM, n0 = (int64_t)blockIdx.x * BN;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
@@ -316,188 +324,6 @@ __global__ __launch_bounds__(kThreads) void k_gemm_f32_small(
   }
 }
 
-// ---------------------------------------------------------------------------
-// Pipelined kernel for fp16/bf16: block tile 128 x BN x 64 (BN = 128 or 64),
-// 4 wavefronts in a 2 x 2 grid, each owning a 64 x BN/2 sub-tile of MFMA 32x32
-// tiles; LDS double-buffered so the next k-tile's global loads overlap the
-// current MFMAs, one barrier per k-tile.  BN is chosen so the grid holds at least
-// two blocks per CU where the problem allows it.
-// LDS layout per operand:
-//   contiguous along k in memory  -> row-major [row][BK+8]: one 16-byte read per
-//                                    8-element fragment;
-//   contiguous along m/n          -> 4-k interleaved [k/4][row][4]: staged with
-//                                    8-byte writes, read as two 8-byte halves.
-// Tiles are assigned XCD-aware: dispatch i runs on XCD i % 8, so the launch index
-// is remapped to give each XCD a contiguous band of tiles (shared A rows in its L2).
-constexpr int V2_BM = 128, V2_BK = 64;
-
-template <typename T, bool KC, int ROWS>
-struct StageV2 {
-  static constexpr int NVEC = KC ? (ROWS * V2_BK) / (8 * kThreads) : 4;
-  static constexpr int UNITS = (V2_BK / 4) * (ROWS / 8);
-  static constexpr int RM_LD = V2_BK + 8;
-  static constexpr int LDS_ELEMS = KC ? ROWS * RM_LD : ROWS * V2_BK;
-  uint4 r[NVEC];
-
-  __device__ void load(const T* __restrict__ g, int64_t ld, int64_t rows_total, int64_t K,
-                       int64_t row0, int64_t k0) {
-    const int t = threadIdx.x;
-    if (KC) {
-#pragma unroll
-      for (int i = 0; i < NVEC; ++i) {
-        const int v = t + i * kThreads;
-        const int64_t row = row0 + v / (V2_BK / 8);
-        const int64_t k = k0 + (v % (V2_BK / 8)) * 8;
-        r[i] = (row < rows_total && k < K) ? *reinterpret_cast<const uint4*>(g + row * ld + k)
-                                           : make_uint4(0, 0, 0, 0);
-      }
-    } else {
-      if (t >= UNITS) return;
-      const int kg = t / (ROWS / 8), rg = t % (ROWS / 8);
-      const int64_t row = row0 + rg * 8;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t k = k0 + kg * 4 + i;
-        r[i] = (k < K && row < rows_total) ? *reinterpret_cast<const uint4*>(g + k * ld + row)
-                                           : make_uint4(0, 0, 0, 0);
-      }
-    }
-  }
-
-  __device__ void store(T* lds) const {
-    const int t = threadIdx.x;
-    if (KC) {
-#pragma unroll
-      for (int i = 0; i < NVEC; ++i) {
-        const int v = t + i * kThreads;
-        const int row = v / (V2_BK / 8), k = (v % (V2_BK / 8)) * 8;
-        *reinterpret_cast<uint4*>(lds + row * RM_LD + k) = r[i];
-      }
-    } else {
-      if (t >= UNITS) return;
-      const int kg = t / (ROWS / 8), rg = t % (ROWS / 8);
-      const T* e0 = reinterpret_cast<const T*>(&r[0]);
-      const T* e1 = reinterpret_cast<const T*>(&r[1]);
-      const T* e2 = reinterpret_cast<const T*>(&r[2]);
-      const T* e3 = reinterpret_cast<const T*>(&r[3]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        T q4[4] = {e0[j], e1[j], e2[j], e3[j]};
-        *reinterpret_cast<uint2*>(lds + (kg * ROWS + rg * 8 + j) * 4) =
-            *reinterpret_cast<const uint2*>(q4);
-      }
-    }
-  }
-
-  // 8-element fragment for `row` (tile-local) and k = ks*16 + h*8 + e.
-  __device__ __forceinline__ typename Vec8<T>::type frag(const T* lds, int row, int ks,
-                                                         int h) const {
-    union {
-      uint4 u;
-      typename Vec8<T>::type v;
-    } r;
-    if (KC) {
-      r.u = *reinterpret_cast<const uint4*>(lds + row * RM_LD + ks * 16 + h * 8);
-    } else {
-      const int g = ks * 4 + h * 2;
-      const uint2 a = *reinterpret_cast<const uint2*>(lds + (g * ROWS + row) * 4);
-      const uint2 b = *reinterpret_cast<const uint2*>(lds + ((g + 1) * ROWS + row) * 4);
-      r.u = make_uint4(a.x, a.y, b.x, b.y);
-    }
-    return r.v;
-  }
-};
-
-template <typename T, typename TC, bool TA, bool TB, int BNv>
-__global__ __launch_bounds__(kThreads) void k_gemm_v2(int64_t M, int64_t N, int64_t K, float alpha,
-                                                      const T* __restrict__ A, int64_t lda,
-                                                      int64_t sa, const T* __restrict__ B,
-                                                      int64_t ldb, int64_t sb, float beta,
-                                                      TC* __restrict__ C, int64_t ldc, int64_t sc,
-    const float* __restrict__ bias) {
-  constexpr int NTW = BNv / 64;  // 32-wide MFMA tiles per wave along n
-  using SA = StageV2<T, !TA, V2_BM>;
-  using SB = StageV2<T, TB, BNv>;
-  __shared__ __attribute__((aligned(16))) T As[2][SA::LDS_ELEMS];
-  __shared__ __attribute__((aligned(16))) T Bs[2][SB::LDS_ELEMS];
-
-  const int64_t gx = gridDim.x, gy = gridDim.y;
-  const int64_t T_ = gx * gy;
-  int64_t lin = (int64_t)blockIdx.y * gx + blockIdx.x;
-  if (T_ % 8 == 0) lin = (lin % 8) * (T_ / 8) + lin / 8;
-  const int64_t tm = lin / gx, tn = lin % gx;
-  const int64_t bz = blockIdx.z;
-  A += bz * sa;
-  B += bz * sb;
-  C += bz * sc;
-  const int64_t m0 = tm * V2_BM, n0 = tn * BNv;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * (BNv / 2);
-  const int lr = lane & 31, lh = lane >> 5;
-
-  f32x16 acc[2][NTW];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < NTW; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  SA sa_;
-  SB sb_;
-  sa_.load(A, lda, M, K, m0, 0);
-  sb_.load(B, ldb, N, K, n0, 0);
-  sa_.store(As[0]);
-  sb_.store(Bs[0]);
-  __syncthreads();
-  int cur = 0;
-  for (int64_t k0 = 0; k0 < K; k0 += V2_BK) {
-    const bool more = k0 + V2_BK < K;
-    if (more) {
-      sa_.load(A, lda, M, K, m0, k0 + V2_BK);
-      sb_.load(B, ldb, N, K, n0, k0 + V2_BK);
-    }
-#pragma unroll
-    for (int ks = 0; ks < V2_BK / 16; ++ks) {
-      typename Vec8<T>::type af[2], bfr[NTW];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = sa_.frag(As[cur], wm + i * 32 + lr, ks, lh);
-#pragma unroll
-      for (int j = 0; j < NTW; ++j) bfr[j] = sb_.frag(Bs[cur], wn + j * 32 + lr, ks, lh);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < NTW; ++j) mfma_v(af[i], bfr[j], acc[i][j]);
-    }
-    if (more) {
-      sa_.store(As[cur ^ 1]);
-      sb_.store(Bs[cur ^ 1]);
-    }
-    __syncthreads();
-    cur ^= 1;
-  }
-
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-      const int64_t col = n0 + wn + j * 32 + lr;
-      if (col >= N) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row = m0 + wm + i * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
-        if (row < M) {
-          float v = alpha * acc[i][j][r];
-          if (bias) v += bias[col];
-          TC* pc = C + row * ldc + col;
-          if (beta != 0.f) v += beta * tg_to_float(*pc);
-          *pc = tg_from_float<TC>(v);
-        }
-      }
-    }
-}
-
-
 // ---------------------------------------------------------------------------- v3
 // fp16/bf16 GEMM with DMA-staged operands: 128x128 block tile, k-tiles of 64, four
 // waves in a 2x2 grid each owning 64x64 of C (2x2 MFMA 32x32x16 tiles).  Both
@@ -510,9 +336,10 @@ __global__ __launch_bounds__(kThreads) void k_gemm_v2(int64_t M, int64_t N, int6
 //   m/n-contiguous operand (A^T, or B): [64 k][128 cols], fragments are two
 //     ds_read_b64_tr_b16 reads (lane = column, 4 consecutive k each).
 // Rows are unpadded with the 16-byte chunks XOR-swizzled by the row index, so both
-// read kinds are free of LDS bank conflicts.  Requires K % 64 == 0 and 16-byte
-// aligned operands; rows/columns past M or N read clamped addresses and only feed
-// C entries that are never stored.
+// read kinds are free of LDS bank conflicts.  Requires 16-byte aligned rows and whole
+// 8-element chunks along each operand's contiguous dimension; rows/columns past M or N
+// read clamped addresses and only feed C entries that are never stored, k past K reads
+// as zero.
 typedef short v4i16_g __attribute__((ext_vector_type(4)));
 #define TG_LDS_G __attribute__((address_space(3)))
 #define TG_GLB_G __attribute__((address_space(1)))
@@ -543,7 +370,7 @@ template <int CH> __device__ __forceinline__ int v3_off(int r, int c) {
 // are k, the column is m or n).  The clamp of rows or columns past the matrix edge
 // therefore depends only on the block, so each lane's byte offset within a tile is
 // computed once; a tile then costs one uniform pointer per wave instruction.  The
-// k extent needs no clamp (K % 64 == 0).
+// k extent needs a mask in the last tile only (copy_tail).
 template <typename T, int R, int CW, int NW, bool KROWS>
 struct V3Dma {
   static constexpr int CH = CW / 8, NI = R * CH / 64, NPW = NI / NW;
@@ -585,6 +412,26 @@ struct V3Dma {
     for (int k = 0; k < NPW; ++k)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TG_LDS_G void*)(lds + (wave + k * NW) * 1024),
                                                16, off[k], soff, 0, 0);
+#endif
+  }
+  // Copy of the last, partial tile: lanes whose k is not among the kleft left write zeros
+  // themselves.
+  __device__ __forceinline__ void copy_tail(const T* base, uint32_t soff, char* lds,
+                                            int64_t kleft) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(base), (short)0, 0x7fffffff, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < NPW; ++k) {
+      const int u = (wave + k * NW) * 64 + lane;
+      const int r = u / CH, c = (u % CH) ^ v3_key<CH>(r);
+      char* dst = lds + (wave + k * NW) * 1024;
+      if ((KROWS ? r : c * 8) < kleft)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TG_LDS_G void*)dst, 16, off[k], soff, 0, 0);
+      else
+        *reinterpret_cast<uint4*>(dst + lane * 16) = make_uint4(0, 0, 0, 0);
+    }
 #endif
   }
   // Instruction k of copy() alone, so a caller can spread a tile's copy over its MFMAs.
@@ -690,10 +537,12 @@ __device__ __forceinline__ float epi_val(float v, float x, float beta, float c) 
   return v;
 }
 
+// TAIL: K may end inside a k-tile (its own instantiation: the extra path costs the others
+// about 1 %).
 // EXT: the caller names the tile (row tile xtm, column tile xtn); otherwise it follows
 // from the block index, XCD-banded.
 template <typename T, typename TC, bool TA, bool TB, int WGM, int WGN, int SM, int SN, int OCC,
-          bool BSUM, int EPI = EPI_NONE, bool EXT = false>
+          bool BSUM, int EPI = EPI_NONE, bool EXT = false, bool TAIL = false>
 __device__ __forceinline__ void v3_tile(
     int64_t M, int64_t N, int64_t K, float alpha, const T* __restrict__ A, int64_t lda,
     const T* __restrict__ B, int64_t ldb, float beta, TC* __restrict__ C, int64_t ldc,
@@ -738,8 +587,9 @@ __device__ __forceinline__ void v3_tile(
   // at (row k0, column m0|n0); the clamps at the M / N edge are per block.
   V3Dma<T, AKC ? TBM : 64, AKC ? 64 : TBM, NW, !AKC> da;
   V3Dma<T, BKC ? TBN : 64, BKC ? 64 : TBN, NW, !BKC> db;
-  da.init(lda, m0, M);
-  db.init(ldb, n0, N);
+  // (a padded operand's columns reach past M or N to the end of the last chunk)
+  da.init(lda, m0, AKC ? M : (M + 7) / 8 * 8);
+  db.init(ldb, n0, BKC ? N : (N + 7) / 8 * 8);
   const T* a_org = A + (AKC ? m0 * lda : m0);
   const T* b_org = B + (BKC ? n0 * ldb : n0);
   auto dma = [&](int64_t k0, char* as, char* bs) {
@@ -818,18 +668,39 @@ __device__ __forceinline__ void v3_tile(
       }
     }
   };
-  if (K > 0) dma(0, a0, b0);
-  for (int64_t k0 = 0; k0 < K; k0 += 2 * V3_BK) {
+  // The full tiles, then the partial one, whose copy goes out beside the last full tile.
+  const int64_t kf = TAIL ? K & ~(int64_t)(V3_BK - 1) : K;
+  auto dma_tail = [&](char* as, char* bs) {
+    if (!TAIL || kf == K) return;
+    da.copy_tail(a_org, (uint32_t)((AKC ? kf : kf * lda) * (int64_t)sizeof(T)), as, K - kf);
+    db.copy_tail(b_org, (uint32_t)((BKC ? kf : kf * ldb) * (int64_t)sizeof(T)), bs, K - kf);
+  };
+  bool odd = false;  // the partial tile is in a1, b1
+  if (kf > 0) dma(0, a0, b0);
+  else dma_tail(a0, b0);
+  for (int64_t k0 = 0; k0 < kf; k0 += 2 * V3_BK) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const bool more1 = k0 + V3_BK < K;
+    const bool more1 = k0 + V3_BK < kf;
+    if (!more1) dma_tail(a1, b1);
     mul(a0, b0, more1, k0 + V3_BK, a1, b1);
-    if (!more1) break;
+    if (!more1) {
+      odd = true;
+      break;
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const bool more2 = k0 + 2 * V3_BK < K;
+    const bool more2 = k0 + 2 * V3_BK < kf;
+    if (!more2) dma_tail(a0, b0);
     mul(a1, b1, more2, k0 + 2 * V3_BK, a0, b0);
     if (!more2) break;
+  }
+  if constexpr (TAIL) {
+    if (kf < K) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      mul(odd ? a1 : a0, odd ? b1 : b0, false, 0, a0, b0);
+    }
   }
   if constexpr (BSUM) {
     if (tm == 0 && wm == 0) {
@@ -978,14 +849,16 @@ __device__ __forceinline__ void v3_tile(
 }
 
 template <typename T, typename TC, bool TA, bool TB, int WGM, int WGN, int SM, int SN, int OCC,
-          bool BSUM = false>
+          bool TAIL, bool BSUM = false>
 __global__ __launch_bounds__(64 * WGM * WGN, OCC) void k_gemm_v3(
-    int64_t M, int64_t N, int64_t K, float alpha, const T* __restrict__ A, int64_t lda,
+    int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha, const T* __restrict__ A, int64_t lda,
     int64_t sa, const T* __restrict__ B, int64_t ldb, int64_t sb, float beta,
     TC* __restrict__ C, int64_t ldc, int64_t sc,
     const float* __restrict__ bias, float* __restrict__ bsum) {
   const int64_t bz = blockIdx.z;
-  v3_tile<T, TC, TA, TB, WGM, WGN, SM, SN, OCC, BSUM>(
+  // (a K split: the last entry's chunk is what is left of the whole extent ktot)
+  K = K < ktot - bz * K ? K : ktot - bz * K;
+  v3_tile<T, TC, TA, TB, WGM, WGN, SM, SN, OCC, BSUM, EPI_NONE, false, TAIL>(
       M, N, K, alpha, A + bz * sa, lda, B + bz * sb, ldb, beta, C + bz * sc, ldc, bias,
       BSUM ? bsum + bz * N : nullptr, nullptr, 0, false);
 }
@@ -1022,7 +895,7 @@ struct V3Group {
   unsigned dbacc;       // bit g: add member g's column sums to db's contents
 };
 
-template <typename T, typename TC, int WGM, int WGN, int SM, int SN, bool BSUM>
+template <typename T, typename TC, int WGM, int WGN, int SM, int SN, bool TAIL, bool BSUM>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void k_gemm_v3g(
     int64_t M, int64_t K, int64_t lda, const V3Group<T, TC> g, int dbt) {
   constexpr int TBN = WGN * SN * 32;
@@ -1035,7 +908,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void k_gemm_v3g(
   const int loc = lin - g.tiles[bz];
   const int64_t N = g.N[bz], gx = (N + TBN - 1) / TBN;
   // (one v3_tile instance per kernel: each holds its own static LDS stages)
-  v3_tile<T, TC, true, false, WGM, WGN, SM, SN, 1, BSUM, EPI_NONE, true>(
+  v3_tile<T, TC, true, false, WGM, WGN, SM, SN, 1, BSUM, EPI_NONE, true, TAIL>(
       M, N, K, 1.f, g.A[bz], lda, g.B[bz], g.ldb[bz], g.beta[bz], g.C[bz], g.ldc[bz], nullptr,
       nullptr,
       g.db[bz], dbt, (g.dbacc >> bz) & 1u, nullptr, 0, loc / gx, loc % gx);
@@ -1046,8 +919,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void k_gemm_v3g(
 // one such tile per CU, else 2 x 2 waves (128 x 128, two blocks per CU).
 
 // Whether a 16-bit GEMM runs on the DMA-staged kernel (k_gemm_v3).
+// padded: rows are padded to whole 8-element chunks, readable and zero behind their end.
 bool v3_ok(int elem, int ta, int tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
-           int64_t sa, const void* B, int64_t ldb, int64_t sb) {
+           int64_t sa, const void* B, int64_t ldb, int64_t sb, bool padded = false) {
   const int VE = 16 / elem;
   const bool vec = tg_aligned16(A) && tg_aligned16(B) && lda % VE == 0 && ldb % VE == 0 &&
                    sa % VE == 0 && sb % VE == 0;
@@ -1056,109 +930,68 @@ bool v3_ok(int elem, int ta, int tb, int64_t M, int64_t N, int64_t K, const void
   // of its rows plus K elements from there, an m/n-contiguous one all K of its rows.
   const int64_t a_span = (ta ? K * lda : 256 * lda + K) * (int64_t)elem;
   const int64_t b_span = (tb ? 256 * ldb + K : K * ldb) * (int64_t)elem;
-  return elem == 2 && vec && M >= 64 && N >= 64 && K >= 64 && M % 8 == 0 && N % 8 == 0 &&
-         K % V3_BK == 0 && a_span < (int64_t{1} << 31) && b_span < (int64_t{1} << 31);
+  // Whole 8-element chunks along each contiguous dimension: K of a k-contiguous operand,
+  // M of a transposed A, N of a plain B.
+  const bool chunks = padded || ((ta || K % 8 == 0) && (!tb || K % 8 == 0) && (!ta || M % 8 == 0) &&
+                      (tb || N % 8 == 0));
+  return elem == 2 && vec && chunks && M > 0 && N > 0 && K > 0 && a_span < (int64_t{1} << 31) &&
+         b_span < (int64_t{1} << 31);
 }
 
-// bsum (non-null only where v3_ok holds, with ta = 1, tb = 0): also write the column
-// sums of B over each batch entry's K range to bsum[batch][N].
+// Block shape and K split of a 16-bit product: the fastest by the times (us) measured per
+// 64-deep k-tile with every CU busy: 256x256 blocks (4x2 waves of 64x128) 1.85,
+// 256x128 (4x2 of 64x64) 1.02, both one block per CU; 128x128 (2x2 of 64x64) 1.08 with
+// two blocks per CU, 0.75 with one; a block's start and store take 4-6.  A K split (chunks
+// of a multiple of 64) adds its finishing launch: 6 us and its traffic at 4.5 TB/s.
+// (256x256 as 2x2 waves of 128x128, one wave per SIMD, measured 3-8 % slower: nothing
+// overlaps a wave's LDS waits and barrier.)
+struct V3Plan {
+  int shape;      // 2: 256x256, 1: 256x128, 0: 128x128
+  int64_t S, kc;
+};
+V3Plan v3_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool can_split) {
+  V3Plan best{0, 1, K};
+  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
+  const double ncu = (double)tg_num_cus();
+  const auto tiles = [&](int64_t bm, int64_t bn) {
+    return (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
+  };
+  double tbest = 1e30;
+  // (K below 2048 stays whole, so such a product's rows do not depend on how many there are)
+  for (int64_t S = 1; S <= (can_split && K >= 2048 ? 32 : 1); S *= 2) {
+    const int64_t kc = S == 1 ? K : ((K + S - 1) / S + 63) / 64 * 64;
+    if (S > 1 && (kc < 256 || (K + kc - 1) / kc != S)) continue;
+    // (a split's partial sums stay within 256 MiB)
+    if (S > 1 && (double)S * (double)M * (double)N * 4.0 > 268435456.0) break;
+    const double kt = (double)((kc + 63) / 64);
+    const double fin = S > 1 ? 6.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 4.5e6 : 0.0;
+    double t[3];
+    t[2] = std::ceil(tiles(256, 256) * S / ncu) * (kt * 1.85 + 6.0);
+    t[1] = std::ceil(tiles(256, 128) * S / ncu) * (kt * 1.02 + 5.0);
+    const double b = tiles(128, 128) * S, pairs = std::floor(b / (2 * ncu));
+    const double rest = b - pairs * 2 * ncu;
+    t[0] = pairs * (kt * 1.08 + 4.0) + (rest > 0 ? kt * (rest > ncu ? 1.08 : 0.75) + 4.0 : 0.0);
+    for (int i = 2; i >= 0; --i)
+      if (t[i] + fin < tbest) {
+        tbest = t[i] + fin;
+        best = V3Plan{i, S, kc};
+      }
+  }
+  return best;
+}
+
 template <typename T, typename TC>
-int launch(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void* A,
-           int64_t lda, int64_t sa, const void* B, int64_t ldb, int64_t sb, float beta, void* C,
-           int64_t ldc, int64_t sc, int64_t batch, hipStream_t s, const float* bias = nullptr,
-           float* bsum = nullptr) {
+int launch_generic(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha,
+                   const T* a, int64_t lda, int64_t sa, const T* b, int64_t ldb, int64_t sb,
+                   float beta, TC* c, int64_t ldc, int64_t sc, int64_t batch, const float* bias,
+                   hipStream_t s) {
   constexpr int VE = 16 / sizeof(T);
-  const bool vec = tg_aligned16(A) && tg_aligned16(B) && lda % VE == 0 && ldb % VE == 0 &&
+  const bool vec = tg_aligned16(a) && tg_aligned16(b) && lda % VE == 0 && ldb % VE == 0 &&
                    sa % VE == 0 && sb % VE == 0;
   dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM), (unsigned)batch);
-  const T* a = (const T*)A;
-  const T* b = (const T*)B;
-  TC* c = (TC*)C;
-  // v2 stages whole 16-byte vectors along every contiguous dimension: extents must be
-  // multiples of 8 so no vector straddles a row end.
-  if (bsum && !(ta && !tb && v3_ok((int)sizeof(T), ta, tb, M, N, K, A, lda, sa, B, ldb, sb))) {
-    tg_set_error("tg_gemm: fused column sums need the DMA-staged 16-bit kernel");
-    return TG_ERR_UNSUPPORTED;
-  }
-  if constexpr (sizeof(T) == 2) {
-  if (v3_ok((int)sizeof(T), ta, tb, M, N, K, A, lda, sa, B, ldb, sb)) {
-    // Block shapes (waves x per-wave tile): 4x2 waves of 64x128 (256x256, one block
-    // and two waves per SIMD) when the problem has enough such tiles to fill the CUs:
-    // fewer global tile bytes per flop than the smaller shapes.  (The same tile as 2x2
-    // waves of 128x128, one wave per SIMD, measured 3-8 % slower: nothing overlaps a
-    // wave's LDS waits and barrier.)  Else 4x2 waves of 64x64 (256x128), else 2x2
-    // waves of 64x64 (128x128, two blocks per CU).
-    const int64_t ncu = tg_num_cus();
-    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256) * batch;
-    const int64_t t128 = ((M + 255) / 256) * ((N + 127) / 128) * batch;
-    const int shape = t256 >= kHugeTiles * ncu / 4 ? 2 : (t128 >= ncu ? 1 : 0);
-#define TG_G3_SHAPE(TA_, TB_, WGM, WGN, SM, SN, OCC)                                       \
-  do {                                                                                     \
-    constexpr int TBM = WGM * SM * 32, TBN = WGN * SN * 32;                                \
-    dim3 g3((unsigned)((N + TBN - 1) / TBN), (unsigned)((M + TBM - 1) / TBM), (unsigned)batch); \
-    if constexpr (TA_ && !TB_) {                                                           \
-      if (bsum) {                                                                          \
-        k_gemm_v3<T, TC, TA_, TB_, WGM, WGN, SM, SN, OCC, true><<<g3, 64 * WGM * WGN, 0, s>>>( \
-            M, N, K, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, bias, bsum);          \
-        break;                                                                             \
-      }                                                                                    \
-    }                                                                                      \
-    k_gemm_v3<T, TC, TA_, TB_, WGM, WGN, SM, SN, OCC><<<g3, 64 * WGM * WGN, 0, s>>>(        \
-        M, N, K, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, bias, nullptr);           \
-  } while (0)
-#define TG_G3(TA_, TB_)                                          \
-  do {                                                           \
-    if (shape == 2) TG_G3_SHAPE(TA_, TB_, 4, 2, 2, 4, 1);        \
-    else if (shape == 1) TG_G3_SHAPE(TA_, TB_, kBigWGM, kBigWGN, kBigSM, kBigSN, 1); \
-    else TG_G3_SHAPE(TA_, TB_, 2, 2, 2, 2, 2);                   \
-  } while (0)
-    if (!ta && !tb) TG_G3(false, false);
-    else if (!ta && tb) TG_G3(false, true);
-    else if (ta && !tb) TG_G3(true, false);
-    else TG_G3(true, true);
-#undef TG_G3_SHAPE
-#undef TG_G3
-    return tg_check_launch("tg_gemm");
-  }
-  if (vec && M >= 128 && N >= 64 && K >= 64 && M % 8 == 0 && N % 8 == 0 && K % 8 == 0) {
-    // BN = 128 unless that leaves fewer than two blocks per CU.
-    const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
-    const bool wide = tiles128 >= 2 * (int64_t)tg_num_cus() && N >= 128;
-    const int bn = wide ? 128 : 64;
-    dim3 g2((unsigned)((N + bn - 1) / bn), (unsigned)((M + V2_BM - 1) / V2_BM), (unsigned)batch);
-#define TG_G2(TA_, TB_)                                                                        \
-  do {                                                                                         \
-    if (wide)                                                                                  \
-      k_gemm_v2<T, TC, TA_, TB_, 128><<<g2, kThreads, 0, s>>>(M, N, K, alpha, a, lda, sa, b,    \
-                                                              ldb, sb, beta, c, ldc, sc, bias); \
-    else                                                                                       \
-      k_gemm_v2<T, TC, TA_, TB_, 64><<<g2, kThreads, 0, s>>>(M, N, K, alpha, a, lda, sa, b, ldb, \
-                                                             sb, beta, c, ldc, sc, bias);    \
-  } while (0)
-    if (!ta && !tb) TG_G2(false, false);
-    else if (!ta && tb) TG_G2(false, true);
-    else if (ta && !tb) TG_G2(true, false);
-    else TG_G2(true, true);
-#undef TG_G2
-    return tg_check_launch("tg_gemm");
-  }
-  }
-  if constexpr (sizeof(T) == 4) {
-    // fewer 128 x 128 tiles than a quarter of the CUs: 32 x 32 tiles, K in four
-    if ((int64_t)grid.x * grid.y * grid.z * 4 < (int64_t)tg_num_cus() && K >= 64) {
-      dim3 gs((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)batch);
-#define TG_GS(TA_, TB_) \
-  k_gemm_f32_small<TC, TA_, TB_><<<gs, kThreads, 0, s>>>(M, N, K, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, bias)
-      if (!ta && !tb) TG_GS(false, false);
-      else if (!ta && tb) TG_GS(false, true);
-      else if (ta && !tb) TG_GS(true, false);
-      else TG_GS(true, true);
-#undef TG_GS
-      return tg_check_launch("tg_gemm");
-    }
-  }
-#define TG_G(TA_, TB_, V_) \
-  k_gemm<T, TC, TA_, TB_, V_><<<grid, kThreads, 0, s>>>(M, N, K, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, bias)
+#define TG_G(TA_, TB_, V_)                                                                  \
+  k_gemm<T, TC, TA_, TB_, V_><<<grid, kThreads, 0, s>>>(M, N, K, ktot, alpha, a, lda, sa, b, ldb, \
+                                                        sb, beta, c, ldc, sc, bias)
   if (vec) {
     if (!ta && !tb) TG_G(false, false, true);
     else if (!ta && tb) TG_G(false, true, true);
@@ -1174,6 +1007,86 @@ int launch(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const v
   return tg_check_launch("tg_gemm");
 }
 
+// Small fp32 products (see tg_gemm_rs_serves).
+int launch_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const float* a,
+               int64_t lda, int64_t sa, const float* b, int64_t ldb, int64_t sb, float beta,
+               float* c, int64_t ldc, int64_t sc, int64_t batch, hipStream_t s,
+               const float* bias) {
+  dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((M + BM - 1) / BM), (unsigned)batch);
+  // fewer 128 x 128 tiles than a quarter of the CUs: 32 x 32 tiles, K in four
+  if ((int64_t)grid.x * grid.y * grid.z * 4 < (int64_t)tg_num_cus() && K >= 64) {
+    dim3 gs((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)batch);
+#define TG_GS(TA_, TB_) \
+  k_gemm_f32_small<float, TA_, TB_><<<gs, kThreads, 0, s>>>(M, N, K, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, bias)
+    if (!ta && !tb) TG_GS(false, false);
+    else if (!ta && tb) TG_GS(false, true);
+    else if (ta && !tb) TG_GS(true, false);
+    else TG_GS(true, true);
+#undef TG_GS
+    return tg_check_launch("tg_gemm");
+  }
+  return launch_generic<float, float>(ta, tb, M, N, K, INT64_MAX, alpha, a, lda, sa, b, ldb, sb,
+                                      beta, c, ldc, sc, batch, bias, s);
+}
+
+// bsum (non-null only where v3_ok holds, with ta = 1, tb = 0): also write the column
+// sums of B over each batch entry's K range to bsum[batch][N].
+template <typename T, typename TC>
+int launch(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const void* A,
+           int64_t lda, int64_t sa, const void* B, int64_t ldb, int64_t sb, float beta, void* C,
+           int64_t ldc, int64_t sc, int64_t batch, hipStream_t s, const float* bias = nullptr,
+           float* bsum = nullptr, int64_t ktot = INT64_MAX, bool padded = false) {
+  const T* a = (const T*)A;
+  const T* b = (const T*)B;
+  TC* c = (TC*)C;
+  if (bsum &&
+      !(ta && !tb && v3_ok((int)sizeof(T), ta, tb, M, N, K, A, lda, sa, B, ldb, sb, padded))) {
+    tg_set_error("tg_gemm: fused column sums need the DMA-staged 16-bit kernel");
+    return TG_ERR_UNSUPPORTED;
+  }
+  if (v3_ok((int)sizeof(T), ta, tb, M, N, K, A, lda, sa, B, ldb, sb, padded)) {
+    const int shape = v3_plan(M, N, K, batch, false).shape;
+    // some batch entry's K ends inside a k-tile
+    const bool ragged = K % V3_BK || (ktot != INT64_MAX && ktot % V3_BK);
+#define TG_G3_RUN(TA_, TB_, WGM, WGN, SM, SN, OCC, TAIL)                                     \
+  do {                                                                                       \
+    if constexpr (TA_ && !TB_) {                                                             \
+      if (bsum) {                                                                            \
+        k_gemm_v3<T, TC, TA_, TB_, WGM, WGN, SM, SN, OCC, TAIL, true>                         \
+            <<<g3, 64 * WGM * WGN, 0, s>>>(M, N, K, ktot, alpha, a, lda, sa, b, ldb, sb, beta, \
+                                           c, ldc, sc, bias, bsum);                          \
+        break;                                                                               \
+      }                                                                                      \
+    }                                                                                        \
+    k_gemm_v3<T, TC, TA_, TB_, WGM, WGN, SM, SN, OCC, TAIL><<<g3, 64 * WGM * WGN, 0, s>>>(     \
+        M, N, K, ktot, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc, sc, bias, nullptr);        \
+  } while (0)
+#define TG_G3_SHAPE(TA_, TB_, WGM, WGN, SM, SN, OCC)                                         \
+  do {                                                                                       \
+    constexpr int TBM = WGM * SM * 32, TBN = WGN * SN * 32;                                  \
+    dim3 g3((unsigned)((N + TBN - 1) / TBN), (unsigned)((M + TBM - 1) / TBM), (unsigned)batch); \
+    if (ragged) TG_G3_RUN(TA_, TB_, WGM, WGN, SM, SN, OCC, true);                            \
+    else TG_G3_RUN(TA_, TB_, WGM, WGN, SM, SN, OCC, false);                                  \
+  } while (0)
+#define TG_G3(TA_, TB_)                                          \
+  do {                                                           \
+    if (shape == 2) TG_G3_SHAPE(TA_, TB_, 4, 2, 2, 4, 1);        \
+    else if (shape == 1) TG_G3_SHAPE(TA_, TB_, kBigWGM, kBigWGN, kBigSM, kBigSN, 1); \
+    else TG_G3_SHAPE(TA_, TB_, 2, 2, 2, 2, 2);                   \
+  } while (0)
+    if (!ta && !tb) TG_G3(false, false);
+    else if (!ta && tb) TG_G3(false, true);
+    else if (ta && !tb) TG_G3(true, false);
+    else TG_G3(true, true);
+#undef TG_G3_SHAPE
+#undef TG_G3_RUN
+#undef TG_G3
+    return tg_check_launch("tg_gemm");
+  }
+  return launch_generic<T, TC>(ta, tb, M, N, K, ktot, alpha, a, lda, sa, b, ldb, sb, beta, c, ldc,
+                               sc, batch, bias, s);
+}
+
 // The fused-epilogue GEMMs on the DMA-staged kernel: GELU backward as C (+)= ...
 // (A [M,K], op(B) = B^T with B [N,K]: a Linear layer's input gradient G W^T), GELU
 // forward and residual as C = A B + bias (B [K,N]: a Linear layer's forward).  Other
@@ -1184,15 +1097,13 @@ int launch_epi(int epi, int64_t M, int64_t N, int64_t K, const void* A, int64_t 
                void* X, int64_t ldx, hipStream_t s) {
   const int tb = epi == EPI_GELU_BWD;
   const int VE = 16 / (int)sizeof(T);
-  if (!v3_ok((int)sizeof(T), 0, tb, M, N, K, A, lda, 0, B, ldb, 0) || !tg_aligned16(C) ||
+  if (K % V3_BK || N < 64 || N % 8 ||
+      !v3_ok((int)sizeof(T), 0, tb, M, N, K, A, lda, 0, B, ldb, 0) || !tg_aligned16(C) ||
       !tg_aligned16(X) || ldc % VE || ldx % VE || (epi == EPI_GELU_BWD && bias)) {
     tg_set_error("tg_gemm_epilogue: shape or alignment outside the fused kernel");
     return TG_ERR_UNSUPPORTED;
   }
-  const int64_t ncu = tg_num_cus();
-  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
-  const int64_t t128 = ((M + 255) / 256) * ((N + 127) / 128);
-  const int shape = t256 >= kHugeTiles * ncu / 4 ? 2 : (t128 >= ncu ? 1 : 0);
+  const int shape = v3_plan(M, N, K, 1, false).shape;
   const T* a = (const T*)A;
   const T* b = (const T*)B;
 #define TG_GE(TB_, E, WGM, WGN, SM, SN, OCC)                                                   \
@@ -1223,7 +1134,7 @@ int gemm_dispatch(const char* who, int dtype_ab, int dtype_c, int trans_a, int t
                   int64_t M, int64_t N, int64_t K, float alpha, const void* A, int64_t lda,
                   int64_t stride_a, const void* B, int64_t ldb, int64_t stride_b, float beta,
                   void* C, int64_t ldc, int64_t stride_c, int64_t batch, const float* bias,
-                  void* stream) {
+                  void* stream, int64_t ktot = INT64_MAX, bool padded = false) {
   TG_REQUIRE(M >= 0 && N >= 0 && K >= 0 && batch >= 0, "%s: negative extent", who);
   if (M == 0 || N == 0 || batch == 0) return TG_OK;
   TG_REQUIRE(C, "%s: null C", who);
@@ -1246,7 +1157,8 @@ int gemm_dispatch(const char* who, int dtype_ab, int dtype_c, int trans_a, int t
   }
 #define TG_GEMM_CALL(TA, TC)                                                                  \
   return launch<TA, TC>(trans_a, trans_b, M, N, K, alpha, A, lda, stride_a, B, ldb, stride_b, \
-                        beta, C, ldc, stride_c, batch, s, bias)
+                        beta, C, ldc, stride_c, batch, s, bias, nullptr, ktot, \
+                        padded)
   if (dtype_ab == TG_F16) {
     if (dtype_c == TG_F32) TG_GEMM_CALL(tg_half, float);
     if (dtype_c == TG_F16) TG_GEMM_CALL(tg_half, tg_half);
@@ -1254,7 +1166,10 @@ int gemm_dispatch(const char* who, int dtype_ab, int dtype_c, int trans_a, int t
     if (dtype_c == TG_F32) TG_GEMM_CALL(tg_bf16, float);
     if (dtype_c == TG_BF16) TG_GEMM_CALL(tg_bf16, tg_bf16);
   } else if (dtype_ab == TG_F32 && dtype_c == TG_F32) {
-    if (!tg_gemm_rs_serves(M, N, K, batch)) TG_GEMM_CALL(float, float);
+    if (!tg_gemm_rs_serves(M, N, K, batch))
+      return launch_f32(trans_a, trans_b, M, N, K, alpha, (const float*)A, lda, stride_a,
+                        (const float*)B, ldb, stride_b, beta, (float*)C, ldc, stride_c, batch, s,
+                        bias);
     return tg_gemm_rs(tg_gemm_rs_plan(M, N, K, batch, false), trans_a, trans_b, M, N, K, alpha,
                       (const float*)A, lda, stride_a, (const float*)B, ldb, stride_b, beta,
                       (float*)C, ldc, stride_c, batch, bias, s);
@@ -1278,6 +1193,11 @@ template <typename TO>
 __device__ __forceinline__ void fin_store(void* out, int64_t i, int64_t n, const float a[4],
                                           float alpha, float beta, const float* bias, int64_t N) {
   TO* o = reinterpret_cast<TO*>(out) + i;
+  if (i + 4 <= n && !bias && beta == 0.f) {  // whole, unbranched: one vector store
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = tg_from_float<TO>(alpha * a[j]);
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (i + j >= n) return;
@@ -1342,24 +1262,100 @@ int split_finish(const char* who, const float* parts, int64_t S, int64_t MN, int
   return tg_check_launch(who);
 }
 
-// K split of a 16-bit product whose output has too few 128x128 tiles for two per CU
-// (qkv/out projections [1024, 1024] and FC weights [1024, 4096] over 8192 tokens), or
-// whose K is very long (the tied head's input gradient over a 32000-word vocabulary: 676
-// -> 563 us in two halves): returns s with K % s == 0 and (K / s) % 64 == 0, or 1.
-int64_t split16(int64_t M, int64_t N, int64_t K) {
-  if (M <= 0 || N <= 0) return 1;
-  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  const int64_t cus = tg_num_cus();
-  int64_t want;
-  if (K >= 16384 && tiles < 4 * cus) want = 2;
-  else if (tiles >= 2 * cus || K < 2048) return 1;
-  else want = std::min((2 * cus + tiles - 1) / tiles, K / 1024);
-  for (int64_t s = want; s > 1; --s)
-    if (K % s == 0 && (K / s) % 64 == 0) return s;
-  return 1;
+size_t al256(size_t n) { return (n + 255) & ~size_t{255}; }
+
+// ---- rows of other lengths: copies with aligned, zero-padded rows ----
+// The DMA-staged kernel needs rows of whole 16-byte chunks.  A 16-bit operand whose rows
+// are not (an odd vocabulary or hidden size) is copied into the workspace with its rows
+// padded by zeros; the copy streams once through memory (4096 x 50257: 180 us) where the
+// element-wise staging of k_gemm costs the product most of its rate (4096 x 1024 x 50257:
+// 2440 us there).  Products too short for that stay on k_gemm: below 2^20 multiply-adds, or
+// with K < 192 below 2^31 (1429 x 1000 x 161: 18 us there, 21 with copies; 64 x 85 x 233: 20
+// and 15).
+struct PackArg {
+  const void* src;
+  uint4* dst;
+  int64_t ld, cols;
+  unsigned chunks;  // 8-element chunks of the whole copy
+};
+constexpr int kPackBlock = 256;
+// One 8-element chunk per thread; blockIdx.y names the operand.  Inside a row two aligned
+// 16-byte loads cover the chunk (every byte of them lies in the row) and are shifted into
+// place; the first and last two chunks of a row go element by element.
+__global__ __launch_bounds__(kPackBlock) void k_pack_rows(PackArg pa, PackArg pb) {
+  const PackArg p = blockIdx.y ? pb : pa;
+  const unsigned q = blockIdx.x * kPackBlock + threadIdx.x;
+  if (q >= p.chunks) return;
+  const unsigned cpr = (unsigned)((p.cols + 7) / 8), r = q / cpr;
+  const int64_t c = (int64_t)(q - r * cpr) * 8;
+  const unsigned short* s = static_cast<const unsigned short*>(p.src) + r * p.ld + c;
+  unsigned o[4];
+  if (c >= 8 && c + 16 <= p.cols) {
+    const uintptr_t u = reinterpret_cast<uintptr_t>(s);
+    const uint4* v = reinterpret_cast<const uint4*>(u & ~(uintptr_t)15);
+    const uint4 a = v[0], b = v[1];
+    unsigned x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    const bool two = u & 8, one = u & 4, half = u & 2;
+#pragma unroll
+    for (int e = 0; e < 6; ++e) x[e] = two ? x[e + 2] : x[e];
+#pragma unroll
+    for (int e = 0; e < 5; ++e) x[e] = one ? x[e + 1] : x[e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = half ? (x[e] >> 16) | (x[e + 1] << 16) : x[e];
+  } else {
+    const int64_t n = p.cols - c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const unsigned lo = 2 * e < n ? s[2 * e] : 0, hi = 2 * e + 1 < n ? s[2 * e + 1] : 0;
+      o[e] = lo | (hi << 16);
+    }
+  }
+  p.dst[q] = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-size_t al256(size_t n) { return (n + 255) & ~size_t{255}; }
+// Bytes of the aligned copies that op(A) [M,K] and op(B) [K,N] with dense rows need (0:
+// none).
+struct PackPlan {
+  int64_t ra, ca, rb, cb;  // stored rows and columns
+  size_t a, b;
+};
+PackPlan pack_plan(int dtype_ab, int ta, int tb, int64_t M, int64_t N, int64_t K) {
+  PackPlan p{ta ? K : M, ta ? M : K, tb ? N : K, tb ? K : N, 0, 0};
+  const double mnk = (double)M * (double)N * (double)K;
+  if ((dtype_ab != TG_F16 && dtype_ab != TG_BF16) ||
+      mnk < (K < 192 ? 2147483648.0 : 1048576.0))
+    return p;
+  const double most = 4294967296.0 - kPackBlock;  // chunks that 32-bit indices count
+  if ((double)p.ra * (double)((p.ca + 7) / 8) > most ||
+      (double)p.rb * (double)((p.cb + 7) / 8) > most)
+    return p;
+  if (p.ca % 8) p.a = al256((size_t)(p.ra * ((p.ca + 7) / 8)) * 16);
+  if (p.cb % 8) p.b = al256((size_t)(p.rb * ((p.cb + 7) / 8)) * 16);
+  return p;
+}
+
+// Copies the operands that the plan names to `to` and points A, lda / B, ldb at them.
+int pack_operands(const PackPlan& p, const void*& A, int64_t& lda, const void*& B, int64_t& ldb,
+                  char* to, hipStream_t s) {
+  PackArg arg[2];
+  int n = 0;
+  if (p.a) {
+    arg[n++] = PackArg{A, reinterpret_cast<uint4*>(to), lda, p.ca,
+                       (unsigned)(p.ra * ((p.ca + 7) / 8))};
+    A = to, lda = (p.ca + 7) / 8 * 8;
+  }
+  if (p.b) {
+    arg[n++] = PackArg{B, reinterpret_cast<uint4*>(to + p.a), ldb, p.cb,
+                       (unsigned)(p.rb * ((p.cb + 7) / 8))};
+    B = to + p.a, ldb = (p.cb + 7) / 8 * 8;
+  }
+  if (n == 0) return TG_OK;
+  if (n == 1) arg[1] = arg[0];
+  const unsigned most = std::max(arg[0].chunks, arg[1].chunks);
+  const dim3 grid((most - 1) / kPackBlock + 1, (unsigned)n);
+  k_pack_rows<<<grid, kPackBlock, 0, s>>>(arg[0], arg[1]);
+  return tg_check_launch("tg_matmul");
+}
 
 // The K split of a 2-D product, and the bytes of its fp32 partial sums.
 struct SplitPlan {
@@ -1376,8 +1372,8 @@ SplitPlan split_plan(int dtype_ab, int64_t M, int64_t N, int64_t K) {
     p.rs = tg_gemm_rs_plan(M, N, K, 1, true);
     p.S = p.rs.S, p.kc = p.rs.kc;
   } else if (dtype_ab != TG_F64) {
-    p.S = split16(M, N, K);
-    p.kc = K / p.S;
+    const V3Plan v = v3_plan(M, N, K, 1, true);
+    p.S = v.S, p.kc = v.kc;
   }
   if (p.S > 1) p.bytes = al256((size_t)(p.S * split_stride(M * N)) * sizeof(float));
   return p;
@@ -1386,10 +1382,11 @@ SplitPlan split_plan(int dtype_ab, int64_t M, int64_t N, int64_t K) {
 struct WgradPlan {
   SplitPlan sp;
   size_t bparts, red;  // sizes of the workspace regions behind the partial sums
+  PackPlan pk;         // and behind those
 };
 
 WgradPlan wgrad_plan(int dtype_ab, int64_t M, int64_t N, int64_t K, bool has_b) {
-  WgradPlan p{split_plan(dtype_ab, M, N, K), 0, 0};
+  WgradPlan p{split_plan(dtype_ab, M, N, K), 0, 0, pack_plan(dtype_ab, 1, 0, M, N, K)};
   if (has_b) {
     p.bparts = al256((size_t)(p.sp.S * N) * sizeof(float));
     p.red = al256(tg_reduce_rows_workspace(K, N));
@@ -1398,9 +1395,11 @@ WgradPlan wgrad_plan(int dtype_ab, int64_t M, int64_t N, int64_t K, bool has_b) 
 }
 }  // namespace
 
-TG_EXPORT size_t tg_matmul_workspace(int dtype_ab, int64_t M, int64_t N, int64_t K) {
+TG_EXPORT size_t tg_matmul_workspace(int dtype_ab, int trans_a, int trans_b, int64_t M, int64_t N,
+                                     int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return split_plan(dtype_ab, M, N, K).bytes;
+  const PackPlan pk = pack_plan(dtype_ab, trans_a, trans_b, M, N, K);
+  return split_plan(dtype_ab, M, N, K).bytes + pk.a + pk.b;
 }
 
 TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int64_t M, int64_t N,
@@ -1408,38 +1407,45 @@ TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int
                         int64_t ldb, const float* bias, float beta, void* C, int64_t ldc,
                         void* workspace, size_t workspace_bytes, void* stream) {
   const char* who = "tg_matmul";
-  if (M > 0 && N > 0 && K > 0 && ldc == N) {  // (the split finish writes a dense C)
-    const SplitPlan p = split_plan(dtype_ab, M, N, K);
-    if (p.S > 1 && workspace_bytes >= p.bytes) {
-      TG_REQUIRE(A && B && C, "%s: null operand", who);
-      TG_REQUIRE(lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N), "%s: bad leading dim", who);
-      TG_REQUIRE(dtype_c == TG_F32 || (dtype_c == dtype_ab && dtype_ab != TG_F32),
-                 "%s: unsupported dtype combination ab=%d c=%d", who, dtype_ab, dtype_c);
-      TG_REQUIRE(workspace, "%s: null workspace", who);
-      float* parts = static_cast<float*>(workspace);
-      const int64_t sa = trans_a ? p.kc * lda : p.kc, sb = trans_b ? p.kc : p.kc * ldb;
-      const int64_t sc = split_stride(M * N);
-      hipStream_t s = tg_stream(stream);
-      const int rc =
-          dtype_ab == TG_F32
-              ? tg_gemm_rs(p.rs, trans_a, trans_b, M, N, K, 1.f, (const float*)A, lda, sa,
-                           (const float*)B, ldb, sb, 0.f, parts, N, sc, p.S, nullptr, s)
-              : gemm_dispatch(who, dtype_ab, TG_F32, trans_a, trans_b, M, N, p.kc, 1.f, A, lda, sa,
-                              B, ldb, sb, 0.f, parts, N, sc, p.S, nullptr, stream);
-      if (rc != TG_OK) return rc;
-      return split_finish(who, parts, p.S, M * N, N, alpha, beta, bias, C, dtype_c, nullptr, 0,
-                          nullptr, 0, 0, s);
-    }
-  }
-  return gemm_dispatch(who, dtype_ab, dtype_c, trans_a, trans_b, M, N, K, alpha, A, lda, 0, B, ldb,
-                       0, beta, C, ldc, 0, 1, bias, stream);
+  const SplitPlan p = M > 0 && N > 0 && K > 0 ? split_plan(dtype_ab, M, N, K) : SplitPlan{};
+  const PackPlan pk = M > 0 && N > 0 && K > 0 ? pack_plan(dtype_ab, trans_a, trans_b, M, N, K)
+                                              : PackPlan{};
+  const size_t need = p.bytes + pk.a + pk.b;
+  if (need == 0 || workspace_bytes < need)
+    return gemm_dispatch(who, dtype_ab, dtype_c, trans_a, trans_b, M, N, K, alpha, A, lda, 0, B,
+                         ldb, 0, beta, C, ldc, 0, 1, bias, stream);
+  TG_REQUIRE(A && B && C, "%s: null operand", who);
+  TG_REQUIRE(workspace, "%s: null workspace", who);
+  TG_REQUIRE(ldc >= N, "%s: ldc %lld < N %lld", who, (long long)ldc, (long long)N);
+  TG_REQUIRE(lda >= (trans_a ? M : K) && ldb >= (trans_b ? K : N), "%s: bad leading dim", who);
+  TG_REQUIRE(dtype_c == TG_F32 || (dtype_c == dtype_ab && dtype_ab != TG_F32),
+             "%s: unsupported dtype combination ab=%d c=%d", who, dtype_ab, dtype_c);
+  hipStream_t s = tg_stream(stream);
+  char* ws = static_cast<char*>(workspace);
+  const bool padded = pk.a || pk.b;
+  int rc = pack_operands(pk, A, lda, B, ldb, ws + p.bytes, s);
+  if (rc != TG_OK) return rc;
+  if (p.S <= 1 || ldc != N)  // (the split finish writes a dense C)
+    return gemm_dispatch(who, dtype_ab, dtype_c, trans_a, trans_b, M, N, K, alpha, A, lda, 0, B,
+                         ldb, 0, beta, C, ldc, 0, 1, bias, stream, INT64_MAX, padded);
+  float* parts = reinterpret_cast<float*>(ws);
+  const int64_t sa = trans_a ? p.kc * lda : p.kc, sb = trans_b ? p.kc : p.kc * ldb;
+  const int64_t sc = split_stride(M * N);
+  rc = dtype_ab == TG_F32
+           ? tg_gemm_rs(p.rs, trans_a, trans_b, M, N, K, 1.f, (const float*)A, lda, sa,
+                        (const float*)B, ldb, sb, 0.f, parts, N, sc, p.S, nullptr, s)
+           : gemm_dispatch(who, dtype_ab, TG_F32, trans_a, trans_b, M, N, p.kc, 1.f, A, lda, sa, B,
+                           ldb, sb, 0.f, parts, N, sc, p.S, nullptr, stream, K, padded);
+  if (rc != TG_OK) return rc;
+  return split_finish(who, parts, p.S, M * N, N, alpha, beta, bias, C, dtype_c, nullptr, 0, nullptr,
+                      0, 0, s);
 }
 
 TG_EXPORT size_t tg_gemm_wgrad_workspace(int dtype_ab, int64_t M, int64_t N, int64_t K,
                                          int with_bias) {
   if (N <= 0 || M < 0 || K < 0) return 0;
   const WgradPlan p = wgrad_plan(dtype_ab, M, N, K, with_bias != 0);
-  return p.sp.bytes + p.bparts + p.red;
+  return p.sp.bytes + p.bparts + p.red + p.pk.a + p.pk.b;
 }
 
 TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const void* X,
@@ -1462,8 +1468,8 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
              "tg_gemm_wgrad: fp64 operands take fp64 gradients");
   if (K > 0) TG_REQUIRE(X && G, "tg_gemm_wgrad: null operand");
   WgradPlan p = wgrad_plan(dtype_ab, M, N, K, db != nullptr);
-  const size_t need = p.sp.bytes + p.bparts + p.red;
-  TG_REQUIRE(workspace_bytes >= need && (workspace || !p.sp.bytes),
+  const size_t need = p.sp.bytes + p.bparts + p.red + p.pk.a + p.pk.b;
+  TG_REQUIRE(workspace_bytes >= need && (workspace || !(p.sp.bytes + p.pk.a + p.pk.b)),
              "tg_gemm_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, need);
   char* ws = static_cast<char*>(workspace);
   float* parts = reinterpret_cast<float*>(ws);
@@ -1475,21 +1481,26 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
   }
   hipStream_t s = tg_stream(stream);
   const int64_t S = p.sp.S, kc = p.sp.kc, sc = split_stride(M * N);
+  const void* G0 = G;
+  const bool padded = p.pk.a || p.pk.b;
+  int rc = TG_OK;
+  if (K > 0)
+    rc = pack_operands(p.pk, X, ldx, G, ldg, ws + p.sp.bytes + p.bparts + p.red, s);
+  if (rc != TG_OK) return rc;
   const float bw = acc_w ? 1.f : 0.f;
   const bool fused = db && K > 0 && N % 4 == 0 && (dtype_ab == TG_F16 || dtype_ab == TG_BF16) &&
-                     v3_ok(2, 1, 0, M, N, kc, X, ldx, kc * ldx, G, ldg, kc * ldg);
-  int rc;
+                     v3_ok(2, 1, 0, M, N, kc, X, ldx, kc * ldx, G, ldg, kc * ldg, padded);
   if (fused) {
 #define TG_WG(T)                                                                              \
   if (S > 1)                                                                                  \
     rc = launch<T, float>(1, 0, M, N, kc, 1.f, X, ldx, kc * ldx, G, ldg, kc * ldg, 0.f, parts, \
-                          N, sc, S, s, nullptr, bparts);                                      \
+                          N, sc, S, s, nullptr, bparts, K, padded);                           \
   else if (dtype_w == TG_F32)                                                                 \
     rc = launch<T, float>(1, 0, M, N, K, 1.f, X, ldx, 0, G, ldg, 0, bw, dW, ldw, 0, 1, s,       \
-                          nullptr, bparts);                                                   \
+                          nullptr, bparts, INT64_MAX, padded);                                \
   else                                                                                        \
     rc = launch<T, T>(1, 0, M, N, K, 1.f, X, ldx, 0, G, ldg, 0, bw, dW, ldw, 0, 1, s, nullptr, \
-                      bparts)
+                      bparts, INT64_MAX, padded)
     if (dtype_ab == TG_F16) { TG_WG(tg_half); } else { TG_WG(tg_bf16); }
 #undef TG_WG
     if (rc != TG_OK) return rc;
@@ -1499,18 +1510,18 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
     if (rc != TG_OK) return rc;
   } else if (S > 1) {
     rc = gemm_dispatch("tg_gemm_wgrad", dtype_ab, TG_F32, 1, 0, M, N, kc, 1.f, X, ldx, kc * ldx,
-                       G, ldg, kc * ldg, 0.f, parts, N, sc, S, nullptr, stream);
+                       G, ldg, kc * ldg, 0.f, parts, N, sc, S, nullptr, stream, K, padded);
     if (rc != TG_OK) return rc;
   } else {
     rc = gemm_dispatch("tg_gemm_wgrad", dtype_ab, dtype_w, 1, 0, M, N, K, 1.f, X, ldx, 0, G, ldg,
-                       0, bw, dW, ldw, 0, 1, nullptr, stream);
+                       0, bw, dW, ldw, 0, 1, nullptr, stream, INT64_MAX, padded);
     if (rc != TG_OK) return rc;
   }
   rc = split_finish("tg_gemm_wgrad", parts, S, S > 1 ? M * N : 0, N, 1.f, bw, nullptr, dW, dtype_w,
                     bparts, fused ? N : 0, db, dtype_b, acc_b, s);
   if (rc != TG_OK) return rc;
   if (db && !fused)
-    return tg_reduce_rows(dtype_ab, G, dtype_b, db, K, N, acc_b, red, p.red, stream);
+    return tg_reduce_rows(dtype_ab, G0, dtype_b, db, K, N, acc_b, red, p.red, stream);
   return TG_OK;
 }
 
@@ -1545,20 +1556,21 @@ int wgrad_group_launch(int shape, const int* idx, int n, int64_t M, const int64_
       if (acc_b && acc_b[m]) grp.dbacc |= 1u << i;
     }
   }
-#define TG_GG(WGM, WGN, SM, SN)                                                                \
-  do {                                                                                         \
-    static_assert(WGM * SM * 32 > 0 && WGN * SN * 32 > 0, "tile");                            \
-    dim3 g3((unsigned)grp.tiles[n]);                                                           \
-    if (any_b)                                                                                 \
-      k_gemm_v3g<T, TC, WGM, WGN, SM, SN, true><<<g3, 64 * WGM * WGN, 0, s>>>(M, K, ldx, grp,   \
-                                                                            dtype_b);          \
-    else                                                                                       \
-      k_gemm_v3g<T, TC, WGM, WGN, SM, SN, false><<<g3, 64 * WGM * WGN, 0, s>>>(M, K, ldx, grp,  \
-                                                                             dtype_b);         \
+#define TG_GGT(WGM, WGN, SM, SN, TAIL, BSUM)                                                \
+  k_gemm_v3g<T, TC, WGM, WGN, SM, SN, TAIL, BSUM><<<g3, 64 * WGM * WGN, 0, s>>>(M, K, ldx, grp, \
+                                                                                dtype_b)
+#define TG_GG(WGM, WGN, SM, SN)                                        \
+  do {                                                                 \
+    dim3 g3((unsigned)grp.tiles[n]);                                   \
+    if (any_b && K % V3_BK) TG_GGT(WGM, WGN, SM, SN, true, true);      \
+    else if (any_b) TG_GGT(WGM, WGN, SM, SN, false, true);             \
+    else if (K % V3_BK) TG_GGT(WGM, WGN, SM, SN, true, false);         \
+    else TG_GGT(WGM, WGN, SM, SN, false, false);                       \
   } while (0)
   if (shape == 2) TG_GG(4, 2, 2, 4);
   else TG_GG(kBigWGM, kBigWGN, kBigSM, kBigSN);
 #undef TG_GG
+#undef TG_GGT
   return tg_check_launch("tg_gemm_wgrad_group");
 }
 

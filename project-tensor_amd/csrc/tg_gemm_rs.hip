@@ -219,6 +219,10 @@ __device__ __forceinline__ void rs_fp32_tiles(const float* __restrict__ A, int64
   }
 }
 
+// STAG: the upper half of the waves multiplies before it stores.  TWO: sums of 512 k are
+// added up in a second accumulator, so that the smaller tiles' sums err no more than the
+// K splits that served their sizes before (64x64 and 128x128; 256x128 has no registers left
+// for it).
 template <bool TA, bool TB, int WGM, int WGN, int SM, int SN, bool STAG, bool TWO>
 __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha, const float* __restrict__ A,
@@ -468,7 +472,8 @@ enum { RS_256x128 = 0, RS_128x128, RS_64x64, RS_SMALL };
 // 1.75 us (one block per CU each), 64x64 1.13 / 1.4 / 1.95 us with one / two / three
 // blocks per CU; a block's start and store take 3-4 us.  The small kernel takes 0.9 us
 // per 128 k plus 2.1 us for each block per CU (its operands come straight from the
-// caches).  A K split adds the finishing launch: 5 us and its traffic at 3.5 TB/s.
+// caches).  A K split adds the finishing launch: 10 us, half of it
+// the host's, and its traffic at 3.5 TB/s.
 // (Measured against the previous kernels, us: 8192x4096x1024 727 -> 402, 1024x4096x8192
 // with A transposed 1086 -> 399, 832x1664x8932 1210 -> 224, 1000^3 117 -> 37,
 // 448x256x32000 867 -> 72, 33x257x784 20 -> 15.)
@@ -485,7 +490,7 @@ TgRsPlan tg_gemm_rs_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool ca
     const int64_t kc = S == 1 ? K : ((K + S - 1) / S + 63) / 64 * 64;
     if (S > 1 && (kc < 128 || (K + kc - 1) / kc != S)) continue;
     const double kt = (double)((kc + BK - 1) / BK);
-    const double fin = S > 1 ? 5.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 3.5e6 : 0.0;
+    const double fin = S > 1 ? 10.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 3.5e6 : 0.0;
     // (a split's partial sums stay within 256 MiB)
     if (S > 1 && (double)S * (double)M * (double)N * 4.0 > 268435456.0) break;
     double t[4];
@@ -516,7 +521,7 @@ int tg_gemm_rs(const TgRsPlan& p, int ta, int tb, int64_t M, int64_t N, int64_t 
                          sc, batch, bias, s)
   switch (p.shape) {
     case RS_256x128: return TG_RSL(4, 2, 2, 2, true, false);
-    case RS_128x128: return TG_RSL(4, 2, 1, 2, true, false);
+    case RS_128x128: return TG_RSL(4, 2, 1, 2, true, true);
     case RS_64x64: return TG_RSL(2, 2, 1, 1, false, true);
     default: break;
   }

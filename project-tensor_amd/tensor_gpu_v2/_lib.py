@@ -93,7 +93,7 @@ SIGNATURES = {
                        _i64, _i64, _f32, _vp, _i64, _i64, _i64, _vp]),
     "tg_gemm_bias": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64,
                             _vp, _vp, _i64, _vp]),
-    "tg_matmul_workspace": (_sz, [_i32, _i64, _i64, _i64]),
+    "tg_matmul_workspace": (_sz, [_i32, _i32, _i32, _i64, _i64, _i64]),
     "tg_matmul": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64,
                          _vp, _f32, _vp, _i64, _vp, _sz, _vp]),
     "tg_gemm_wgrad_workspace": (_sz, [_i32, _i64, _i64, _i64, _i32]),
@@ -343,7 +343,7 @@ def gemm_epilogue(epi, a, b, x, out, bias=None, beta=0.0):
         _dev(bias, "bias")
         if bias.dtype != torch.float32 or bias.numel() != N:
             raise ValueError("gemm_epilogue: bias must be fp32 [N]")
-    if _matmul_ws(dtype_code(a), M, N, K):
+    if _matmul_ws(dtype_code(a), 0, 1 if epi == "gelu_bwd" else 0, M, N, K):
         # the plain product would run K-split (another summation order): not fused, so
         # a fused result always equals the separate kernels' bit for bit
         return False
@@ -1204,11 +1204,11 @@ def _gemm_bias_launch(a, b, bias, out, trans_b):
     M, K = a.shape
     N = out.shape[1]
     code = _TORCH_TO_CODE[a.dtype]
-    # (16-bit forwards run unsplit: their fused-epilogue forms do)
-    nb = _matmul_ws(code, M, N, K) if code == F32 else 0
+    tb = 1 if trans_b else 0
+    nb = _matmul_ws(code, 0, tb, M, N, K)
     ws = workspace(nb, out.device) if nb else None
     _check("tg_matmul", (_lib or load()).tg_matmul(
-        code, _TORCH_TO_CODE[out.dtype], 0, 1 if trans_b else 0, M, N, K, 1.0, a.data_ptr(), K,
+        code, _TORCH_TO_CODE[out.dtype], 0, tb, M, N, K, 1.0, a.data_ptr(), K,
         b.data_ptr(), b.shape[1], bias.data_ptr(), 0.0, out.data_ptr(), N,
         ws.data_ptr() if nb else None, nb, stream_handle()))
     return out
@@ -1340,15 +1340,15 @@ def wgrad_group(xs, gs, dws, acc_ws, dbs=None, acc_bs=None):
 _MATMUL_WS = {}
 
 
-def _matmul_ws(code, M, N, K):
-    """Workspace bytes of tg_matmul for this dtype code and shape (0: the product runs
-    without a K split), kept by shape: training loops repeat them."""
-    key = (code, M, N, K)
+def _matmul_ws(code, ta, tb, M, N, K):
+    """Workspace bytes of tg_matmul for this dtype code, orientation and shape (0: the
+    product runs without a K split), kept by shape: training loops repeat them."""
+    key = (code, ta, tb, M, N, K)
     nb = _MATMUL_WS.get(key)
     if nb is None:
         if len(_MATMUL_WS) > 4096:
             _MATMUL_WS.clear()
-        nb = _MATMUL_WS[key] = load().tg_matmul_workspace(code, M, N, K)
+        nb = _MATMUL_WS[key] = load().tg_matmul_workspace(code, ta, tb, M, N, K)
     return nb
 
 
@@ -1380,10 +1380,11 @@ def matmul2d(a, b, out=None, trans_a=False, trans_b=False, alpha=1.0, beta=0.0, 
     if out.dtype not in (torch.float32, a.dtype):
         raise TypeError(f"gemm: C must be float32 or {a.dtype}, got {out.dtype}")
     ensure_device(out.device.index)
-    nb = _matmul_ws(code, M, N, K)
+    ta, tb = int(bool(trans_a)), int(bool(trans_b))
+    nb = _matmul_ws(code, ta, tb, M, N, K)
     ws = workspace(nb, out.device) if nb else None
     _check("tg_matmul", load().tg_matmul(
-        code, dtype_code(out), int(bool(trans_a)), int(bool(trans_b)), M, N, K, float(alpha),
+        code, dtype_code(out), ta, tb, M, N, K, float(alpha),
         ptr(a), lda, ptr(b), ldb, None, float(beta), ptr(out), N, ptr(ws), nb, stream_handle()))
     return out
 

@@ -1,0 +1,120 @@
+"""16-bit products at ragged sizes and alignments: k past the last tile (masked DMA), any
+M and N, odd leading dimensions (the register-staged kernel), K splits whose last chunk is
+short, and the fused and grouped forms at such sizes, against float64 products of the same
+16-bit operands."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DT = {"fp16": torch.float16, "bf16": torch.bfloat16}
+EPS = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
+
+
+def L():
+    from tensor_gpu_v2 import _lib
+    return _lib
+
+
+def _bound(c, a, b, what, add=0.0):
+    """16-bit products are exact in fp32; a sum of K of them rounds at most once per MFMA
+    of 16 k (2^-23 of sum |a||b| each) and once when it is stored."""
+    K = a.shape[1]
+    want = a.double() @ b.double() + add
+    mag = a.double().abs() @ b.double().abs() + abs(add)
+    tol = (K // 16 + 40) * 2.0 ** -23 * mag + 1.01 * EPS[c.dtype] * want.abs() + 1e-7
+    err = (c.double() - want).abs()
+    assert bool((err <= tol).all()), f"{what}: {(err - tol).max().item():.2e}"
+
+
+def _mk(g, r, c, dt, pad=0, off=0):
+    """[r, c] with `pad` extra columns of NaN and a base `off` elements into its buffer."""
+    buf = torch.full((r * (c + pad) + off + 8,), float("nan"), device="cuda", dtype=dt)
+    v = buf[off:off + r * (c + pad)].view(r, c + pad)
+    v[:, :c] = torch.randn(r, c, generator=g, device="cuda").to(dt)
+    return v[:, :c]
+
+
+SHAPES = [(1, 8, 8), (8, 8, 1), (1, 1, 1), (5, 7, 9), (64, 64, 72), (129, 136, 200), (300, 264, 65),
+          (1917, 808, 808), (3290, 768, 768), (257, 1000, 4104), (70, 50257, 64), (513, 1025, 777),
+          (4100, 2056, 104)]
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_matmul_ragged(cuda, M, N, K, dt):
+    dt = DT[dt]
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + N + K)
+    for ta in (False, True):
+        for tb in (False, True):
+            a = _mk(g, K, M, dt) if ta else _mk(g, M, K, dt)
+            b = _mk(g, N, K, dt) if tb else _mk(g, K, N, dt)
+            A, B = (a.t() if ta else a), (b.t() if tb else b)
+            for odt in (dt, torch.float32):
+                c = L().matmul2d(a.contiguous(), b.contiguous(), trans_a=ta, trans_b=tb,
+                                 out_dtype=odt)
+                _bound(c, A, B, f"matmul2d {ta} {tb} {odt}")
+
+
+@pytest.mark.parametrize("M,N,K,pad,off", [(130, 136, 72, 8, 0), (130, 136, 72, 24, 8),
+                                           (200, 130, 100, 3, 1), (2100, 4200, 65, 1, 3),
+                                           (1000, 1000, 200, 5, 2), (40, 24, 7, 2, 1)])
+def test_gemm_padded_rows(cuda, M, N, K, pad, off):
+    """Padded leading dimensions (NaN in the padding: reading it would show) at aligned and
+    odd row starts, accumulating, in a batch."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    dt = torch.float16
+    for ta in (False, True):
+        for tb in (False, True):
+            a = _mk(g, K, M, dt, pad, off) if ta else _mk(g, M, K, dt, pad, off)
+            b = _mk(g, N, K, dt, pad, off) if tb else _mk(g, K, N, dt, pad, off)
+            c = torch.ones(2, M, N, device="cuda")
+            L().gemm(a, b, c, ta, tb, 1.0, 1.0, M, N, K, a.stride(0), b.stride(0), N, 0, 0, M * N,
+                     2)
+            assert torch.equal(c[0], c[1])
+            _bound(c[0], a.t() if ta else a, b.t() if tb else b, f"padded {ta} {tb}", 1.0)
+
+
+@pytest.mark.parametrize("K,M,N", [(7230, 64, 64), (3290, 768, 2304), (1917, 808, 3232),
+                                   (85, 40, 48), (7231, 72, 63), (9, 8, 8)])
+def test_wgrad_ragged_tokens(cuda, K, M, N):
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, gr = _mk(g, K, M, torch.bfloat16), _mk(g, K, N, torch.bfloat16)
+    x, gr = x.contiguous(), gr.contiguous()
+    dw, db = torch.ones(M, N, device="cuda"), torch.ones(N, device="cuda")
+    L().wgrad(x, gr, dw, True, db, True)
+    _bound(dw, x.t(), gr, "wgrad", 1.0)
+    mag = gr.double().abs().sum(0) + 1
+    assert bool(((db.double() - gr.double().sum(0) - 1).abs() <= (K + 8) * 2.0 ** -23 * mag).all())
+    # grouped: the members of one input shape in one call equal the members' own products
+    ws = [torch.zeros(M, N, device="cuda") for _ in range(3)]
+    bs = [torch.zeros(N, device="cuda") for _ in range(3)]
+    L().wgrad_group([x, x, x], [gr, gr * 0.5, gr], ws, [False] * 3, bs, [False] * 3)
+    assert torch.equal(ws[0], ws[2]) and torch.equal(bs[0], bs[2])
+    _bound(ws[1], x.t(), gr * 0.5, "wgrad_group")
+
+
+@pytest.mark.parametrize("M,N,K", [(357, 512, 128), (1917, 3232, 808), (61, 136, 72), (257, 264, 1000)])
+def test_epilogue_ragged_equals_separate(cuda, M, N, K):
+    dt = torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(N)
+    a, b = _mk(g, M, K, dt).contiguous(), (_mk(g, K, N, dt).contiguous() * 0.05)
+    bias = torch.randn(N, generator=g, device="cuda")
+    r = _mk(g, M, N, dt).contiguous()
+    ref = torch.empty(M, N, device="cuda", dtype=dt)
+    L().gemm_bias(a, b, bias, ref)
+    _bound(ref, torch.cat([a.double(), torch.ones(M, 1, device="cuda").double()], 1),
+           torch.cat([b.double(), bias.double()[None]], 0), "bias")
+    out, act = torch.empty_like(ref), torch.empty_like(ref)
+    if L().gemm_epilogue("gelu_fwd", a, b, act, out, bias):
+        assert torch.equal(out, ref)
+        assert torch.equal(act, L().act_fwd("gelu", ref))
+    out = torch.empty_like(ref)
+    if L().gemm_epilogue("residual", a, b, r, out, bias):
+        assert torch.equal(out, ref + r)
+    # GELU backward: A [M, K] @ W^T with W [N, K]
+    w = _mk(g, N, K, dt).contiguous()
+    d = torch.empty_like(ref)
+    if L().gemm_epilogue("gelu_bwd", a, w, r, d):
+        want = torch.empty_like(ref)
+        L().act_bwd("gelu", r, L().matmul2d(a, w, trans_b=True), want, False)
+        assert torch.equal(d, want)
