@@ -1128,16 +1128,14 @@ __device__ __forceinline__ void gen_acc(f32x16 (&acc)[NDB], const float* Xs, int
 
 // Forward.  grid = (ceil(Sq/128), B*H); one workgroup = 128 queries (4 waves x 32,
 // lane = query, Q in registers), key tiles of 32 staged in LDS.
+// (Ks, Vs: LDS of gen_lds<DP>() / 2 bytes each)
+template <int DP> constexpr int gen_lds() { return 2 * 32 * (DP + 4) * (int)sizeof(float); }
 template <typename T, int DP>
-__global__ __launch_bounds__(kThreads) void k_fa_fwd_gen(const T* __restrict__ Q,
-                                                         const T* __restrict__ K,
-                                                         const T* __restrict__ V,
-                                                         T* __restrict__ O, float* __restrict__ LSE,
-                                                         int64_t Sq, int64_t Sk, int D,
-                                                         float scale, int causal, FaLay lay) {
-  constexpr int NS = DP / 2, NDB = DP / 32, LD = DP + 4;
-  __shared__ __attribute__((aligned(16))) float Ks[32 * LD];
-  __shared__ __attribute__((aligned(16))) float Vs[32 * LD];
+__device__ __forceinline__ void fa_fwd_gen(float* Ks, float* Vs, const T* __restrict__ Q,
+                                           const T* __restrict__ K, const T* __restrict__ V,
+                                           T* __restrict__ O, float* __restrict__ LSE, int64_t Sq,
+                                           int64_t Sk, int D, float scale, int causal, FaLay lay) {
+  constexpr int NS = DP / 2, NDB = DP / 32;
   int64_t tile, bh;
   fa_block(tile, bh, lay.G);
   Q += lay.ha(bh, Sq, D);
@@ -1212,14 +1210,12 @@ __global__ __launch_bounds__(kThreads) void k_fa_fwd_gen(const T* __restrict__ Q
 // dO in registers, key tiles of 32 in LDS; the workgroup writes head-dim columns
 // [z*DO, z*DO + DO) of dQ (S and dP are recomputed per column range).
 template <typename T, int DP, int DO>
-__global__ __launch_bounds__(kThreads) void k_fa_bwd_dq_gen(
-    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    const T* __restrict__ O, const T* __restrict__ dO, const float* __restrict__ LSE,
-    float* __restrict__ Dv, T* __restrict__ dQ, int64_t Sq, int64_t Sk, int D, float scale,
-    int causal, int accumulate, FaLay lay) {
-  constexpr int NS = DP / 2, NDB = DO / 32, LD = DP + 4;
-  __shared__ __attribute__((aligned(16))) float Ks[32 * LD];
-  __shared__ __attribute__((aligned(16))) float Vs[32 * LD];
+__device__ __forceinline__ void fa_bwd_dq_gen(
+    float* Ks, float* Vs, const T* __restrict__ Q, const T* __restrict__ K,
+    const T* __restrict__ V, const T* __restrict__ O, const T* __restrict__ dO,
+    const float* __restrict__ LSE, float* __restrict__ Dv, T* __restrict__ dQ, int64_t Sq,
+    int64_t Sk, int D, float scale, int causal, int accumulate, FaLay lay) {
+  constexpr int NS = DP / 2, NDB = DO / 32;
   int64_t tile, bh;
   fa_block(tile, bh, lay.G);
   Q += lay.ha(bh, Sq, D);
@@ -1292,15 +1288,12 @@ __global__ __launch_bounds__(kThreads) void k_fa_bwd_dq_gen(
 // tiles of 32 (Q, dO, their LSE and D) in LDS; the workgroup writes head-dim columns
 // [z*DO, z*DO + DO) of dK and dV.
 template <typename T, int DP, int DO>
-__global__ __launch_bounds__(kThreads) void k_fa_bwd_dkdv_gen(
-    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
-    const T* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ Dv,
-    T* __restrict__ dK, T* __restrict__ dV, int64_t Sq, int64_t Sk, int D, float scale,
-    int causal, int accumulate, FaLay lay) {
-  constexpr int NS = DP / 2, NDB = DO / 32, LD = DP + 4;
-  __shared__ __attribute__((aligned(16))) float Qs[32 * LD];
-  __shared__ __attribute__((aligned(16))) float dOs[32 * LD];
-  __shared__ float ls[32], ds[32];
+__device__ __forceinline__ void fa_bwd_dkdv_gen(
+    float* Qs, float* dOs, float* ls, float* ds, const T* __restrict__ Q, const T* __restrict__ K,
+    const T* __restrict__ V, const T* __restrict__ dO, const float* __restrict__ LSE,
+    const float* __restrict__ Dv, T* __restrict__ dK, T* __restrict__ dV, int64_t Sq, int64_t Sk,
+    int D, float scale, int causal, int accumulate, FaLay lay) {
+  constexpr int NS = DP / 2, NDB = DO / 32;
   int64_t tile, bh;
   fa_block(tile, bh, lay.G);
   Q += lay.ha(bh, Sq, D);
@@ -1368,11 +1361,47 @@ __global__ __launch_bounds__(kThreads) void k_fa_bwd_dkdv_gen(
   }
 }
 
-// Output head-dim columns per workgroup of the generic backward: all of DP up to 128,
-// else half of it (the registers of a wave then hold K, V (or Q, dO) for the whole
+template <typename T, int DP>
+__global__ __launch_bounds__(kThreads) void k_fa_fwd_gen(const T* __restrict__ Q,
+                                                         const T* __restrict__ K,
+                                                         const T* __restrict__ V,
+                                                         T* __restrict__ O, float* __restrict__ LSE,
+                                                         int64_t Sq, int64_t Sk, int D,
+                                                         float scale, int causal, FaLay lay) {
+  __shared__ __attribute__((aligned(16))) char sm[gen_lds<DP>()];
+  float* f = reinterpret_cast<float*>(sm);
+  fa_fwd_gen<T, DP>(f, f + gen_lds<DP>() / 8, Q, K, V, O, LSE, Sq, Sk, D, scale, causal, lay);
+}
+
+template <typename T, int DP, int DO>
+__global__ __launch_bounds__(kThreads) void k_fa_bwd_dq_gen(
+    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
+    const T* __restrict__ O, const T* __restrict__ dO, const float* __restrict__ LSE,
+    float* __restrict__ Dv, T* __restrict__ dQ, int64_t Sq, int64_t Sk, int D, float scale,
+    int causal, int accumulate, FaLay lay) {
+  __shared__ __attribute__((aligned(16))) char sm[gen_lds<DP>()];
+  float* f = reinterpret_cast<float*>(sm);
+  fa_bwd_dq_gen<T, DP, DO>(f, f + gen_lds<DP>() / 8, Q, K, V, O, dO, LSE, Dv, dQ, Sq, Sk, D, scale,
+                           causal, accumulate, lay);
+}
+
+template <typename T, int DP, int DO>
+__global__ __launch_bounds__(kThreads) void k_fa_bwd_dkdv_gen(
+    const T* __restrict__ Q, const T* __restrict__ K, const T* __restrict__ V,
+    const T* __restrict__ dO, const float* __restrict__ LSE, const float* __restrict__ Dv,
+    T* __restrict__ dK, T* __restrict__ dV, int64_t Sq, int64_t Sk, int D, float scale,
+    int causal, int accumulate, FaLay lay) {
+  __shared__ __attribute__((aligned(16))) char sm[gen_lds<DP>()];
+  __shared__ float ls[32], ds[32];
+  float* f = reinterpret_cast<float*>(sm);
+  fa_bwd_dkdv_gen<T, DP, DO>(f, f + gen_lds<DP>() / 8, ls, ds, Q, K, V, dO, LSE, Dv, dK, dV, Sq, Sk,
+                             D, scale, causal, accumulate, lay);
+}
+
+// Output head-dim columns per workgroup of the generic backward: half of DP (the registers of a wave then hold K, V (or Q, dO) for the whole
 // head dim plus accumulators for half of it).
 template <int DP> struct GenSplit {
-  static constexpr int DO = DP <= 128 ? DP : DP / 2;
+  static constexpr int DO = DP / 2;
   static_assert(DP % DO == 0 && DO % 32 == 0, "head-dim split");
 };
 
@@ -1401,8 +1430,714 @@ int bwd_gen_t(const void* q, const void* k, const void* v, const void* o, const 
   return tg_check_launch("tg_flash_attn_bwd");
 }
 
-// Padded head dims of the generic path.
-#define TG_GEN_DP(X) X(32) X(64) X(96) X(128) X(192) X(256)
+// ================================================= split operands: fp32, other head dims
+// FlashAttention for fp32 data and for fp16 / bf16 head dims other than 64 and 128 (up to
+// 128; larger ones and unaligned fp32 values take the generic kernels above), on the
+// 16-bit matrix cores with fp32 accuracy of everything the generic kernels keep in fp32:
+// an fp32 operand is split exactly into three bf16 terms h + m + l (each the bf16 rounding
+// of what is left), and so are P and dS; of the nine term products the six of weight >=
+// 2^-16 are formed (as in tg_gemm_rs.hip).  fp16 / bf16 data multiply S = Q K^T and
+// dP = dO V^T as they are; in the products with P or dS, those are two bf16 terms (16
+// bits, far below the rounding of the 16-bit results) against bf16 data as it is or fp16
+// data as two exact bf16 terms.
+// What bounded the generic kernels was the fp32 matrix cores' rate (1/16 of the 16-bit
+// one) and element-wise staging.  Per 32 x 32 sub-tile at d = 64 the fp32 forward takes 48
+// bf16 MFMAs instead of 64 fp32 ones of twice the time, the backward 168 instead of 224.
+// fp32 values that the split cannot hold (nonzero below 2^-102, at or past 2^127, Inf, NaN)
+// make the workgroup run the generic kernel's body instead.
+//
+// Workgroup: 4 waves x 32 rows (queries; keys in the dK/dV kernel), the other operand in
+// tiles of BN rows, loaded into registers one tile ahead and written to LDS as planes
+// [BN][DP] with an odd number of 16-byte chunks per row (both the 16-byte row reads and the
+// transpose reads are then free of bank conflicts).
+typedef __bf16 bfv8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bfv2 __attribute__((ext_vector_type(2)));
+typedef unsigned short usv2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4_e __attribute__((ext_vector_type(4), aligned(4)));  // any dword
+
+// ROWP: planes of a row operand (S, dP); TRP: planes of a transposed operand (with P or
+// dS); SAME: the same planes; PT: terms of P and dS.
+template <typename T> struct Fx;
+template <> struct Fx<float> {
+  static constexpr int ROWP = 3, TRP = 3, PT = 3, BN = 32;
+  static constexpr bool SAME = true;
+};
+template <> struct Fx<tg_bf16> {
+  static constexpr int ROWP = 1, TRP = 1, PT = 2, BN = 64;
+  static constexpr bool SAME = true;
+};
+template <> struct Fx<tg_half> {
+  static constexpr int ROWP = 1, TRP = 2, PT = 2, BN = 64;
+  static constexpr bool SAME = false;
+};
+// Row fragments: fp32 data as bf16 terms, 16-bit data as it is.
+template <typename T> struct FxRow { typedef bfv8 type; };
+template <> struct FxRow<tg_half> { typedef Vec8<tg_half>::type type; };
+
+// Operand values seen outside the split's range (fp32 only).
+struct FxSeen {
+  usv2 lo = {0xffff, 0xffff}, hi = {0, 0};
+  __device__ __forceinline__ void see(unsigned h) {
+    const usv2 k = __builtin_bit_cast(usv2, h) << 1;  // drops the signs
+    lo = __builtin_elementwise_min(lo, (usv2)(k - (usv2)1));  // zero wraps to the top
+    hi = __builtin_elementwise_max(hi, k);
+  }
+  __device__ __forceinline__ bool bad() const {
+    return lo[0] < 0x18ff || lo[1] < 0x18ff || hi[0] >= 0xfe00 || hi[1] >= 0xfe00;
+  }
+};
+
+// Two floats as NT bf16 terms (packed pairs).
+template <int NT>
+__device__ __forceinline__ void split2(float x0, float x1, unsigned (&t)[NT]) {
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    t[i] = __builtin_bit_cast(unsigned, bfv2{(__bf16)x0, (__bf16)x1});
+    if (i + 1 < NT) {
+      x0 -= __builtin_bit_cast(float, t[i] << 16);
+      x1 -= __builtin_bit_cast(float, t[i] & 0xffff0000u);
+    }
+  }
+}
+template <typename T> __device__ __forceinline__ float raw2f(unsigned w, int hi) {
+  const unsigned short u = hi ? (unsigned short)(w >> 16) : (unsigned short)w;
+  return (float)__builtin_bit_cast(T, u);
+}
+
+// 8 elements of a row (n of them valid, the others zero) as raw dwords.
+template <typename T> struct FxRaw {
+  static constexpr int W = 2 * sizeof(T);
+  unsigned w[W];
+  __device__ __forceinline__ void load(const T* p) {
+#pragma unroll
+    for (int h = 0; h < W / 4; ++h) {
+      const u32x4_e a = *reinterpret_cast<const u32x4_e*>(reinterpret_cast<const char*>(p) + 16 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[4 * h + e] = a[e];
+    }
+  }
+  __device__ __forceinline__ void load_n(const T* p, int n) {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int e = 0; e < W; ++e) w[e] = e < n ? __builtin_bit_cast(unsigned, p[e]) : 0u;
+    } else {
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        const unsigned lo = 2 * e < n ? __builtin_bit_cast(unsigned short, p[2 * e]) : 0u;
+        const unsigned hi = 2 * e + 1 < n ? __builtin_bit_cast(unsigned short, p[2 * e + 1]) : 0u;
+        w[e] = lo | (hi << 16);
+      }
+    }
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int e = 0; e < W; ++e) w[e] = 0u;
+  }
+  __device__ __forceinline__ float at(int e) const {
+    if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, w[e]);
+    else return raw2f<T>(w[e / 2], e & 1);
+  }
+  // row planes
+  __device__ __forceinline__ void rows(uint4 (&q)[Fx<T>::ROWP], FxSeen& seen) const {
+    if constexpr (sizeof(T) == 4) {
+      unsigned* o[3] = {reinterpret_cast<unsigned*>(&q[0]), reinterpret_cast<unsigned*>(&q[1]),
+                        reinterpret_cast<unsigned*>(&q[2])};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        unsigned t[3];
+        split2<3>(at(2 * e), at(2 * e + 1), t);
+        seen.see(t[0]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) o[i][e] = t[i];
+      }
+    } else {
+      q[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+  // transposed-operand planes where they differ (fp16: two bf16 terms)
+  __device__ __forceinline__ void terms(uint4 (&q)[2]) const {
+    unsigned* a = reinterpret_cast<unsigned*>(&q[0]);
+    unsigned* b = reinterpret_cast<unsigned*>(&q[1]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      unsigned t[2];
+      split2<2>(at(2 * e), at(2 * e + 1), t);
+      a[e] = t[0];
+      b[e] = t[1];
+    }
+  }
+};
+
+// A staged operand: BN rows x DP, ROW and/or TR planes.
+template <typename T, int DP, bool ROW, bool TR>
+struct FxOp {
+  static constexpr int BN = Fx<T>::BN, CH = DP / 8, RSB = (CH | 1) * 16;
+  static constexpr int PB = BN * RSB;  // bytes of a plane
+  static constexpr bool SEP = TR && !Fx<T>::SAME;                   // own TR planes
+  static constexpr bool RP = ROW || !SEP;                           // row planes are stored
+  static constexpr int TR0 = SEP ? (ROW ? Fx<T>::ROWP : 0) : 0;     // first TR plane
+  static constexpr int NPL = (RP ? Fx<T>::ROWP : 0) + (SEP ? Fx<T>::TRP : 0);
+  static constexpr int BYTES = NPL * PB;
+  static constexpr int NCH = (BN * CH + kThreads - 1) / kThreads;
+  FxRaw<T> raw[NCH];
+  // rows row0 .. of a [nrows, D] operand; rows past nrows and columns past D become zero.
+  // vec: rows are whole 16-byte (fp32: dword) aligned chunks.
+  __device__ __forceinline__ void load(const T* __restrict__ g, int64_t row0, int64_t nrows,
+                                       int rs, int D, bool vec) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int u = threadIdx.x + i * kThreads, r = u / CH, c = (u % CH) * 8;
+      int64_t row = row0 + r;
+      row = row < nrows ? row : nrows - 1;
+      if (vec) {
+        raw[i].load(g + row * rs + (c < D ? c : 0));
+      } else {
+        raw[i].load_n(g + row * rs + c, D - c);
+      }
+    }
+  }
+  __device__ __forceinline__ void store(char* lds, int64_t row0, int64_t nrows, int D,
+                                        FxSeen& seen) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int u = threadIdx.x + i * kThreads, r = u / CH, c = u % CH;
+      if (BN * CH % kThreads && u >= BN * CH) break;
+      if (row0 + r >= nrows || c * 8 >= D) raw[i].clear();
+      char* d = lds + r * RSB + c * 16;
+      if constexpr (RP) {
+        uint4 q[Fx<T>::ROWP];
+        raw[i].rows(q, seen);
+#pragma unroll
+        for (int p = 0; p < Fx<T>::ROWP; ++p) *reinterpret_cast<uint4*>(d + p * PB) = q[p];
+      }
+      if constexpr (SEP) {
+        uint4 q[2];
+        raw[i].terms(q);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) *reinterpret_cast<uint4*>(d + (TR0 + p) * PB) = q[p];
+      }
+    }
+  }
+};
+
+// A wave's own rows as B operands: lane l32 holds row `row`, chunk 2ks + h per k-step.
+template <typename T, int DP>
+struct FxOwn {
+  typedef typename FxRow<T>::type frag;
+  frag f[DP / 16][Fx<T>::ROWP];
+  __device__ __forceinline__ void load(const T* __restrict__ g, int64_t row, int rs, int D,
+                                       bool vec, int h, FxSeen& seen) {
+#pragma unroll
+    for (int ks = 0; ks < DP / 16; ++ks) {
+      const int c = ks * 16 + h * 8;
+      FxRaw<T> r;
+      if (vec) {
+        r.load(g + row * rs + (c < D ? c : 0));
+        if (c >= D) r.clear();
+      } else {
+        r.load_n(g + row * rs + c, D - c);
+      }
+      uint4 q[Fx<T>::ROWP];
+      r.rows(q, seen);
+#pragma unroll
+      for (int p = 0; p < Fx<T>::ROWP; ++p) f[ks][p] = __builtin_bit_cast(frag, q[p]);
+    }
+  }
+};
+
+__device__ __forceinline__ f32x16 fx_mfma(bfv8 a, bfv8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 fx_mfma(Vec8<tg_half>::type a, Vec8<tg_half>::type b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// C tile of 32 staged rows (at `t`) against the wave's own rows, over the head dim.
+template <typename T, int DP>
+__device__ __forceinline__ f32x16 fx_rows(const char* t, int PB, const FxOwn<T, DP>& own, int l32,
+                                          int h) {
+  typedef typename FxRow<T>::type frag;
+  constexpr int RSB = (DP / 8 | 1) * 16, NP = Fx<T>::ROWP;
+  f32x16 c;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) c[r] = 0.f;
+  const char* b = t + l32 * RSB + h * 16;
+#pragma unroll
+  for (int ks = 0; ks < DP / 16; ++ks) {
+    frag a[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) a[p] = *reinterpret_cast<const frag*>(b + p * PB + ks * 32);
+    if constexpr (NP == 3) {
+      constexpr int PA[6] = {0, 0, 1, 1, 0, 2}, PO[6] = {0, 1, 0, 1, 2, 0};
+#pragma unroll
+      for (int i = 0; i < 6; ++i) c = fx_mfma(a[PA[i]], own.f[ks][PO[i]], c);
+    } else {
+      c = fx_mfma(a[0], own.f[ks][0], c);
+    }
+  }
+  return c;
+}
+
+// The 16 values of a lane's C-tile column as PT bf16 terms, two 8-element k-steps each.
+template <int PT> struct FxP {
+  bfv8 t[PT][2];
+  __device__ __forceinline__ void split(const float (&v)[16]) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      uint4 q[PT];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        unsigned x[PT];
+        split2<PT>(v[8 * s + 2 * e], v[8 * s + 2 * e + 1], x);
+#pragma unroll
+        for (int i = 0; i < PT; ++i) reinterpret_cast<unsigned*>(&q[i])[e] = x[i];
+      }
+#pragma unroll
+      for (int i = 0; i < PT; ++i) t[i][s] = __builtin_bit_cast(bfv8, q[i]);
+    }
+  }
+};
+
+// acc[dt] += products of P (32 staged rows of this sub-tile on the k axis) with the
+// staged operand's columns dt*32 .. +31; TRA: the staged operand is the A operand (the
+// result has the head dim on its rows), else P is.
+template <typename T, int DP, bool TRA>
+__device__ __forceinline__ void fx_acc(f32x16 (&acc)[DP / 32], const char* t, int PB,
+                                       const FxP<Fx<T>::PT>& p, int lane) {
+  constexpr int RSB = (DP / 8 | 1) * 16, NP = Fx<T>::TRP;
+  const int h = lane >> 5, s = lane & 15, nh = (lane >> 4) & 1;
+  const char* b0 = t + (4 * h + (s >> 2)) * RSB + (16 * nh + 4 * (s & 3)) * 2;
+#pragma unroll
+  for (int sg = 0; sg < 2; ++sg)
+#pragma unroll
+    for (int dt = 0; dt < DP / 32; ++dt) {
+      bfv8 x[NP];
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const char* b = b0 + i * PB + sg * 16 * RSB + dt * 64;
+        union {
+          v4i16 q[2];
+          bfv8 v;
+        } u;
+        u.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TG_LDS v4i16*)b);
+        u.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TG_LDS v4i16*)(b + 8 * RSB));
+        x[i] = u.v;
+      }
+      auto mul = [&](int i, int k) {
+        acc[dt] = TRA ? fx_mfma(x[i], p.t[k][sg], acc[dt]) : fx_mfma(p.t[k][sg], x[i], acc[dt]);
+      };
+      mul(0, 0);
+      mul(0, 1);
+      if constexpr (NP >= 2) mul(1, 0);
+      if constexpr (NP == 3) {
+        mul(1, 1);
+        mul(0, 2);
+        mul(2, 0);
+      }
+    }
+}
+
+template <typename T, int DP, int OCC>
+__global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
+    const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
+    T* __restrict__ O0, float* __restrict__ LSE0, int64_t Sq, int64_t Sk, int D, float scale,
+    int causal, int vec, FaLay lay) {
+  using OK = FxOp<T, DP, true, false>;
+  using OV = FxOp<T, DP, false, true>;
+  constexpr int BN = Fx<T>::BN, RSB = OK::RSB, NDB = DP / 32;
+  constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = sizeof(T) == 4 ? gen_lds<DP>() : 0;
+  __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
+  char *ks = sm, *vs = sm + OK::BYTES;
+  int64_t tile, bh;
+  fa_block(tile, bh, lay.G);
+  const T* Q = Q0 + lay.ha(bh, Sq, D);
+  const T* K = K0 + lay.ha(bh, Sk, D);
+  const T* V = V0 + lay.ha(bh, Sk, D);
+  T* O = O0 + lay.ho(bh, Sq, D);
+  float* LSE = LSE0 + bh * Sq;
+  const int rs = lay.rsa, ro = lay.rso;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int h = lane >> 5, l32 = lane & 31;
+  const int64_t qb = causal ? (int64_t)gridDim.x - 1 - tile : tile;
+  const int64_t qw = qb * 128 + wave * 32, q = qw + l32;
+  FxSeen seen;
+  FxOwn<T, DP> own;
+  own.load(Q, q < Sq ? q : Sq - 1, rs, D, vec, h, seen);
+  f32x16 acc[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  const float sl2 = scale * kLog2e;
+  float m = -INFINITY, l = 0.f;
+  const int64_t kend = causal ? (qb * 128 + 128 < Sk ? qb * 128 + 128 : Sk) : Sk;
+  OK ok;
+  OV ov;
+  ok.load(K, 0, Sk, rs, D, vec);
+  ov.load(V, 0, Sk, rs, D, vec);
+  for (int64_t k0 = 0; k0 < kend; k0 += BN) {
+    __syncthreads();
+    ok.store(ks, k0, Sk, D, seen);
+    ov.store(vs, k0, Sk, D, seen);
+    if (k0 + BN < kend) {
+      ok.load(K, k0 + BN, Sk, rs, D, vec);
+      ov.load(V, k0 + BN, Sk, rs, D, vec);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kt = 0; kt < BN / 32; ++kt) {
+      const int64_t kb = k0 + kt * 32;
+      if (kb >= kend || (causal && kb > qw + 31)) break;
+      f32x16 s = fx_rows<T, DP>(ks + kt * 32 * RSB, OK::PB, own, l32, h);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] *= sl2;
+      if (kb + 32 > Sk || (causal && kb + 31 > qw)) {
+        // keys past Sk or past this lane's query
+        int64_t last = Sk - 1 - kb - 4 * h;
+        if (causal && q - kb - 4 * h < last) last = q - kb - 4 * h;
+        const int thr = (int)last;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + (r & 3) > thr) s[r] = -INFINITY;
+      }
+      float mloc = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, s[r]);
+      mloc = xhalf_max(mloc);
+      // O^T and l are rescaled only when some lane's maximum rose by more than kLazy
+      if (__any(mloc > m + kLazy)) {
+        const float mn = fmaxf(m, mloc), alpha = fexp2(m - (mn == -INFINITY ? 0.f : mn));
+        l *= alpha;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        m = mn;
+      }
+      const float mref = m == -INFINITY ? 0.f : m;  // (no key seen yet: p = 0)
+      float p[16], ps = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        p[r] = fexp2(s[r] - mref);
+        ps += p[r];
+      }
+      l += xhalf_sum(ps);
+      FxP<Fx<T>::PT> pt;
+      pt.split(p);
+      fx_acc<T, DP, true>(acc, vs + OV::TR0 * OV::PB + kt * 32 * RSB, OV::PB, pt, lane);
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (__syncthreads_or(seen.bad())) {
+      float* f = reinterpret_cast<float*>(sm);
+      fa_fwd_gen<T, DP>(f, f + gen_lds<DP>() / 8, Q0, K0, V0, O0, LSE0, Sq, Sk, D, scale, causal,
+                        lay);
+      return;
+    }
+  }
+  if (q < Sq) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = 32 * db + 8 * g + 4 * h;
+        T* o = O + q * ro + d;
+        if (vec && d < D) {
+          T w[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w[i] = (T)(acc[db][4 * g + i] * inv);
+          if constexpr (sizeof(T) == 4) {
+            u32x4_e x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = __builtin_bit_cast(unsigned, w[i]);
+            *reinterpret_cast<u32x4_e*>(o) = x;
+          } else {
+            *reinterpret_cast<uint2*>(o) = *reinterpret_cast<const uint2*>(w);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (d + i < D) o[i] = (T)(acc[db][4 * g + i] * inv);
+        }
+      }
+    if (h == 0) LSE[q] = l > 0.f ? (m + log2f(l)) / kLog2e : -INFINITY;
+  }
+}
+
+// out[row][d] (+)= acc (rows row0 + crow, columns dt*32 + l32).
+template <typename T, int DP>
+__device__ __forceinline__ void fx_store(T* __restrict__ out, int rs, int64_t row0, int64_t nrows,
+                                         int D, const f32x16 (&acc)[DP / 32], float mul,
+                                         int accumulate, int l32, int h) {
+#pragma unroll
+  for (int db = 0; db < DP / 32; ++db) {
+    const int d = 32 * db + l32;
+    if (d >= D) continue;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int64_t row = row0 + crow(r, h);
+      if (row < nrows) {
+        T* o = out + row * rs + d;
+        *o = (T)(acc[db][r] * mul + (accumulate ? (float)*o : 0.f));
+      }
+    }
+  }
+}
+
+template <typename T, int DP, int OCC>
+__global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
+    const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
+    const T* __restrict__ O0, const T* __restrict__ dO0, const float* __restrict__ LSE0,
+    float* __restrict__ Dv0, T* __restrict__ dQ0, int64_t Sq, int64_t Sk, int D, float scale,
+    int causal, int accumulate, int vec, FaLay lay) {
+  using OK = FxOp<T, DP, true, true>;
+  using OV = FxOp<T, DP, true, false>;
+  constexpr int BN = Fx<T>::BN, RSB = OK::RSB, NDB = DP / 32;
+  constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = sizeof(T) == 4 ? gen_lds<DP>() : 0;
+  __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
+  char *ks = sm, *vs = sm + OK::BYTES;
+  int64_t tile, bh;
+  fa_block(tile, bh, lay.G);
+  const T* Q = Q0 + lay.ha(bh, Sq, D);
+  const T* O = O0 + lay.ho(bh, Sq, D);
+  const T* dO = dO0 + lay.ho(bh, Sq, D);
+  T* dQ = dQ0 + lay.ha(bh, Sq, D);
+  const T* K = K0 + lay.ha(bh, Sk, D);
+  const T* V = V0 + lay.ha(bh, Sk, D);
+  const float* LSE = LSE0 + bh * Sq;
+  float* Dv = Dv0 + bh * Sq;
+  const int rs = lay.rsa, ro = lay.rso;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int h = lane >> 5, l32 = lane & 31;
+  const int64_t qb = causal ? (int64_t)gridDim.x - 1 - tile : tile;
+  const int64_t qw = qb * 128 + wave * 32, q = qw + l32, qc = q < Sq ? q : Sq - 1;
+  FxSeen seen;
+  FxOwn<T, DP> own, od;
+  own.load(Q, qc, rs, D, vec, h, seen);
+  od.load(dO, qc, ro, D, vec, h, seen);
+  // D = rowsum(dO * O), the lane halves holding alternate 8-column chunks
+  float dsum = 0.f;
+  for (int ks_ = 0; ks_ < DP / 16; ++ks_) {
+    const int c = ks_ * 16 + h * 8;
+    if (c >= D) break;
+    FxRaw<T> a, b;
+    if (vec) {
+      a.load(O + qc * ro + c);
+      b.load(dO + qc * ro + c);
+    } else {
+      a.load_n(O + qc * ro + c, D - c);
+      b.load_n(dO + qc * ro + c, D - c);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dsum += a.at(e) * b.at(e);
+  }
+  dsum += __shfl_xor(dsum, 32, 64);
+  if (h == 0 && q < Sq) Dv[q] = dsum;
+  const float lq = LSE[qc] * kLog2e, sl2 = scale * kLog2e;
+  f32x16 acc[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  const int64_t kend = causal ? (qb * 128 + 128 < Sk ? qb * 128 + 128 : Sk) : Sk;
+  OK ok;
+  OV ov;
+  ok.load(K, 0, Sk, rs, D, vec);
+  ov.load(V, 0, Sk, rs, D, vec);
+  for (int64_t k0 = 0; k0 < kend; k0 += BN) {
+    __syncthreads();
+    ok.store(ks, k0, Sk, D, seen);
+    ov.store(vs, k0, Sk, D, seen);
+    if (k0 + BN < kend) {
+      ok.load(K, k0 + BN, Sk, rs, D, vec);
+      ov.load(V, k0 + BN, Sk, rs, D, vec);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kt = 0; kt < BN / 32; ++kt) {
+      const int64_t kb = k0 + kt * 32;
+      if (kb >= kend || (causal && kb > qw + 31)) break;
+      const f32x16 s = fx_rows<T, DP>(ks + kt * 32 * RSB, OK::PB, own, l32, h);
+      const f32x16 dp = fx_rows<T, DP>(vs + kt * 32 * RSB, OV::PB, od, l32, h);
+      int thr = 1 << 30;
+      if (kb + 32 > Sk || (causal && kb + 31 > qw)) {
+        int64_t last = Sk - 1 - kb - 4 * h;
+        if (causal && q - kb - 4 * h < last) last = q - kb - 4 * h;
+        thr = (int)last;
+      }
+      float ds[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float p = 8 * (r >> 2) + (r & 3) > thr ? 0.f : fexp2(fmaf(s[r], sl2, -lq));
+        ds[r] = p * (dp[r] - dsum) * scale;
+      }
+      FxP<Fx<T>::PT> pt;
+      pt.split(ds);
+      fx_acc<T, DP, false>(acc, ks + OK::TR0 * OK::PB + kt * 32 * RSB, OK::PB, pt, lane);
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (__syncthreads_or(seen.bad())) {
+      float* f = reinterpret_cast<float*>(sm);
+      fa_bwd_dq_gen<T, DP, DP>(f, f + gen_lds<DP>() / 8, Q0, K0, V0, O0, dO0, LSE0, Dv0, dQ0, Sq, Sk,
+                               D, scale, causal, accumulate, lay);
+      return;
+    }
+  }
+  fx_store<T, DP>(dQ, rs, qw, Sq, D, acc, 1.f, accumulate, l32, h);
+}
+
+template <typename T, int DP, int OCC>
+__global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
+    const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
+    const T* __restrict__ dO0, const float* __restrict__ LSE0, const float* __restrict__ Dv0,
+    T* __restrict__ dK0, T* __restrict__ dV0, int64_t Sq, int64_t Sk, int D, float scale,
+    int causal, int accumulate, int vec, FaLay lay) {
+  using OQ = FxOp<T, DP, true, true>;
+  constexpr int BN = Fx<T>::BN, RSB = OQ::RSB, NDB = DP / 32;
+  constexpr int BYTES = 2 * OQ::BYTES, GEN = sizeof(T) == 4 ? gen_lds<DP>() : 0;
+  __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
+  __shared__ __attribute__((aligned(16))) float ls[BN], dsm[BN];
+  char *qs = sm, *dos = sm + OQ::BYTES;
+  int64_t tile, bh;
+  fa_block(tile, bh, lay.G);
+  const T* Q = Q0 + lay.ha(bh, Sq, D);
+  const T* dO = dO0 + lay.ho(bh, Sq, D);
+  const T* K = K0 + lay.ha(bh, Sk, D);
+  const T* V = V0 + lay.ha(bh, Sk, D);
+  T* dK = dK0 + lay.ha(bh, Sk, D);
+  T* dV = dV0 + lay.ha(bh, Sk, D);
+  const float* LSE = LSE0 + bh * Sq;
+  const float* Dv = Dv0 + bh * Sq;
+  const int rs = lay.rsa, ro = lay.rso;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int h = lane >> 5, l32 = lane & 31;
+  // causal: the first key blocks see the most queries, so they are dispatched first
+  const int64_t kblk = tile * 128, kw = kblk + wave * 32, key = kw + l32;
+  FxSeen seen;
+  FxOwn<T, DP> kf, vf;
+  kf.load(K, key < Sk ? key : Sk - 1, rs, D, vec, h, seen);
+  vf.load(V, key < Sk ? key : Sk - 1, rs, D, vec, h, seen);
+  const float sl2 = scale * kLog2e;
+  f32x16 dk[NDB], dv[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.f;
+  const int64_t qstart = causal ? kblk : 0;
+  OQ oq, od;
+  float lv = 0.f, dd = 0.f;
+  auto rows = [&](int64_t q0) {
+    const int64_t qq = q0 + (threadIdx.x % BN), qc = qq < Sq ? qq : Sq - 1;
+    lv = LSE[qc];
+    dd = Dv[qc];
+  };
+  if (qstart < Sq) {
+    rows(qstart);
+    oq.load(Q, qstart, Sq, rs, D, vec);
+    od.load(dO, qstart, Sq, ro, D, vec);
+  }
+  for (int64_t q0 = qstart; q0 < Sq; q0 += BN) {
+    __syncthreads();
+    oq.store(qs, q0, Sq, D, seen);
+    od.store(dos, q0, Sq, D, seen);
+    if (threadIdx.x < BN) {  // (+inf past Sq: P = 0 there)
+      ls[threadIdx.x] = q0 + threadIdx.x < Sq ? lv * kLog2e : INFINITY;
+      dsm[threadIdx.x] = q0 + threadIdx.x < Sq ? dd : 0.f;
+    }
+    if (q0 + BN < Sq) {
+      rows(q0 + BN);
+      oq.load(Q, q0 + BN, Sq, rs, D, vec);
+      od.load(dO, q0 + BN, Sq, ro, D, vec);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < BN / 32; ++t) {
+      const int64_t qb0 = q0 + t * 32;
+      if (qb0 >= Sq) break;
+      if (causal && qb0 + 31 < kw) continue;  // wholly before this wave's keys
+      const f32x16 s = fx_rows<T, DP>(qs + t * 32 * RSB, OQ::PB, kf, l32, h);
+      const f32x16 dp = fx_rows<T, DP>(dos + t * 32 * RSB, OQ::PB, vf, l32, h);
+      const bool diag = causal && kw + 31 > qb0;
+      const int mb = diag ? (int)(key - qb0) - 4 * h : -1;  // rows below it are masked
+      float p[16], ds[16];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 a = *reinterpret_cast<const float4*>(ls + t * 32 + 8 * g + 4 * h);
+        const float4 b = *reinterpret_cast<const float4*>(dsm + t * 32 + 8 * g + 4 * h);
+        const float la[4] = {a.x, a.y, a.z, a.w}, db[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * g + i;
+          p[r] = 8 * g + i < mb ? 0.f : fexp2(fmaf(s[r], sl2, -la[i]));
+          ds[r] = p[r] * (dp[r] - db[i]) * scale;
+        }
+      }
+      FxP<Fx<T>::PT> pt;
+      pt.split(p);
+      fx_acc<T, DP, false>(dv, dos + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
+      pt.split(ds);
+      fx_acc<T, DP, false>(dk, qs + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (__syncthreads_or(seen.bad())) {
+      float* f = reinterpret_cast<float*>(sm);
+      fa_bwd_dkdv_gen<T, DP, DP>(f, f + gen_lds<DP>() / 8, ls, dsm, Q0, K0, V0, dO0, LSE0, Dv0, dK0,
+                                 dV0, Sq, Sk, D, scale, causal, accumulate, lay);
+      return;
+    }
+  }
+  fx_store<T, DP>(dK, rs, kw, Sk, D, dk, 1.f, accumulate, l32, h);
+  fx_store<T, DP>(dV, rs, kw, Sk, D, dv, 1.f, accumulate, l32, h);
+}
+
+template <typename T, int DP> struct FxOcc {
+  // workgroups per CU that the registers allow without spills
+  static constexpr int FWD = sizeof(T) == 4 && DP > 64 ? 1 : 2;
+  static constexpr int DQ = sizeof(T) == 4 && DP > 64 ? 1 : 2;
+  static constexpr int DKDV = sizeof(T) == 4 ? (DP > 32 ? 1 : 2) : (DP > 64 ? 1 : 2);
+};
+
+template <typename T, int DP>
+int fwd_split_t(const void* q, const void* k, const void* v, void* o, float* lse, int64_t BH,
+                int64_t Sq, int64_t Sk, int D, float scale, int causal, int vec, FaLay lay,
+                hipStream_t s) {
+  dim3 grid((unsigned)((Sq + 127) / 128), (unsigned)BH);
+  k_fa_fwd_split<T, DP, FxOcc<T, DP>::FWD><<<grid, kThreads, 0, s>>>(
+      (const T*)q, (const T*)k, (const T*)v, (T*)o, lse, Sq, Sk, D, scale, causal, vec, lay);
+  return tg_check_launch("tg_flash_attn_fwd");
+}
+template <typename T, int DP>
+int bwd_split_t(const void* q, const void* k, const void* v, const void* o, const void* dout,
+                const float* lse, void* dq, void* dk, void* dv, int64_t BH, int64_t Sq, int64_t Sk,
+                int D, float scale, int causal, int acc, float* dvec, int vec, FaLay lay,
+                hipStream_t s) {
+  dim3 gq((unsigned)((Sq + 127) / 128), (unsigned)BH);
+  k_fa_bwd_dq_split<T, DP, FxOcc<T, DP>::DQ><<<gq, kThreads, 0, s>>>(
+      (const T*)q, (const T*)k, (const T*)v, (const T*)o, (const T*)dout, lse, dvec, (T*)dq, Sq, Sk,
+      D, scale, causal, acc, vec, lay);
+  dim3 gkv((unsigned)((Sk + 127) / 128), (unsigned)BH);
+  k_fa_bwd_dkdv_split<T, DP, FxOcc<T, DP>::DKDV><<<gkv, kThreads, 0, s>>>(
+      (const T*)q, (const T*)k, (const T*)v, (const T*)dout, lse, dvec, (T*)dk, (T*)dv, Sq, Sk, D,
+      scale, causal, acc, vec, lay);
+  return tg_check_launch("tg_flash_attn_bwd");
+}
+
+// Whether every row of these operands is made of whole chunks the kernels may load 16
+// bytes (fp32: 8 dwords) at a time.
+bool fx_vec(int dtype, int64_t D, const FaLay& lay, std::initializer_list<const void*> ptrs) {
+  if (D % 8) return false;
+  if (dtype == TG_F32) return true;
+  for (const void* p : ptrs)
+    if (!tg_aligned16(p)) return false;
+  return lay.rsa % 8 == 0 && lay.rso % 8 == 0;
+}
+
+// Padded head dims: the split-operand kernels up to 128, the generic ones past it.
+#define TG_FX_DP(X) X(32) X(64) X(96) X(128)
+#define TG_GEN_DP(X) X(192) X(256)
 
 int gen_dp(int64_t D) {
   if (D <= 32) return 32;
@@ -1415,8 +2150,13 @@ int gen_dp(int64_t D) {
 
 template <typename T>
 int fwd_gen(const void* q, const void* k, const void* v, void* o, float* lse, int64_t BH,
-            int64_t Sq, int64_t Sk, int D, float scale, int causal, FaLay lay, hipStream_t s) {
+            int64_t Sq, int64_t Sk, int D, float scale, int causal, int vec, FaLay lay,
+            hipStream_t s) {
   switch (gen_dp(D)) {
+#define C(DP) \
+  case DP: return fwd_split_t<T, DP>(q, k, v, o, lse, BH, Sq, Sk, D, scale, causal, vec, lay, s);
+    TG_FX_DP(C)
+#undef C
 #define C(DP) \
   case DP: return fwd_gen_t<T, DP>(q, k, v, o, lse, BH, Sq, Sk, D, scale, causal, lay, s);
     TG_GEN_DP(C)
@@ -1428,8 +2168,14 @@ int fwd_gen(const void* q, const void* k, const void* v, void* o, float* lse, in
 template <typename T>
 int bwd_gen(const void* q, const void* k, const void* v, const void* o, const void* dout,
             const float* lse, void* dq, void* dk, void* dv, int64_t BH, int64_t Sq, int64_t Sk,
-            int D, float scale, int causal, int acc, float* dvec, FaLay lay, hipStream_t s) {
+            int D, float scale, int causal, int acc, float* dvec, int vec, FaLay lay,
+            hipStream_t s) {
   switch (gen_dp(D)) {
+#define C(DP)                                                                                  \
+  case DP: return bwd_split_t<T, DP>(q, k, v, o, dout, lse, dq, dk, dv, BH, Sq, Sk, D, scale, \
+                                     causal, acc, dvec, vec, lay, s);
+    TG_FX_DP(C)
+#undef C
 #define C(DP)                                                                                  \
   case DP: return bwd_gen_t<T, DP>(q, k, v, o, dout, lse, dq, dk, dv, BH, Sq, Sk, D, scale,   \
                                    causal, acc, dvec, lay, s);
@@ -1535,7 +2281,7 @@ int fa_fwd(int dtype, const void* q, const void* k, const void* v, void* o, floa
     void* oc = (void*)off(o, b0 * H * Sq * D, es);
     float* lc = lse + b0 * H * Sq;
     const FaLay lay = fa_lay(layout, H, D, fa_group(BH, causal, 1));
-    const int Di = (int)D;
+    const int Di = (int)D, vec = fx_vec(dtype, D, lay, {qc, kc, vc, oc});
     if (fast) {
       if (dtype == TG_F16)
         st = D == 64 ? fwd_t<tg_half, 64>(qc, kc, vc, oc, lc, BH, Sq, Sk, scale, causal, lay, s)
@@ -1544,11 +2290,11 @@ int fa_fwd(int dtype, const void* q, const void* k, const void* v, void* o, floa
         st = D == 64 ? fwd_t<tg_bf16, 64>(qc, kc, vc, oc, lc, BH, Sq, Sk, scale, causal, lay, s)
                      : fwd_t<tg_bf16, 128>(qc, kc, vc, oc, lc, BH, Sq, Sk, scale, causal, lay, s);
     } else if (dtype == TG_F32) {
-      st = fwd_gen<float>(qc, kc, vc, oc, lc, BH, Sq, Sk, Di, scale, causal, lay, s);
+      st = fwd_gen<float>(qc, kc, vc, oc, lc, BH, Sq, Sk, Di, scale, causal, vec, lay, s);
     } else if (dtype == TG_F16) {
-      st = fwd_gen<tg_half>(qc, kc, vc, oc, lc, BH, Sq, Sk, Di, scale, causal, lay, s);
+      st = fwd_gen<tg_half>(qc, kc, vc, oc, lc, BH, Sq, Sk, Di, scale, causal, vec, lay, s);
     } else {
-      st = fwd_gen<tg_bf16>(qc, kc, vc, oc, lc, BH, Sq, Sk, Di, scale, causal, lay, s);
+      st = fwd_gen<tg_bf16>(qc, kc, vc, oc, lc, BH, Sq, Sk, Di, scale, causal, vec, lay, s);
     }
     if (st) return st;
   }
@@ -1585,7 +2331,7 @@ int fa_bwd(int dtype, const void* q, const void* k, const void* v, const void* o
     const float* lc = lse + b0 * H * Sq;
     float* dvec = (float*)workspace + b0 * H * Sq;
     const FaLay lay = fa_lay(layout, H, D, fa_group_bwd(BH, causal, Sq > Sk ? Sq : Sk, D));
-    const int Di = (int)D;
+    const int Di = (int)D, vec = fx_vec(dtype, D, lay, {qc, kc, vc, oc, gc, dqc, dkc, dvc});
     if (fast) {
       if (dtype == TG_F16)
         st = D == 64 ? bwd_t<tg_half, 64>(qc, kc, vc, oc, gc, lc, dqc, dkc, dvc, BH, Sq, Sk,
@@ -1599,13 +2345,13 @@ int fa_bwd(int dtype, const void* q, const void* k, const void* v, const void* o
                                            scale, causal, accumulate, dvec, lay, s);
     } else if (dtype == TG_F32) {
       st = bwd_gen<float>(qc, kc, vc, oc, gc, lc, dqc, dkc, dvc, BH, Sq, Sk, Di, scale, causal,
-                          accumulate, dvec, lay, s);
+                          accumulate, dvec, vec, lay, s);
     } else if (dtype == TG_F16) {
       st = bwd_gen<tg_half>(qc, kc, vc, oc, gc, lc, dqc, dkc, dvc, BH, Sq, Sk, Di, scale, causal,
-                            accumulate, dvec, lay, s);
+                            accumulate, dvec, vec, lay, s);
     } else {
       st = bwd_gen<tg_bf16>(qc, kc, vc, oc, gc, lc, dqc, dkc, dvc, BH, Sq, Sk, Di, scale, causal,
-                            accumulate, dvec, lay, s);
+                            accumulate, dvec, vec, lay, s);
     }
     if (st) return st;
   }

@@ -1,0 +1,112 @@
+"""FlashAttention on the split-operand kernels (fp32; fp16 / bf16 head dims other than 64 and
+128) against float64, at the edges of their tiles, head dims and layouts, and fp32 values
+outside the split's range."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DT = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}
+
+
+def L():
+    from tensor_gpu_v2 import _lib
+    return _lib
+
+
+def _ref(q, k, v, do, scale, causal):
+    q, k, v = (t.double().detach().requires_grad_(True) for t in (q, k, v))
+    s = (q * scale) @ k.transpose(-1, -2).contiguous()
+    if causal:
+        m = torch.triu(torch.ones(s.shape[-2:], dtype=torch.bool, device="cuda"), 1)
+        s = s.masked_fill(m, -float("inf"))
+    o = torch.softmax(s, -1) @ v
+    return [o.detach()] + list(torch.autograd.grad(o, (q, k, v), do.double()))
+
+
+def _close(got, want, dt, what, extra=1.0):
+    """2-norm: fp32 sums of up to 2^11 terms and exponentials of O(10) arguments, a few
+    2^-24 each; 16-bit results are rounded once (and o, which D is formed from, too)."""
+    lim = {torch.float32: 3e-6, torch.float16: 1e-3, torch.bfloat16: 8e-3}[dt] * extra
+    e = float((got.double() - want).norm() / want.norm().clamp_min(1e-30))
+    assert e < lim, f"{what}: {e:.2e}"
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("D", [1, 8, 20, 32, 33, 64, 72, 80, 96, 100, 128])
+@pytest.mark.parametrize("Sq,Sk,causal", [(1, 1, False), (33, 33, True), (128, 128, True),
+                                          (65, 200, False), (300, 31, False), (257, 257, True)])
+def test_split_attention(cuda, D, Sq, Sk, causal, dt):
+    dt = DT[dt]
+    g = torch.Generator(device="cuda").manual_seed(D * 1000 + Sq + Sk)
+    for layout in (0, 1):
+        def mk(S):
+            if layout == 0:
+                return torch.randn(2, 3, S, D, generator=g, device="cuda").to(dt)
+            return torch.randn(2, S, 3, D, generator=g, device="cuda").to(dt).permute(0, 2, 1, 3)
+        q, k, v, do = mk(Sq), mk(Sk), mk(Sk), mk(Sq)
+        sc = D ** -0.5
+        o, lse = L().flash_attn_fwd(q, k, v, sc, causal, layout)
+        grads = [L().fa_empty(2, 3, S, D, dt, q.device, layout) for S in (Sq, Sk, Sk)]
+        for t in grads:
+            t.fill_(0.5)
+        L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, causal, True, layout)
+        want = _ref(q, k, v, do, sc, causal)
+        _close(o, want[0], dt, "o")
+        for t, w, n in zip(grads, want[1:], ("dq", "dk", "dv")):
+            if float(w.norm()) > 1e-9:  # (one key: dq and dk are zero)
+                _close(t, w + 0.5, dt, n, 2.0)
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("D", [32, 80])
+def test_split_attention_packed(cuda, D, dt):
+    dt = DT[dt]
+    B, S, H = 2, 190, 4
+    g = torch.Generator(device="cuda").manual_seed(D)
+    qkv = torch.randn(B, S, 3 * H * D, generator=g, device="cuda").to(dt)
+    do = torch.randn(B, S, H * D, generator=g, device="cuda").to(dt)
+    o, lse = L().flash_attn_fwd_qkv(qkv, H, D ** -0.5, True)
+    d = torch.empty_like(qkv)
+    L().flash_attn_bwd_qkv(qkv, o, do, lse, d, H, D ** -0.5, True, False)
+    q, k, v = (t.permute(0, 2, 1, 3) for t in qkv.reshape(B, S, 3, H, D).unbind(2))
+    want = _ref(q, k, v, do.reshape(B, S, H, D).permute(0, 2, 1, 3), D ** -0.5, True)
+    back = [t.permute(0, 2, 1, 3).reshape(B, S, H * D) for t in want]
+    _close(o, back[0], dt, "o")
+    _close(d, torch.cat(back[1:], -1), dt, "dqkv", 2.0)
+
+
+@pytest.mark.parametrize("D", [24, 64, 128])
+@pytest.mark.parametrize("kind", ["tiny", "huge", "negative_scale", "large_scores", "inf"])
+def test_split_attention_fp32_extremes(cuda, D, kind):
+    """Operands that the bf16 split cannot hold run on the fp32 matrix cores."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    mk = lambda: torch.randn(1, 2, 150, D, generator=g, device="cuda")  # noqa: E731
+    q, k, v, do = mk(), mk(), mk(), mk()
+    sc = D ** -0.5
+    if kind == "tiny":
+        v *= 1e-34
+        do[0, 0, 3] *= 1e-33
+    elif kind == "huge":
+        v[0, 1, 7] *= 1e38
+        do *= 1e-10
+    elif kind == "negative_scale":
+        sc = -0.4
+    elif kind == "large_scores":
+        q *= 40.0
+        k -= 3.0
+    elif kind == "inf":
+        v[0, 0, 11, 2] = float("inf")
+    o, lse = L().flash_attn_fwd(q, k, v, sc, False)
+    want = _ref(q, k, v, do, sc, False)
+    if kind == "inf":
+        assert torch.equal(torch.isfinite(o), torch.isfinite(want[0]))
+        return
+    if kind == "huge":
+        assert torch.equal(torch.isfinite(o), torch.isfinite(want[0].float()))
+    ok = torch.isfinite(want[0].float())
+    _close(o[ok], want[0][ok], torch.float32, "o", 200.0 if kind == "large_scores" else 2.0)
+    grads = [torch.empty_like(q) for _ in range(3)]
+    L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, False, False)
+    if kind in ("tiny", "negative_scale"):
+        for t, w, n in zip(grads, want[1:], ("dq", "dk", "dv")):
+            _close(t, w, torch.float32, n, 10.0)
