@@ -941,8 +941,10 @@ bool v3_ok(int elem, int ta, int tb, int64_t M, int64_t N, int64_t K, const void
 // Block shape and K split of a 16-bit product: the fastest by the times (us) measured per
 // 64-deep k-tile with every CU busy: 256x256 blocks (4x2 waves of 64x128) 1.85,
 // 256x128 (4x2 of 64x64) 1.02, both one block per CU; 128x128 (2x2 of 64x64) 1.08 with
-// two blocks per CU, 0.75 with one; a block's start and store take 4-6.  A K split (chunks
-// of a multiple of 64) adds its finishing launch: 6 us and its traffic at 4.5 TB/s.
+// two blocks on every CU, 0.9 with two on a few, 0.7 with one; a block's start and store
+// take 4-6.  A K split (chunks of a multiple of 64) adds its finishing launch: 4 us and its
+// traffic at 6 TB/s (whole and in two: 2048x1024x4096 41 and 31 us, 3072x768x3072 33 and 30,
+// 4096x1024x4096 45 and 47, so whole).
 // (256x256 as 2x2 waves of 128x128, one wave per SIMD, measured 3-8 % slower: nothing
 // overlaps a wave's LDS waits and barrier.)
 struct V3Plan {
@@ -964,13 +966,14 @@ V3Plan v3_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool can_split) {
     // (a split's partial sums stay within 256 MiB)
     if (S > 1 && (double)S * (double)M * (double)N * 4.0 > 268435456.0) break;
     const double kt = (double)((kc + 63) / 64);
-    const double fin = S > 1 ? 6.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 4.5e6 : 0.0;
+    const double fin = S > 1 ? 4.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 6e6 : 0.0;
     double t[3];
     t[2] = std::ceil(tiles(256, 256) * S / ncu) * (kt * 1.85 + 6.0);
     t[1] = std::ceil(tiles(256, 128) * S / ncu) * (kt * 1.02 + 5.0);
     const double b = tiles(128, 128) * S, pairs = std::floor(b / (2 * ncu));
     const double rest = b - pairs * 2 * ncu;
-    t[0] = pairs * (kt * 1.08 + 4.0) + (rest > 0 ? kt * (rest > ncu ? 1.08 : 0.75) + 4.0 : 0.0);
+    const double tk = rest > ncu ? 0.9 + 0.18 * (rest - ncu) / ncu : 0.7;
+    t[0] = pairs * (kt * 1.08 + 4.0) + (rest > 0 ? kt * tk + 4.0 : 0.0);
     for (int i = 2; i >= 0; --i)
       if (t[i] + fin < tbest) {
         tbest = t[i] + fin;
@@ -1103,7 +1106,13 @@ int launch_epi(int epi, int64_t M, int64_t N, int64_t K, const void* A, int64_t 
     tg_set_error("tg_gemm_epilogue: shape or alignment outside the fused kernel");
     return TG_ERR_UNSUPPORTED;
   }
-  const int shape = v3_plan(M, N, K, 1, false).shape;
+  // 256x256 blocks only where they fill the CUs: their epilogues stream two outputs or an
+  // operand more, which 156 of 256 CUs do slower than 256x128 blocks on all of them
+  // (3136x3072x768, GELU backward: 73 and 59 us)
+  const int64_t ncu = tg_num_cus();
+  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256);
+  const int64_t t128 = ((M + 255) / 256) * ((N + 127) / 128);
+  const int shape = t256 >= ncu ? 2 : (t128 >= ncu ? 1 : 0);
   const T* a = (const T*)A;
   const T* b = (const T*)B;
 #define TG_GE(TB_, E, WGM, WGN, SM, SN, OCC)                                                   \
