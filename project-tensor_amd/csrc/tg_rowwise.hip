@@ -6,9 +6,10 @@
 // Register path: a row is split across TPR threads (a wavefront when TPR=64,
 // the whole 256-thread block when TPR=256), each thread holding VPT 16-byte
 // vectors, so every element of x/y/dy is read from HBM exactly once.  Row sums
-// use wavefront butterflies plus one LDS exchange when TPR=256.  Shapes that do
-// not fit (cols not a multiple of the vector width, misaligned, or very wide)
-// take the looping wavefront-per-row path, which re-reads the row from cache.
+// use wavefront butterflies plus one LDS exchange when TPR=256.  RAG instances take
+// the rows that do not start on 16 bytes (cols not a multiple of the vector width,
+// or a misaligned base).  Very wide rows, and ragged ones of at most 16 vectors, take
+// the looping wavefront-per-row path, which re-reads the row from cache.
 #include "tg_common.h"
 
 #include <mutex>
@@ -43,9 +44,64 @@ __device__ __forceinline__ float group_max(float v, float* red) {
   return v;
 }
 
+// Vector number `vi` of a row at p, elements from row_c0 on.  RAG: the row starts at any
+// element, so the vector is one 16-byte access aligned to its elements only (global memory
+// takes those).  The last vector of a row with cols % V != 0 is the row's last V elements
+// (cols >= V): its first `row_dup` ones belong to the vector before it, load as `fill` and
+// are not stored.  (Loading the last cols % V elements one by one instead puts their latency
+// into every row: LayerNorm backward fp16 [32768, 101] 28 us by the looping kernels, 49 so.)
+typedef unsigned row_u32x4 __attribute__((ext_vector_type(4), aligned(2), may_alias));
+template <typename T, bool RAG>
+__device__ __forceinline__ int row_c0(int vi, int cols) {
+  constexpr int V = tg_vec16<T>::N;
+  return RAG && vi * V + V > cols ? cols - V : vi * V;
+}
+template <typename T, bool RAG>
+__device__ __forceinline__ int row_dup(int vi, int cols) {
+  return vi * tg_vec16<T>::N - row_c0<T, RAG>(vi, cols);
+}
+template <typename T, bool RAG, bool NT>
+__device__ __forceinline__ tg_vec16<T> row_ld_all(const T* p, int vi, int cols) {
+  if constexpr (!RAG) {
+    return tg_ld16<NT>(p + vi * tg_vec16<T>::N);
+  } else {
+    tg_vec16<T> r;
+    const row_u32x4 u = *reinterpret_cast<const row_u32x4*>(p + row_c0<T, RAG>(vi, cols));
+    __builtin_memcpy(&r, &u, 16);
+    return r;
+  }
+}
+template <typename T, bool RAG, bool NT>
+__device__ __forceinline__ tg_vec16<T> row_ld(const T* p, int vi, int cols, float fill) {
+  tg_vec16<T> r = row_ld_all<T, RAG, NT>(p, vi, cols);
+  if constexpr (RAG) {
+    const int dup = row_dup<T, RAG>(vi, cols);
+#pragma unroll
+    for (int j = 0; j < tg_vec16<T>::N - 1; ++j)
+      if (j < dup) r.v[j] = tg_from_float<T>(fill);
+  }
+  return r;
+}
+template <typename T, bool RAG, bool NT>
+__device__ __forceinline__ void row_st(T* p, int vi, int cols, const tg_vec16<T>& r) {
+  constexpr int V = tg_vec16<T>::N;
+  if constexpr (!RAG) {
+    tg_st16<NT>(p + vi * V, r);
+  } else if (vi * V + V <= cols) {
+    row_u32x4 u;
+    __builtin_memcpy(&u, &r, 16);
+    *reinterpret_cast<row_u32x4*>(p + vi * V) = u;
+  } else {
+    const int dup = row_dup<T, RAG>(vi, cols);
+#pragma unroll
+    for (int j = 1; j < V; ++j)
+      if (j >= dup) p[cols - V + j] = r.v[j];
+  }
+}
+
 // ============================ softmax ======================================
 // Forward: y = exp(x - max) / sum(exp(x - max))   (_core.py:1286-1292)
-template <typename T, int TPR, int VPT>
+template <typename T, int TPR, int VPT, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_softmax_fwd_reg(const T* __restrict__ x,
                                                             T* __restrict__ y, int64_t rows,
                                                             int cols) {
@@ -55,7 +111,7 @@ __global__ __launch_bounds__(kBlock) void k_softmax_fwd_reg(const T* __restrict_
   const int t = threadIdx.x % TPR;
   const int64_t row = (int64_t)blockIdx.x * G + threadIdx.x / TPR;
   const bool live = row < rows;
-  const int nv = cols / V;
+  const int nv = (cols + V - 1) / V;
   const T* xr = x + (live ? row : 0) * (int64_t)cols;
   float xv[VPT][V];
   float m = -INFINITY;
@@ -63,7 +119,7 @@ __global__ __launch_bounds__(kBlock) void k_softmax_fwd_reg(const T* __restrict_
   for (int k = 0; k < VPT; ++k) {
     const int vi = t + k * TPR;
     if (live && vi < nv) {
-      tg_vec16<T> a = tg_load16(xr + vi * V);
+      tg_vec16<T> a = row_ld<T, RAG, false>(xr, vi, cols, -INFINITY);
 #pragma unroll
       for (int j = 0; j < V; ++j) {
         xv[k][j] = tg_to_float(a.v[j]);
@@ -95,13 +151,13 @@ __global__ __launch_bounds__(kBlock) void k_softmax_fwd_reg(const T* __restrict_
       tg_vec16<T> o;
 #pragma unroll
       for (int j = 0; j < V; ++j) o.v[j] = tg_from_float<T>(xv[k][j] * inv);
-      tg_store16(yr + vi * V, o);
+      row_st<T, RAG, false>(yr, vi, cols, o);
     }
   }
 }
 
 // Backward: dx (+)= y * (dy - sum(dy * y))   (_core.py:1294-1297)
-template <typename T, int TPR, int VPT, bool ACC, bool NT>
+template <typename T, int TPR, int VPT, bool ACC, bool NT, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_softmax_bwd_reg(const T* __restrict__ y,
                                                             const T* __restrict__ dy,
                                                             T* __restrict__ dx, int64_t rows,
@@ -112,7 +168,7 @@ __global__ __launch_bounds__(kBlock) void k_softmax_bwd_reg(const T* __restrict_
   const int t = threadIdx.x % TPR;
   const int64_t row = (int64_t)blockIdx.x * G + threadIdx.x / TPR;
   const bool live = row < rows;
-  const int nv = cols / V;
+  const int nv = (cols + V - 1) / V;
   const int64_t off = (live ? row : 0) * (int64_t)cols;
   tg_vec16<T> yv[VPT], gv[VPT];
   float s[1] = {0.f};
@@ -120,8 +176,8 @@ __global__ __launch_bounds__(kBlock) void k_softmax_bwd_reg(const T* __restrict_
   for (int k = 0; k < VPT; ++k) {
     const int vi = t + k * TPR;
     if (live && vi < nv) {
-      yv[k] = tg_ld16<NT>(y + off + vi * V);
-      gv[k] = tg_ld16<NT>(dy + off + vi * V);
+      yv[k] = row_ld<T, RAG, NT>(y + off, vi, cols, 0.f);
+      gv[k] = row_ld<T, RAG, NT>(dy + off, vi, cols, 0.f);
 #pragma unroll
       for (int j = 0; j < V; ++j) s[0] += tg_to_float(yv[k].v[j]) * tg_to_float(gv[k].v[j]);
     }
@@ -133,14 +189,14 @@ __global__ __launch_bounds__(kBlock) void k_softmax_bwd_reg(const T* __restrict_
     const int vi = t + k * TPR;
     if (vi < nv) {
       tg_vec16<T> o;
-      if (ACC) o = tg_ld16<NT>(dx + off + vi * V);
+      if (ACC) o = row_ld<T, RAG, NT>(dx + off, vi, cols, 0.f);
 #pragma unroll
       for (int j = 0; j < V; ++j) {
         float r = tg_to_float(yv[k].v[j]) * (tg_to_float(gv[k].v[j]) - s[0]);
         if (ACC) r += tg_to_float(o.v[j]);
         o.v[j] = tg_from_float<T>(r);
       }
-      tg_st16<NT>(dx + off + vi * V, o);
+      row_st<T, RAG, NT>(dx + off, vi, cols, o);
     }
   }
 }
@@ -190,13 +246,26 @@ __global__ __launch_bounds__(kBlock) void k_softmax_bwd_loop(const T* __restrict
   }
 }
 
-// Choose threads-per-row and vectors-per-thread for the register path.
-// Returns false if the row does not fit the register path.
+// Choose threads-per-row and vectors-per-thread for the register path, and whether its
+// rows are ragged.  Returns false if the row does not fit the register path.
+// Ragged rows, us by the looping kernels (element loads, the row read two or three times,
+// one wavefront per row) and by the register path, forward + backward:
+//                          softmax      LayerNorm
+//   fp32 [22182,   311]   33 ->  26     56 ->  43
+//   fp32 [ 8192,  1023]   46 ->  28     64 ->  39
+//   fp32 [32768,  2047]  461 -> 237    627 -> 274
+//   fp16 [ 1856,  1881]   23 ->  11     41 ->  26
+//   fp16 [ 4096,  4095]  102 ->  32    137 ->  60
+//   fp16 [32768,   101]   19 ->  21     40 ->  47
+// The last: 13 vectors leave 51 of 64 lanes idle, the loop's two elements a lane none; fp32
+// [32768, 65], 17 vectors, 20 -> 17 and 41 -> 38.  So the register path from 17 vectors on.
 template <typename T>
-bool pick_reg_shape(int64_t cols, bool aligned, int* tpr, int* vpt) {
+bool pick_reg_shape(int64_t cols, bool aligned, int* tpr, int* vpt, bool* rag) {
   constexpr int V = tg_vec16<T>::N;
-  if (!aligned || cols % V != 0 || cols <= 0) return false;
-  const int64_t nv = cols / V;
+  if (cols < V) return false;
+  const int64_t nv = (cols + V - 1) / V;
+  *rag = !aligned || cols % V != 0;
+  if (*rag && nv <= 16) return false;
   if (nv <= 64 * 4) {
     *tpr = 64;
     *vpt = nv <= 64 ? 1 : nv <= 128 ? 2 : 4;
@@ -224,11 +293,17 @@ bool pick_reg_shape(int64_t cols, bool aligned, int* tpr, int* vpt) {
 template <typename T>
 int softmax_fwd_t(const void* x, void* y, int64_t rows, int64_t cols, hipStream_t s) {
   int tpr = 0, vpt = 0;
-  if (pick_reg_shape<T>(cols, tg_aligned16(x) && tg_aligned16(y), &tpr, &vpt)) {
+  bool rag = false;
+  if (pick_reg_shape<T>(cols, tg_aligned16(x) && tg_aligned16(y), &tpr, &vpt, &rag)) {
     const int64_t g = kBlock / tpr;
     const unsigned blocks = (unsigned)((rows + g - 1) / g);
-#define L(TPR, VPT) \
-  k_softmax_fwd_reg<T, TPR, VPT><<<blocks, kBlock, 0, s>>>((const T*)x, (T*)y, rows, (int)cols)
+#define L(TPR, VPT)                                                                           \
+  if (rag)                                                                                    \
+    k_softmax_fwd_reg<T, TPR, VPT, true><<<blocks, kBlock, 0, s>>>((const T*)x, (T*)y, rows,  \
+                                                                   (int)cols);                \
+  else                                                                                        \
+    k_softmax_fwd_reg<T, TPR, VPT, false><<<blocks, kBlock, 0, s>>>((const T*)x, (T*)y, rows, \
+                                                                    (int)cols)
     TG_REG_DISPATCH(L)
 #undef L
   } else {
@@ -242,22 +317,25 @@ template <typename T>
 int softmax_bwd_t(const void* y, const void* dy, void* dx, int64_t rows, int64_t cols, int acc,
                   hipStream_t s) {
   int tpr = 0, vpt = 0;
+  bool rag = false;
   const bool al = tg_aligned16(y) && tg_aligned16(dy) && tg_aligned16(dx);
-  if (pick_reg_shape<T>(cols, al, &tpr, &vpt)) {
+  if (pick_reg_shape<T>(cols, al, &tpr, &vpt, &rag)) {
     const int64_t g = kBlock / tpr;
     const unsigned blocks = (unsigned)((rows + g - 1) / g);
     const bool nt = (int64_t)sizeof(T) * rows * cols >= kNtBytes;
 #define SMARGS (const T*)y, (const T*)dy, (T*)dx, rows, (int)cols
     if (acc) {
 #define L(TPR, VPT)                                                                            \
-  if (nt) k_softmax_bwd_reg<T, TPR, VPT, true, true><<<blocks, kBlock, 0, s>>>(SMARGS); \
-  else k_softmax_bwd_reg<T, TPR, VPT, true, false><<<blocks, kBlock, 0, s>>>(SMARGS)
+  if (rag) k_softmax_bwd_reg<T, TPR, VPT, true, false, true><<<blocks, kBlock, 0, s>>>(SMARGS); \
+  else if (nt) k_softmax_bwd_reg<T, TPR, VPT, true, true, false><<<blocks, kBlock, 0, s>>>(SMARGS); \
+  else k_softmax_bwd_reg<T, TPR, VPT, true, false, false><<<blocks, kBlock, 0, s>>>(SMARGS)
       TG_REG_DISPATCH(L)
 #undef L
     } else {
-#define L(TPR, VPT)                                                                             \
-  if (nt) k_softmax_bwd_reg<T, TPR, VPT, false, true><<<blocks, kBlock, 0, s>>>(SMARGS); \
-  else k_softmax_bwd_reg<T, TPR, VPT, false, false><<<blocks, kBlock, 0, s>>>(SMARGS)
+#define L(TPR, VPT)                                                                            \
+  if (rag) k_softmax_bwd_reg<T, TPR, VPT, false, false, true><<<blocks, kBlock, 0, s>>>(SMARGS); \
+  else if (nt) k_softmax_bwd_reg<T, TPR, VPT, false, true, false><<<blocks, kBlock, 0, s>>>(SMARGS); \
+  else k_softmax_bwd_reg<T, TPR, VPT, false, false, false><<<blocks, kBlock, 0, s>>>(SMARGS)
       TG_REG_DISPATCH(L)
 #undef L
     }
@@ -278,7 +356,7 @@ int softmax_bwd_t(const void* y, const void* dy, void* dx, int64_t rows, int64_t
 // Forward (_nn.py:900-917): mean, population variance over the row,
 // xhat = (x-mean)/sqrt(var+eps), y = gamma*xhat + beta.  Saves mean and
 // rstd = 1/sqrt(var+eps) per row (fp32).
-template <typename T, int TPR, int VPT>
+template <typename T, int TPR, int VPT, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_ln_fwd_reg(const T* __restrict__ x,
                                                        const float* __restrict__ gamma,
                                                        const float* __restrict__ beta,
@@ -291,7 +369,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_reg(const T* __restrict__ x,
   const int t = threadIdx.x % TPR;
   const int64_t row = (int64_t)blockIdx.x * G + threadIdx.x / TPR;
   const bool live = row < rows;
-  const int nv = cols / V;
+  const int nv = (cols + V - 1) / V;
   const int64_t off = (live ? row : 0) * (int64_t)cols;
   float xv[VPT][V];
   float s[1] = {0.f};
@@ -299,7 +377,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_reg(const T* __restrict__ x,
   for (int k = 0; k < VPT; ++k) {
     const int vi = t + k * TPR;
     if (live && vi < nv) {
-      tg_vec16<T> a = tg_load16(x + off + vi * V);
+      tg_vec16<T> a = row_ld<T, RAG, false>(x + off, vi, cols, 0.f);
 #pragma unroll
       for (int j = 0; j < V; ++j) {
         xv[k][j] = tg_to_float(a.v[j]);
@@ -319,7 +397,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_reg(const T* __restrict__ x,
     if (live && vi < nv) {
 #pragma unroll
       for (int j = 0; j < V; ++j) {
-        const float d = xv[k][j] - mu;
+        const float d = !RAG || j >= row_dup<T, RAG>(vi, cols) ? xv[k][j] - mu : 0.f;
         q[0] += d * d;
       }
     }
@@ -336,12 +414,13 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_reg(const T* __restrict__ x,
     const int vi = t + k * TPR;
     if (vi < nv) {
       tg_vec16<T> o;
+      const int c0 = row_c0<T, RAG>(vi, cols);
 #pragma unroll
       for (int j = 0; j < V; ++j) {
-        const int c = vi * V + j;
+        const int c = c0 + j;
         o.v[j] = tg_from_float<T>(gamma[c] * ((xv[k][j] - mu) * rs) + beta[c]);
       }
-      tg_store16(y + off + vi * V, o);
+      row_st<T, RAG, false>(y + off, vi, cols, o);
     }
   }
 }
@@ -383,7 +462,7 @@ __global__ __launch_bounds__(kBlock) void k_ln_fwd_loop(const T* __restrict__ x,
 // is dx itself (accumulate in place) or another buffer (a gradient shared with another
 // node, summed into this node's own buffer without copying it first); each element of
 // dxin is read by the thread that writes that element of dx, before the write.
-template <typename T, int TPR, int VPT, bool ACC, bool NT>
+template <typename T, int TPR, int VPT, bool ACC, bool NT, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_ln_bwd_reg(
     const T* __restrict__ x, const float* __restrict__ mean, const float* __restrict__ rstd,
     const float* __restrict__ gamma, const T* __restrict__ dy, T* dx, const T* dxin,
@@ -393,14 +472,14 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_reg(
   __shared__ float red[8];
   const int t = threadIdx.x % TPR;
   const int grp = threadIdx.x / TPR;
-  const int nv = cols / V;
+  const int nv = (cols + V - 1) / V;
   float gam[VPT][V], pg[VPT][V], pb[VPT][V];
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int vi = t + k * TPR;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      gam[k][j] = (vi < nv) ? gamma[vi * V + j] : 0.f;
+      gam[k][j] = (vi < nv) ? gamma[row_c0<T, RAG>(vi, cols) + j] : 0.f;
       pg[k][j] = 0.f;
       pb[k][j] = 0.f;
     }
@@ -429,9 +508,9 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_reg(
       for (int k = 0; k < VPT; ++k) {
         const int vi = t + k * TPR;
         if (vi < nv) {
-          b.x[k] = tg_ld16<NT>(x + off + vi * V);
-          b.y[k] = tg_ld16<NT>(dy + off + vi * V);
-          if (kPreO) b.o[k] = tg_ld16<NT>(dxin + off + vi * V);
+          b.x[k] = row_ld_all<T, RAG, NT>(x + off, vi, cols);
+          b.y[k] = row_ld_all<T, RAG, NT>(dy + off, vi, cols);
+          if (kPreO) b.o[k] = row_ld_all<T, RAG, NT>(dxin + off, vi, cols);
         }
       }
       b.mu = mean[row];
@@ -452,7 +531,8 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_reg(
 #pragma unroll
         for (int j = 0; j < V; ++j) {
           xh[k][j] = (tg_to_float(b.x[k].v[j]) - mu) * rs;
-          dyv[k][j] = tg_to_float(b.y[k].v[j]);
+          // (masked here: a select in fetch would wait for its load)
+          dyv[k][j] = RAG && j < row_dup<T, RAG>(vi, cols) ? 0.f : tg_to_float(b.y[k].v[j]);
           const float g = dyv[k][j] * gam[k][j];
           sums[0] += g;
           sums[1] += g * xh[k][j];
@@ -475,14 +555,14 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_reg(
         const int vi = t + k * TPR;
         if (vi < nv) {
           tg_vec16<T> o;
-          if (ACC && !kPreO) o = tg_ld16<NT>(dxin + off + vi * V);
+          if (ACC && !kPreO) o = row_ld_all<T, RAG, NT>(dxin + off, vi, cols);
 #pragma unroll
           for (int j = 0; j < V; ++j) {
             float r = rs * (dyv[k][j] * gam[k][j] - mg - xh[k][j] * mgx);
             if (ACC) r += tg_to_float(kPreO ? b.o[k].v[j] : o.v[j]);
             o.v[j] = tg_from_float<T>(r);
           }
-          tg_st16<NT>(dx + off + vi * V, o);
+          row_st<T, RAG, NT>(dx + off, vi, cols, o);
         }
       }
     }
@@ -532,10 +612,12 @@ __global__ __launch_bounds__(kBlock) void k_ln_bwd_reg(
       __syncthreads();
     }
     if (grp == 0 && vi < nv) {
-      float* pgo = part + (int64_t)blockIdx.x * cols + vi * V;
-      float* pbo = part + ((int64_t)gridDim.x + blockIdx.x) * cols + vi * V;
+      const int c0 = row_c0<T, RAG>(vi, cols);
+      float* pgo = part + (int64_t)blockIdx.x * cols + c0;
+      float* pbo = part + ((int64_t)gridDim.x + blockIdx.x) * cols + c0;
 #pragma unroll
       for (int j = 0; j < V; ++j) {
+        if (RAG && j < row_dup<T, RAG>(vi, cols)) continue;
         pgo[j] = pg[k][j];
         pbo[j] = pb[k][j];
       }
@@ -713,14 +795,17 @@ template <typename T>
 int ln_fwd_t(const void* x, const float* gamma, const float* beta, void* y, float* mean,
              float* rstd, int64_t rows, int64_t cols, float eps, hipStream_t s) {
   int tpr = 0, vpt = 0;
-  if (pick_reg_shape<T>(cols, tg_aligned16(x) && tg_aligned16(y), &tpr, &vpt)) {
+  bool rag = false;
+  if (pick_reg_shape<T>(cols, tg_aligned16(x) && tg_aligned16(y), &tpr, &vpt, &rag)) {
     const int64_t g = kBlock / tpr;
     const unsigned blocks = (unsigned)((rows + g - 1) / g);
-#define L(TPR, VPT)                                                                     \
-  k_ln_fwd_reg<T, TPR, VPT><<<blocks, kBlock, 0, s>>>((const T*)x, gamma, beta, (T*)y, mean, \
-                                                      rstd, rows, (int)cols, eps)
+#define LNARGS (const T*)x, gamma, beta, (T*)y, mean, rstd, rows, (int)cols, eps
+#define L(TPR, VPT)                                                             \
+  if (rag) k_ln_fwd_reg<T, TPR, VPT, true><<<blocks, kBlock, 0, s>>>(LNARGS);   \
+  else k_ln_fwd_reg<T, TPR, VPT, false><<<blocks, kBlock, 0, s>>>(LNARGS)
     TG_REG_DISPATCH(L)
 #undef L
+#undef LNARGS
   } else {
     k_ln_fwd_loop<T><<<(unsigned)((rows + 3) / 4), kBlock, 0, s>>>(
         (const T*)x, gamma, beta, (T*)y, mean, rstd, rows, cols, eps);
@@ -729,7 +814,7 @@ int ln_fwd_t(const void* x, const float* gamma, const float* beta, void* y, floa
 }
 
 struct LnBwdPlan {
-  bool reg;
+  bool reg, rag;
   int tpr, vpt;
   int64_t nparts;  // number of dgamma (and dbeta) partial rows in the workspace
 };
@@ -737,8 +822,15 @@ struct LnBwdPlan {
 template <typename T>
 LnBwdPlan ln_bwd_plan(int64_t rows, int64_t cols, bool aligned) {
   LnBwdPlan p{};
-  p.reg = pick_reg_shape<T>(cols, aligned, &p.tpr, &p.vpt);
+  p.reg = pick_reg_shape<T>(cols, aligned, &p.tpr, &p.vpt, &p.rag);
+  // ragged rows of 64 16-bit elements a thread do not stay in the registers: fp16
+  // [2000, 16383] 218 us by the looping kernels, 228 (294 adding to dx) here; of 32,
+  // [3000, 8191], 138 and 82
+  if (p.reg && p.rag && p.vpt * tg_vec16<T>::N > 32) p.reg = false;
   p.nparts = p.reg ? ln_bwd_blocks(rows, p.tpr) : colsum_splits(rows, cols);
+  // (ragged rows: at most 8 MB of partials, which the fixed scratch of the form without a
+  // workspace holds, as it held the looping kernels')
+  if (p.reg && p.rag && p.nparts * cols > (1 << 20)) p.nparts = (1 << 20) / cols;
   return p;
 }
 
@@ -758,19 +850,22 @@ int ln_bwd_t(const void* x, const float* mean, const float* rstd, const float* g
   if (p.reg) {
     const unsigned blocks = (unsigned)p.nparts;
     const int tpr = p.tpr, vpt = p.vpt;
+    const bool rag = p.rag;
     const bool nt = (int64_t)sizeof(T) * rows * cols >= kNtBytes;
 #define LNARGS \
   (const T*)x, mean, rstd, gamma, (const T*)dy, (T*)dx, (const T*)dxin, part, rows, (int)cols
     if (acc_dx) {
-#define L(TPR, VPT)                                                                           \
-  if (nt) k_ln_bwd_reg<T, TPR, VPT, true, true><<<blocks, kBlock, 0, s>>>(LNARGS); \
-  else k_ln_bwd_reg<T, TPR, VPT, true, false><<<blocks, kBlock, 0, s>>>(LNARGS)
+#define L(TPR, VPT)                                                                            \
+  if (rag) k_ln_bwd_reg<T, TPR, VPT, true, false, true><<<blocks, kBlock, 0, s>>>(LNARGS);     \
+  else if (nt) k_ln_bwd_reg<T, TPR, VPT, true, true, false><<<blocks, kBlock, 0, s>>>(LNARGS); \
+  else k_ln_bwd_reg<T, TPR, VPT, true, false, false><<<blocks, kBlock, 0, s>>>(LNARGS)
       TG_REG_DISPATCH(L)
 #undef L
     } else {
 #define L(TPR, VPT)                                                                            \
-  if (nt) k_ln_bwd_reg<T, TPR, VPT, false, true><<<blocks, kBlock, 0, s>>>(LNARGS); \
-  else k_ln_bwd_reg<T, TPR, VPT, false, false><<<blocks, kBlock, 0, s>>>(LNARGS)
+  if (rag) k_ln_bwd_reg<T, TPR, VPT, false, false, true><<<blocks, kBlock, 0, s>>>(LNARGS);    \
+  else if (nt) k_ln_bwd_reg<T, TPR, VPT, false, true, false><<<blocks, kBlock, 0, s>>>(LNARGS); \
+  else k_ln_bwd_reg<T, TPR, VPT, false, false, false><<<blocks, kBlock, 0, s>>>(LNARGS)
       TG_REG_DISPATCH(L)
 #undef L
     }
