@@ -285,8 +285,10 @@ __global__ __launch_bounds__(kThreads) void k_axpby8(const TX* __restrict__ x, c
 
 // z = x for one dtype (alpha 1, beta 0): the seed of a backward and every gradient that is
 // copied as it is.  HBM-bound; one 16-byte vector per thread, each instruction contiguous
-// over the wavefront, non-temporal past 128 MB (fp32, k_axpby8's two vectors per thread in a
-// grid-stride loop and here: 17 MB 7.5 and 6.2 us, 268 MB 103 and 83, 1 GB 427 and 330).
+// over the wavefront, non-temporal past 128 MB (k_axpby8's 8 elements per thread in a
+// grid-stride loop and here: fp32 17 MB 7.5 and 6.2 us, 268 MB 103 and 83, 1 GB 427 and 330;
+// fp16 268 MB 100 and 83).  16-bit types below that size stay there: one vector per thread
+// already, and 32 MB is 12.8 us there and 13.2 here.
 template <bool NT>
 __global__ __launch_bounds__(kActThreads) void k_copy16(const uint4* __restrict__ x,
                                                         uint4* __restrict__ z, int64_t n16,
@@ -318,7 +320,8 @@ int launch_axpby(const void* x, const void* y, void* z, float a, float b, int64_
                  hipStream_t s) {
   // (a grid's work-items are counted in 32 bits: 2^32 vectors of 16 bytes)
   if (std::is_same<TX, TY>::value && a == 1.f && b == 0.f && x != z && tg_aligned16(x) &&
-      tg_aligned16(z) && n < (int64_t{1} << 33))
+      tg_aligned16(z) && n < (int64_t{1} << 33) &&
+      (sizeof(TX) == 4 || n * (int64_t)sizeof(TX) >= kNtBytes))
     return launch_copy(x, z, n * (int64_t)sizeof(TX), s);
   if (tg_aligned16(x) && tg_aligned16(y) && tg_aligned16(z)) {
     const int64_t n8 = n / 8;
