@@ -110,8 +110,12 @@ struct RsOp {
     for (int i = 0; i < NCH; ++i) p[i] += step;
   }
   // Split the held chunks into the three planes at lds; tiny: least of the 16-bit keys
-  // 2|h| - 1 seen (zero wraps to the top), for the check of small operands.
+  // 2|h| - 1 seen (zero wraps to the top), for the check of small operands.  ALT: every
+  // second row (m or n) with its sign turned round.
+  template <bool ALT>
   __device__ __forceinline__ void store(char* lds, u16x2& tiny) const {
+    static_assert(!KC || NT / CH % 2 == 0, "a thread's rows must share their parity");
+    const unsigned turn = (ALT && KC) ? (threadIdx.x / CH & 1u) << 31 : 0u;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int u = threadIdx.x + i * NT, r = u / CH, c = u % CH;
@@ -122,7 +126,13 @@ struct RsOp {
       unsigned* ql = reinterpret_cast<unsigned*>(&q[2]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x0 = v[i][2 * e], x1 = v[i][2 * e + 1];
+        float x0 = v[i][2 * e], x1 = v[i][2 * e + 1];
+        if (ALT && KC) {
+          x0 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x0) ^ turn);
+          x1 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x1) ^ turn);
+        } else if (ALT) {
+          x1 = -x1;
+        }
         const unsigned h = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x0, (__bf16)x1});
         const float r0 = x0 - __builtin_bit_cast(float, h << 16);
         const float r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
@@ -219,6 +229,11 @@ __device__ __forceinline__ void rs_fp32_tiles(const float* __restrict__ A, int64
   }
 }
 
+// The bf16 matrix instructions round a sum down by ~2^-24 on average.  One entry does not
+// show it, but a sum over many rows of C (a bias gradient behind this product) would add it
+// up: 9.7e-6 of its size over 13632 rows, where the fp32 instructions gave 1.3e-6.  Odd rows
+// of A are therefore multiplied with their signs turned round, and their entries of C turned
+// back, so that neighbouring rows err to opposite sides.
 // STAG: the upper half of the waves multiplies before it stores.  TWO: sums of 512 k are
 // added up in a second accumulator, so that the smaller tiles' sums err no more than the
 // K splits that served their sizes before (64x64 and 128x128; 256x128 has no registers left
@@ -310,16 +325,16 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     __syncthreads();
     if (late) mul(as, bs);
     if (k0 + BK < K) {
-      oa.store(an, tiny);
-      ob.store(bn, tiny);
+      oa.template store<true>(an, tiny);
+      ob.template store<false>(bn, tiny);
       if (k0 + 2 * BK < K) load(k0 + 2 * BK);
     }
     if (!late) mul(as, bs);
   };
   if (K > 0) {
     load(0);
-    oa.store(a0, tiny);
-    ob.store(b0, tiny);
+    oa.template store<true>(a0, tiny);
+    ob.template store<false>(b0, tiny);
     if (BK < K) load(BK);
     for (int64_t k0 = 0; k0 < K; k0 += 2 * BK) {
       step(k0, a0, b0, a1, b1);
@@ -347,6 +362,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
     }
+    // the odd rows of A went in with their signs turned round
+#pragma unroll
+    for (int i = 0; i < SM; ++i)
+#pragma unroll
+      for (int j = 0; j < SN; ++j)
+#pragma unroll
+        for (int r = 1; r < 16; r += 2) acc[i][j][r] = -acc[i][j][r];
     // operands the split cannot hold: redo the tile on the fp32 matrix cores
     bool bad = tiny[0] < 0x18ff || tiny[1] < 0x18ff;  // a nonzero |x| below 2^-102
 #pragma unroll

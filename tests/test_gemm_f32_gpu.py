@@ -115,3 +115,19 @@ def test_matmul_f32_values_outside_the_split(cuda, M, N, K, kind):
     err = (got - want).abs()
     ok = err[fin] <= (6 * (K // 16 + 1) + K) * 2.0 ** -23 * mag[fin] + K * 1.5e-45
     assert bool(ok.all()), f"{kind}: {(err[fin] / mag[fin]).max().item():.2e}"
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_column_sums_are_not_biased(cuda, ta, tb):
+    """Sums of n = 131072 rows of a product of unit normals (entries of size sqrt(K)): an entry
+    takes K / 16 sums, each off by up to 2^-24 of its size.  Errors to either side add up to
+    sqrt(n) of them (held to 4 sigma); errors to one side would to n of about half of them, 45
+    times the bound."""
+    M, N, K = 131072, 256, 368
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randn(*((K, M) if ta else (M, K)), device="cuda", generator=g)
+    b = torch.randn(*((N, K) if tb else (K, N)), device="cuda", generator=g)
+    c = L().matmul2d(a, b, trans_a=bool(ta), trans_b=bool(tb))
+    ref = a.double().sum(1 if ta else 0) @ (b.double().T if tb else b.double())
+    err = float((c.double().sum(0) - ref).abs().max())
+    assert err <= 4 * M ** 0.5 * (K / 16) * 2.0 ** -24 * K ** 0.5, err
