@@ -1,6 +1,7 @@
 // FlashAttention forward and backward for gfx950, reference: flash_attention
-// (_core.py:1686-1870).  Tuned kernels for fp16 / bf16 with head dim 64 or 128; generic
-// kernels (fp32 matrix cores, any head dim up to 256) for fp32 and other head dims.
+// (_core.py:1686-1870).  Tuned kernels for fp16 / bf16 with head dim 64 or 128;
+// split-operand kernels (16-bit matrix cores, fp32 accuracy) for fp32 and for the other
+// head dims up to 128; generic kernels (fp32 matrix cores) for head dims 129 to 256.
 //
 // Tensors are contiguous [B, H, S, D]; lse is [B, H, Sq] fp32 (natural log).
 // causal masks key > query (top-left aligned, as the reference's col > row).
@@ -1046,8 +1047,9 @@ int bwd_t(const void* q, const void* k, const void* v, const void* o, const void
   return tg_check_launch("tg_flash_attn_bwd");
 }
 
-// ============================================================ generic head dims / fp32
-// Any head dim D <= 256 and fp32 as well as fp16/bf16 inputs: the same algorithm as
+// ============================================================ generic kernels
+// Head dims past 128, and workgroups whose fp32 values the split-operand kernels below
+// cannot hold; fp32 as well as fp16/bf16 inputs: the same algorithm as
 // the kernels above on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), so fp32
 // attention keeps fp32 precision.  D is padded with zeros to DP, a multiple of 32,
 // inside the kernels; loads and stores are element-wise (no alignment requirement).
@@ -1431,8 +1433,8 @@ int bwd_gen_t(const void* q, const void* k, const void* v, const void* o, const 
 }
 
 // ================================================= split operands: fp32, other head dims
-// FlashAttention for fp32 data and for fp16 / bf16 head dims other than 64 and 128 (up to
-// 128; larger ones and unaligned fp32 values take the generic kernels above), on the
+// FlashAttention for fp32 data and for what the tuned fp16 / bf16 kernels leave, at head
+// dims up to 128 (larger ones take the generic kernels above) and any alignment, on the
 // 16-bit matrix cores with fp32 accuracy of everything the generic kernels keep in fp32:
 // an fp32 operand is split exactly into three bf16 terms h + m + l (each the bf16 rounding
 // of what is left), and so are P and dS; of the nine term products the six of weight >=
@@ -2224,7 +2226,8 @@ int fa_group_bwd(int64_t BH, int causal, int64_t S, int64_t D) {
 }
 
 // The tuned fp16/bf16 kernels serve head dims 64 and 128 with 16-byte aligned operands;
-// everything else runs on the generic fp32-MFMA kernels.
+// everything else runs on the split-operand kernels (head dims up to 128) or the generic
+// fp32-MFMA ones.
 bool fa_fast(int dtype, int64_t D, std::initializer_list<const void*> ptrs) {
   if (dtype == TG_F32 || (D != 64 && D != 128)) return false;
   for (const void* p : ptrs)
