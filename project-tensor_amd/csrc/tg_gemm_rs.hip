@@ -12,10 +12,14 @@
 // fp32 ones (v_mfma_f32_32x32x2_f32) of twice the issue time each, and the accumulator is
 // rounded once per 16 k instead of once per 2, so the sums are as exact as the fp32
 // matrix cores' (measured against float64).
-// Values the split cannot hold are caught and redone: a block that sees a nonzero operand
-// below 2^-102 (its low term could leave bf16's normal range) or that ends with a
-// non-finite accumulator (an infinite or NaN operand, or an overflow that the split could
-// have caused by itself) computes its tile again on the fp32 matrix cores.
+// Both operands are multiplied by 2^24 before they are split, and the sums by 2^-48 at the
+// end: every fp32 number is a multiple of 2^-149, so every term of its split is one of
+// 2^-125, a normal bf16 number, and the split is exact for subnormal operands too.  What
+// that leaves to catch is overflow: a block that ends with a non-finite accumulator (an
+// infinite or NaN operand, one of 2^104 or more, or a sum of 2^80 or more) computes its tile
+// again on the fp32 matrix cores, operands unstaged: 8192x4096x1024 with an infinity in every
+// row block 1430 us, 360 without.  (Unscaled, an operand below 2^-102 had to be redone the
+// same way, and softmax outputs 71 below their row's maximum are such operands.)
 //
 // Block: WGM x WGN waves, each SM*32 x SN*32 of C.  k-tiles of 32 are loaded into
 // registers (16-byte loads at element alignment), split, and written to LDS as three
@@ -35,10 +39,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 #define TG_LDS_RS __attribute__((address_space(3)))
 
 constexpr int BK = 32;
+constexpr int kScaleExp = 24;  // operands are scaled by 2^kScaleExp
+constexpr float kScale = 1 << kScaleExp;
 
 // Four floats at 4-byte alignment (a global load takes any dword address).
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
@@ -109,13 +114,13 @@ struct RsOp {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) p[i] += step;
   }
-  // Split the held chunks into the three planes at lds; tiny: least of the 16-bit keys
-  // 2|h| - 1 seen (zero wraps to the top), for the check of small operands.  ALT: every
-  // second row (m or n) with its sign turned round.
+  // Split the held chunks, times kScale, into the three planes at lds.  ALT: every second
+  // row (m or n) with its sign turned round.
   template <bool ALT>
-  __device__ __forceinline__ void store(char* lds, u16x2& tiny) const {
+  __device__ __forceinline__ void store(char* lds) const {
     static_assert(!KC || NT / CH % 2 == 0, "a thread's rows must share their parity");
-    const unsigned turn = (ALT && KC) ? (threadIdx.x / CH & 1u) << 31 : 0u;
+    const float by0 = ALT && KC && (threadIdx.x / CH & 1) ? -kScale : kScale;
+    const float by1 = ALT && !KC ? -kScale : by0;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int u = threadIdx.x + i * NT, r = u / CH, c = u % CH;
@@ -126,13 +131,7 @@ struct RsOp {
       unsigned* ql = reinterpret_cast<unsigned*>(&q[2]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float x0 = v[i][2 * e], x1 = v[i][2 * e + 1];
-        if (ALT && KC) {
-          x0 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x0) ^ turn);
-          x1 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x1) ^ turn);
-        } else if (ALT) {
-          x1 = -x1;
-        }
+        const float x0 = v[i][2 * e] * by0, x1 = v[i][2 * e + 1] * by1;
         const unsigned h = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x0, (__bf16)x1});
         const float r0 = x0 - __builtin_bit_cast(float, h << 16);
         const float r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
@@ -142,8 +141,6 @@ struct RsOp {
         qh[e] = h;
         qm[e] = m;
         ql[e] = __builtin_bit_cast(unsigned, bf16x2{(__bf16)s0, (__bf16)s1});
-        const u16x2 k = __builtin_bit_cast(u16x2, h);
-        tiny = __builtin_elementwise_min(tiny, (u16x2)((k << 1) - (u16x2)1));
       }
 #pragma unroll
       for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint4*>(lds + pl * PLANE + off) = q[pl];
@@ -290,7 +287,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
   oa.init(A, lda, m0, M);
   ob.init(B, ldb, n0, N);
   const bool ea = TA && m0 + TBM > M, eb = !TB && n0 + TBN > N;
-  u16x2 tiny = {0xffff, 0xffff};
   auto load = [&](int64_t k0) {
     const bool ek = k0 + BK > K;
     oa.load(ea || ek, K - k0);
@@ -325,16 +321,16 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     __syncthreads();
     if (late) mul(as, bs);
     if (k0 + BK < K) {
-      oa.template store<true>(an, tiny);
-      ob.template store<false>(bn, tiny);
+      oa.template store<true>(an);
+      ob.template store<false>(bn);
       if (k0 + 2 * BK < K) load(k0 + 2 * BK);
     }
     if (!late) mul(as, bs);
   };
   if (K > 0) {
     load(0);
-    oa.template store<true>(a0, tiny);
-    ob.template store<false>(b0, tiny);
+    oa.template store<true>(a0);
+    ob.template store<false>(b0);
     if (BK < K) load(BK);
     for (int64_t k0 = 0; k0 < K; k0 += 2 * BK) {
       step(k0, a0, b0, a1, b1);
@@ -362,23 +358,27 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
     }
-    // the odd rows of A went in with their signs turned round
-#pragma unroll
-    for (int i = 0; i < SM; ++i)
-#pragma unroll
-      for (int j = 0; j < SN; ++j)
-#pragma unroll
-        for (int r = 1; r < 16; r += 2) acc[i][j][r] = -acc[i][j][r];
     // operands the split cannot hold: redo the tile on the fp32 matrix cores
-    bool bad = tiny[0] < 0x18ff || tiny[1] < 0x18ff;  // a nonzero |x| below 2^-102
+    bool bad = false;
 #pragma unroll
     for (int i = 0; i < SM; ++i)
 #pragma unroll
       for (int j = 0; j < SN; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
-    if (__syncthreads_or(bad))
+    if (__syncthreads_or(bad)) {
       rs_fp32_tiles<TA, TB, SM, SN>(A, lda, B, ldb, M, N, K, m0 + wm, n0 + wn, acc);
+    } else {
+      // both scales off again (one rounding where the entry is subnormal), and the odd rows
+      // of A went in with their signs turned round
+#pragma unroll
+      for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int j = 0; j < SN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[i][j][r] = ldexpf(r & 1 ? -acc[i][j][r] : acc[i][j][r], -2 * kScaleExp);
+    }
   }
 #pragma unroll
   for (int i = 0; i < SM; ++i)

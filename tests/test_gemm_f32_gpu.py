@@ -131,3 +131,32 @@ def test_column_sums_are_not_biased(cuda, ta, tb):
     ref = a.double().sum(1 if ta else 0) @ (b.double().T if tb else b.double())
     err = float((c.double().sum(0) - ref).abs().max())
     assert err <= 4 * M ** 0.5 * (K / 16) * 2.0 ** -24 * K ** 0.5, err
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(40, 50, 100), (70, 2050, 300), (700, 800, 500), (1100, 2060, 129)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_matmul_f32_subnormal_operands(cuda, M, N, K, ta, tb, mixed):
+    """Operands down to the least subnormal number, beside ordinary ones, count in full: the
+    bound is that of ordinary operands, plus one rounding of a subnormal entry a product."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a = _mk(g, M, K)
+    if mixed:
+        e = torch.randint(-149, 1, (M, K), generator=g, device="cuda").double()
+        a = (a.double() * 2.0 ** e).float()
+    a[1] = 4e-41      # rounds to zero in bf16
+    a[2] = 1e-42
+    a[3] = 2.0 ** -149
+    b = _mk(g, K, N)
+    b[:, 1] *= 1e20
+    if mixed:
+        b[:, 2] = -3e-44
+        b[:, 3] *= 1e-18
+    c = L().matmul2d(a.t().contiguous() if ta else a, b.t().contiguous() if tb else b,
+                     trans_a=bool(ta), trans_b=bool(tb))
+    want = a.double() @ b.double()
+    mag = a.double().abs() @ b.double().abs()
+    n = 6 * (K // 16 + 1) + 40
+    err = (c.double() - want).abs()
+    assert bool((err <= (n * 2.0 ** -23 + 2.0 ** -22) * mag + K * 1.5e-45).all())
+    assert bool((c[1:4, 1] != 0).all())
