@@ -7,11 +7,10 @@
 // round-to-nearest each.  24 significand bits fall into 8 + 8 + 8, so the split is exact.
 // Of the nine products of two split operands the six with weight >= 2^-16 are kept,
 //   hh + hm + mh + mm + hl + lh,
-// accumulated in fp32; the three that are dropped are together below 2^-23.5 of the
-// product and of either sign.  Six bf16 MFMAs (v_mfma_f32_32x32x16_bf16) replace eight
-// fp32 ones (v_mfma_f32_32x32x2_f32) of twice the issue time each, and the accumulator is
-// rounded once per 16 k instead of once per 2, so the sums are as exact as the fp32
-// matrix cores' (measured against float64).
+// accumulated in fp32; the three that are dropped (a term is at most 2^-8 of the one before
+// it) are together at most 2^-24 of the product, and of either sign.  Six bf16 MFMAs
+// (v_mfma_f32_32x32x16_bf16) replace eight fp32 ones (v_mfma_f32_32x32x2_f32) of twice the
+// issue time each.
 // Both operands are multiplied by 2^24 before they are split, and the sums by 2^-48 at the
 // end: every fp32 number is a multiple of 2^-149, so every term of its split is one of
 // 2^-125, a normal bf16 number, and the split is exact for subnormal operands too.  What
@@ -44,6 +43,7 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 constexpr int BK = 32;
 constexpr int kScaleExp = 24;  // operands are scaled by 2^kScaleExp
 constexpr float kScale = 1 << kScaleExp;
+constexpr int kTurn = 2 * BK;  // k extent of one partial sum
 
 // Four floats at 4-byte alignment (a global load takes any dword address).
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
@@ -114,13 +114,8 @@ struct RsOp {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) p[i] += step;
   }
-  // Split the held chunks, times kScale, into the three planes at lds.  ALT: every second
-  // row (m or n) with its sign turned round.
-  template <bool ALT>
-  __device__ __forceinline__ void store(char* lds) const {
-    static_assert(!KC || NT / CH % 2 == 0, "a thread's rows must share their parity");
-    const float by0 = ALT && KC && (threadIdx.x / CH & 1) ? -kScale : kScale;
-    const float by1 = ALT && !KC ? -kScale : by0;
+  // Split the held chunks, times `by` (+-kScale), into the three planes at lds.
+  __device__ __forceinline__ void store(char* lds, float by) const {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int u = threadIdx.x + i * NT, r = u / CH, c = u % CH;
@@ -131,7 +126,7 @@ struct RsOp {
       unsigned* ql = reinterpret_cast<unsigned*>(&q[2]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x0 = v[i][2 * e] * by0, x1 = v[i][2 * e + 1] * by1;
+        const float x0 = v[i][2 * e] * by, x1 = v[i][2 * e + 1] * by;
         const unsigned h = __builtin_bit_cast(unsigned, bf16x2{(__bf16)x0, (__bf16)x1});
         const float r0 = x0 - __builtin_bit_cast(float, h << 16);
         const float r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
@@ -226,16 +221,20 @@ __device__ __forceinline__ void rs_fp32_tiles(const float* __restrict__ A, int64
   }
 }
 
-// The bf16 matrix instructions round a sum down by ~2^-24 on average.  One entry does not
-// show it, but a sum over many rows of C (a bias gradient behind this product) would add it
-// up: 9.7e-6 of its size over 13632 rows, where the fp32 instructions gave 1.3e-6.  Odd rows
-// of A are therefore multiplied with their signs turned round, and their entries of C turned
-// back, so that neighbouring rows err to opposite sides.
-// STAG: the upper half of the waves multiplies before it stores.  TWO: sums of 512 k are
-// added up in a second accumulator, so that the smaller tiles' sums err no more than the
-// K splits that served their sizes before (64x64 and 128x128; 256x128 has no registers left
-// for it).
-template <bool TA, bool TB, int WGM, int WGN, int SM, int SN, bool STAG, bool TWO>
+// How the sums are kept as exact as the fp32 matrix cores': an MFMA rounds its result once,
+// and drops what of its addends lies below, which takes sums down by a little more than it
+// takes them up.  Six MFMAs per 16 k into one accumulator leave an entry up to 1.2 times as
+// far off as v_mfma_f32_32x32x2 does (non-negative A: 4096x4096x2048 6.7e-7 of the 2-norm,
+// 5.8e-7 there), and column sums of C, a bias gradient behind it, 10 times (pairs of rows
+// with opposite signs take that back for zero-mean entries only).  So every 64 k are summed
+// from zero and added to a second accumulator by the vector unit, every second time with A's
+// signs, and the partial sum's, turned round, so that neighbouring partial sums err to
+// opposite sides: entries 1.7e-7 there, column sums at or below those of the fp32
+// instructions for operands of either or of one sign.  4096x4096x2048 takes 380 us, 366 with
+// one accumulator; partial sums of 128 k take 368, but leave column sums of offset operands
+// 2 to 4 times as far off as the fp32 instructions at K = 512.
+// STAG: the upper half of the waves multiplies before it stores.
+template <bool TA, bool TB, int WGM, int WGN, int SM, int SN, bool STAG>
 __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha, const float* __restrict__ A,
     int64_t lda, int64_t sa, const float* __restrict__ B, int64_t ldb, int64_t sb, float beta,
@@ -275,13 +274,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     for (int j = 0; j < SN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  f32x16 sum[TWO ? SM : 1][TWO ? SN : 1];
-  if constexpr (TWO) {
+  f32x16 sum[SM][SN];
 #pragma unroll
-    for (int i = 0; i < SM; ++i)
+  for (int i = 0; i < SM; ++i)
 #pragma unroll
-      for (int j = 0; j < SN; ++j) sum[i][j] = acc[i][j];
-  }
+    for (int j = 0; j < SN; ++j) sum[i][j] = acc[i][j];
   OA oa;
   OB ob;
   oa.init(A, lda, m0, M);
@@ -292,7 +289,18 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     oa.load(ea || ek, K - k0);
     ob.load(eb || ek, K - k0);
   };
-  auto mul = [&](const char* as, const char* bs) {
+  auto mul = [&](int64_t k0, const char* as, const char* bs) {
+    if (k0 % kTurn == 0 && k0 > 0) {
+      // the partial sum is whole: add it (in whole vectors: element by element the compiler
+      // keeps the arrays in scratch memory)
+#pragma unroll
+      for (int i = 0; i < SM; ++i)
+#pragma unroll
+        for (int j = 0; j < SN; ++j) {
+          sum[i][j] = acc[i][j] - sum[i][j];
+          acc[i][j] = f32x16{};
+        }
+    }
 #pragma unroll
     for (int ks = 0; ks < BK / 16; ++ks) {
       bf16x8 af[SM][3], bf[SN][3];
@@ -317,47 +325,31 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
   // tile t is multiplied from one buffer while tile t + 1 (in registers) is split into
   // the other and tile t + 2 is loaded
   const bool late = STAG && wave >= WGM * WGN / 2;
+  auto turned = [&](int64_t k0) { return k0 / kTurn % 2 != 0; };
   auto step = [&](int64_t k0, const char* as, const char* bs, char* an, char* bn) {
     __syncthreads();
-    if (late) mul(as, bs);
+    if (late) mul(k0, as, bs);
     if (k0 + BK < K) {
-      oa.template store<true>(an);
-      ob.template store<false>(bn);
+      oa.store(an, turned(k0 + BK) ? -kScale : kScale);
+      ob.store(bn, kScale);
       if (k0 + 2 * BK < K) load(k0 + 2 * BK);
     }
-    if (!late) mul(as, bs);
+    if (!late) mul(k0, as, bs);
   };
   if (K > 0) {
     load(0);
-    oa.template store<true>(a0);
-    ob.template store<false>(b0);
+    oa.store(a0, kScale);
+    ob.store(b0, kScale);
     if (BK < K) load(BK);
     for (int64_t k0 = 0; k0 < K; k0 += 2 * BK) {
       step(k0, a0, b0, a1, b1);
       if (k0 + BK >= K) break;
       step(k0 + BK, a1, b1, a0, b0);
-      if constexpr (TWO) {
-        if ((k0 & (512 - 1)) == 512 - 2 * BK) {
-#pragma unroll
-          for (int i = 0; i < SM; ++i)
-#pragma unroll
-            for (int j = 0; j < SN; ++j)
-#pragma unroll
-              for (int r = 0; r < 16; ++r) {
-                sum[i][j][r] += acc[i][j][r];
-                acc[i][j][r] = 0.f;
-              }
-        }
-      }
     }
-    if constexpr (TWO) {
 #pragma unroll
-      for (int i = 0; i < SM; ++i)
+    for (int i = 0; i < SM; ++i)
 #pragma unroll
-        for (int j = 0; j < SN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
-    }
+      for (int j = 0; j < SN; ++j) acc[i][j] -= sum[i][j];
     // operands the split cannot hold: redo the tile on the fp32 matrix cores
     bool bad = false;
 #pragma unroll
@@ -369,15 +361,14 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
     if (__syncthreads_or(bad)) {
       rs_fp32_tiles<TA, TB, SM, SN>(A, lda, B, ldb, M, N, K, m0 + wm, n0 + wn, acc);
     } else {
-      // both scales off again (one rounding where the entry is subnormal), and the odd rows
-      // of A went in with their signs turned round
+      // both scales off again (one rounding where the entry is subnormal)
 #pragma unroll
       for (int i = 0; i < SM; ++i)
 #pragma unroll
         for (int j = 0; j < SN; ++j)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            acc[i][j][r] = ldexpf(r & 1 ? -acc[i][j][r] : acc[i][j][r], -2 * kScaleExp);
+            acc[i][j][r] = ldexpf(turned(K - 1) ? -acc[i][j][r] : acc[i][j][r], -2 * kScaleExp);
     }
   }
 #pragma unroll
@@ -461,7 +452,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_gemm_f32_small(
   }
 }
 
-template <int WGM, int WGN, int SM, int SN, bool STAG, bool TWO>
+template <int WGM, int WGN, int SM, int SN, bool STAG>
 int rs_launch(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha,
               const float* A, int64_t lda, int64_t sa, const float* B, int64_t ldb, int64_t sb,
               float beta, float* C, int64_t ldc, int64_t sc, int64_t batch, const float* bias,
@@ -474,7 +465,7 @@ int rs_launch(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t ktot, flo
   }
   const dim3 grid((unsigned)(gx * gy), 1, (unsigned)batch);
 #define TG_RS(TA_, TB_)                                                                      \
-  k_gemm_rs<TA_, TB_, WGM, WGN, SM, SN, STAG, TWO><<<grid, 64 * WGM * WGN, 0, s>>>(                      \
+  k_gemm_rs<TA_, TB_, WGM, WGN, SM, SN, STAG><<<grid, 64 * WGM * WGN, 0, s>>>(               \
       M, N, K, ktot, alpha, A, lda, sa, B, ldb, sb, beta, C, ldc, sc, bias, (int)gx,          \
       (int)(gx * gy))
   if (!ta && !tb) TG_RS(false, false);
@@ -542,9 +533,9 @@ int tg_gemm_rs(const TgRsPlan& p, int ta, int tb, int64_t M, int64_t N, int64_t 
   rs_launch<__VA_ARGS__>(ta, tb, M, N, kc, ktot, alpha, A, lda, sa, B, ldb, sb, beta, C, ldc, \
                          sc, batch, bias, s)
   switch (p.shape) {
-    case RS_256x128: return TG_RSL(4, 2, 2, 2, true, false);
-    case RS_128x128: return TG_RSL(4, 2, 1, 2, true, true);
-    case RS_64x64: return TG_RSL(2, 2, 1, 1, false, true);
+    case RS_256x128: return TG_RSL(4, 2, 2, 2, true);
+    case RS_128x128: return TG_RSL(4, 2, 1, 2, true);
+    case RS_64x64: return TG_RSL(2, 2, 1, 1, false);
     default: break;
   }
 #undef TG_RSL

@@ -160,3 +160,54 @@ def test_matmul_f32_subnormal_operands(cuda, M, N, K, ta, tb, mixed):
     err = (c.double() - want).abs()
     assert bool((err <= (n * 2.0 ** -23 + 2.0 ** -22) * mag + K * 1.5e-45).all())
     assert bool((c[1:4, 1] != 0).all())
+
+
+def _operands(kind, g, M, N, K):
+    a, b = _mk(g, M, K), _mk(g, K, N)
+    return {"normal": (a, b), "relu": (a.relu(), b), "positive": (a.abs(), b.abs()),
+            "offset": (a + 3, b + 3)}[kind]
+
+
+@pytest.mark.parametrize("kind", ["normal", "relu", "positive", "offset"])
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 2048), (1024, 1024, 1024), (700, 800, 4096)])
+@pytest.mark.parametrize("ta", [False, True])
+def test_entries_are_no_further_off_than_a_partial_sum_scheme(cuda, M, N, K, kind, ta):
+    """Partial sums of 64 k, added in fp32: the additions round by 2^-24 / sqrt(3) of a sum
+    that grows to its size over K / 64 of them (1.4e-7 in the 2-norm at K = 2048), the
+    partial sums themselves are off by about 1e-7 of theirs; held to twice that.  One
+    accumulator over K would be off by 6 to 7e-7 at K = 2048."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = _operands(kind, g, M, N, K)
+    c = L().matmul2d(a.t().contiguous() if ta else a, b, trans_a=ta)
+    want = a.double() @ b.double()
+    e = float((c.double() - want).norm() / want.norm())
+    lim = 2 * ((K / 128) ** 0.5 * 2.0 ** -24 / 3 ** 0.5 + 1e-7)
+    assert e < lim, f"{e:.2e} {lim:.2e}"
+
+
+@pytest.mark.parametrize("kind", ["normal", "relu", "positive", "offset"])
+@pytest.mark.parametrize("M,N,K", [(8192, 1024, 368), (13632, 368, 1472), (2048, 2304, 512)])
+def test_column_sums_of_one_sign(cuda, M, N, K, kind):
+    """Entries that err to either side at random (up to 2.5e-7 of their size) leave 1/sqrt(M)
+    of that in a column sum relative to M entries; allowed are 4 times it and 8e-9, an eighth
+    of fp32's own rounding of the sum.  One accumulator leaves 3 to 6e-8."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = _operands(kind, g, M, N, K)
+    c = L().matmul2d(a, b)
+    want = a.double() @ b.double()
+    d = (c.double() - want).sum(0)
+    e = float(d.norm() / (want.norm(dim=0) * M ** 0.5).norm())
+    assert e < 4 * 2.5e-7 / M ** 0.5 + 8e-9, f"{e:.2e}"
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 800, 500), (2100, 4200, 300), (4096, 2048, 1024)])
+@pytest.mark.parametrize("ta", [False, True])
+def test_equal_rows_give_equal_rows(cuda, M, N, K, ta):
+    """A row's result does not depend on where in the operand the row stands."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    a, b = _mk(g, M, K), _mk(g, K, N)
+    for r in (1, 2, 77, M // 2, M - 1):
+        a[r] = a[0]
+    c = L().matmul2d(a.t().contiguous() if ta else a, b, trans_a=ta)
+    for r in (1, 2, 77, M // 2, M - 1):
+        assert torch.equal(c[r], c[0])
