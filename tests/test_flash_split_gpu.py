@@ -110,3 +110,24 @@ def test_split_attention_fp32_extremes(cuda, D, kind):
     if kind in ("tiny", "negative_scale"):
         for t, w, n in zip(grads, want[1:], ("dq", "dk", "dv")):
             _close(t, w, torch.float32, n, 10.0)
+
+
+@pytest.mark.parametrize("D", [24, 64, 128])
+@pytest.mark.parametrize("S,causal", [(150, False), (257, True)])
+def test_split_attention_fp32_subnormal_columns(cuda, D, S, causal):
+    """Columns of subnormal operands (their bf16 rounding is zero) beside ordinary ones: each
+    result column that is formed from one keeps its value, to the rounding of subnormals (a
+    multiple of 2^-149 each, about 1e-3 of these results)."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v, do = (torch.randn(1, 2, S, D, generator=g, device="cuda") for _ in range(4))
+    for t, c in ((q, 1), (k, 2), (v, 3), (do, 4)):
+        t[..., c] *= 1e-41
+    sc = D ** -0.5
+    o, lse = L().flash_attn_fwd(q, k, v, sc, causal)
+    grads = [torch.empty_like(q) for _ in range(3)]
+    L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, causal, False)
+    want = _ref(q, k, v, do, sc, causal)
+    for t, w, c, n in zip([o] + grads, want, (3, 2, 1, 4), ("o", "dq", "dk", "dv")):
+        _close(t, w, torch.float32, n, 2.0)
+        a, b = t[..., c].double() * 1e41, w[..., c] * 1e41
+        assert float((a - b).norm() / b.norm()) < 2e-2, n
