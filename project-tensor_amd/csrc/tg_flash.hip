@@ -1495,6 +1495,46 @@ struct FxSeen {
     return hi[0] >= lim || hi[1] >= lim;
   }
 };
+// As in the GEMM (k_gemm_rs): fp32 sums over staged rows are formed in parts of fx_part
+// rows, every second part from operands with their signs turned round, so that the parts err
+// to opposite sides; S and dP come out turned, too.  TWO: the parts are added up in a second
+// accumulator; else, where the registers do not hold one, the accumulator changes its sign.
+// Column sums of dQ, dK and dV (a bias gradient behind them), S 4096, unit normals: 2e-7 of
+// the entries with one accumulator and no turns, 2e-8 so, as on the fp32 matrix cores.
+template <bool TWO> constexpr int fx_part() { return TWO ? 128 : 64; }
+// The row after the part that begins at `row`, of `rows`; that part's sign.
+template <typename T, bool TWO>
+__device__ __forceinline__ int64_t fx_part_end(int64_t row, int64_t rows) {
+  return sizeof(T) == 4 && row + fx_part<TWO>() < rows ? row + fx_part<TWO>() : rows;
+}
+template <typename T, bool TWO> __device__ __forceinline__ float fx_sign(int64_t row) {
+  return sizeof(T) == 4 && (row / fx_part<TWO>()) % 2 != 0 ? -1.f : 1.f;
+}
+// The end of a part.
+template <typename T, bool TWO, int N, int M>
+__device__ __forceinline__ void fx_turn(f32x16 (&acc)[N], f32x16 (&sum)[M]) {
+  if (sizeof(T) != 4) return;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if constexpr (TWO) {
+      sum[i] = acc[i] - sum[i];
+      acc[i] = f32x16{};
+    } else {
+      acc[i] = -acc[i];
+    }
+  }
+}
+// The whole sum, after the last part; sg: that part's sign.
+template <typename T, bool TWO, int N, int M>
+__device__ __forceinline__ void fx_whole(f32x16 (&acc)[N], f32x16 (&sum)[M], float sg) {
+  if (sizeof(T) != 4) return;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if constexpr (TWO) acc[i] = sum[i] * sg;
+    else acc[i] *= -sg;
+  }
+}
+
 // Whether a scale factor leaves the scaled intermediates their range, and a result is one.
 __device__ __forceinline__ bool fx_bad_scale(float scale) {
   return !(fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p40f);
@@ -1558,15 +1598,15 @@ template <typename T> struct FxRaw {
     if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, w[e]);
     else return raw2f<T>(w[e / 2], e & 1);
   }
-  // row planes
-  __device__ __forceinline__ void rows(uint4 (&q)[Fx<T>::ROWP], FxSeen& seen) const {
+  // row planes (fp32 data times by)
+  __device__ __forceinline__ void rows(uint4 (&q)[Fx<T>::ROWP], float by, FxSeen& seen) const {
     if constexpr (sizeof(T) == 4) {
       unsigned* o[3] = {reinterpret_cast<unsigned*>(&q[0]), reinterpret_cast<unsigned*>(&q[1]),
                         reinterpret_cast<unsigned*>(&q[2])};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         unsigned t[3];
-        split2<3>(at(2 * e) * fx_by<T>(), at(2 * e + 1) * fx_by<T>(), t);
+        split2<3>(at(2 * e) * by, at(2 * e + 1) * by, t);
         seen.see(t[0]);
 #pragma unroll
         for (int i = 0; i < 3; ++i) o[i][e] = t[i];
@@ -1617,7 +1657,7 @@ struct FxOp {
       }
     }
   }
-  __device__ __forceinline__ void store(char* lds, int64_t row0, int64_t nrows, int D,
+  __device__ __forceinline__ void store(char* lds, int64_t row0, int64_t nrows, int D, float by,
                                         FxSeen& seen) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
@@ -1627,7 +1667,7 @@ struct FxOp {
       char* d = lds + r * RSB + c * 16;
       if constexpr (RP) {
         uint4 q[Fx<T>::ROWP];
-        raw[i].rows(q, seen);
+        raw[i].rows(q, by, seen);
 #pragma unroll
         for (int p = 0; p < Fx<T>::ROWP; ++p) *reinterpret_cast<uint4*>(d + p * PB) = q[p];
       }
@@ -1659,7 +1699,7 @@ struct FxOwn {
         r.load_n(g + row * rs + c, D - c);
       }
       uint4 q[Fx<T>::ROWP];
-      r.rows(q, seen);
+      r.rows(q, fx_by<T>(), seen);
 #pragma unroll
       for (int p = 0; p < Fx<T>::ROWP; ++p) f[ks][p] = __builtin_bit_cast(frag, q[p]);
     }
@@ -1758,7 +1798,7 @@ __device__ __forceinline__ void fx_acc(f32x16 (&acc)[DP / 32], const char* t, in
     }
 }
 
-template <typename T, int DP, int OCC>
+template <typename T, int DP, int OCC, bool TWO>
 __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
     const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
     T* __restrict__ O0, float* __restrict__ LSE0, int64_t Sq, int64_t Sk, int D, float scale,
@@ -1789,6 +1829,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  f32x16 sum[TWO ? NDB : 1] = {};
   const float sl2 = scale * kLog2e * fx_un<T>();
   float m = -INFINITY, l = 0.f;
   const int64_t kend = causal ? (qb * 128 + 128 < Sk ? qb * 128 + 128 : Sk) : Sk;
@@ -1796,58 +1837,71 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
   OV ov;
   ok.load(K, 0, Sk, rs, D, vec);
   ov.load(V, 0, Sk, rs, D, vec);
-  for (int64_t k0 = 0; k0 < kend; k0 += BN) {
-    __syncthreads();
-    ok.store(ks, k0, Sk, D, seen);
-    ov.store(vs, k0, Sk, D, seen);
-    if (k0 + BN < kend) {
-      ok.load(K, k0 + BN, Sk, rs, D, vec);
-      ov.load(V, k0 + BN, Sk, rs, D, vec);
+  for (int64_t p0 = 0; p0 < kend;) {
+    const float sg = fx_sign<T, TWO>(p0);
+    const int64_t pend = fx_part_end<T, TWO>(p0, kend);
+    for (int64_t k0 = p0; k0 < pend; k0 += BN) {
+      __syncthreads();
+      ok.store(ks, k0, Sk, D, sg * fx_by<T>(), seen);
+      ov.store(vs, k0, Sk, D, sg * fx_by<T>(), seen);
+      if (k0 + BN < kend) {
+        ok.load(K, k0 + BN, Sk, rs, D, vec);
+        ov.load(V, k0 + BN, Sk, rs, D, vec);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int kt = 0; kt < BN / 32; ++kt) {
+        const int64_t kb = k0 + kt * 32;
+        if (kb >= kend || (causal && kb > qw + 31)) break;
+        f32x16 s = fx_rows<T, DP>(ks + kt * 32 * RSB, OK::PB, own, l32, h);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] *= sg * sl2;
+        if (kb + 32 > Sk || (causal && kb + 31 > qw)) {
+          // keys past Sk or past this lane's query
+          int64_t last = Sk - 1 - kb - 4 * h;
+          if (causal && q - kb - 4 * h < last) last = q - kb - 4 * h;
+          const int thr = (int)last;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (8 * (r >> 2) + (r & 3) > thr) s[r] = -INFINITY;
+        }
+        float mloc = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, s[r]);
+        mloc = xhalf_max(mloc);
+        // O^T and l are rescaled only when some lane's maximum rose by more than kLazy; fp32:
+        // whenever one rose (v_exp_f32 errs more past 1: the probabilities of S 4096 unit
+        // normals added up to 1 + 3.2e-7 under kLazy and to 1 + 2.0e-7 so; forward 4 % slower)
+        if (__any(mloc > m + (sizeof(T) == 4 ? 0.f : kLazy))) {
+          const float mn = fmaxf(m, mloc), alpha = fexp2(m - (mn == -INFINITY ? 0.f : mn));
+          l *= alpha;
+#pragma unroll
+          for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+          if constexpr (TWO) {
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) sum[db] *= alpha;
+          }
+          m = mn;
+        }
+        const float mref = m == -INFINITY ? 0.f : m;  // (no key seen yet: p = 0)
+        float p[16], ps = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          p[r] = fexp2(s[r] - mref);
+          ps += p[r];
+        }
+        l += xhalf_sum(ps);
+        FxP<Fx<T>::PT> pt;
+        pt.split(p);
+        fx_acc<T, DP, true>(acc, vs + OV::TR0 * OV::PB + kt * 32 * RSB, OV::PB, pt, lane);
+      }
     }
-    __syncthreads();
-#pragma unroll
-    for (int kt = 0; kt < BN / 32; ++kt) {
-      const int64_t kb = k0 + kt * 32;
-      if (kb >= kend || (causal && kb > qw + 31)) break;
-      f32x16 s = fx_rows<T, DP>(ks + kt * 32 * RSB, OK::PB, own, l32, h);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] *= sl2;
-      if (kb + 32 > Sk || (causal && kb + 31 > qw)) {
-        // keys past Sk or past this lane's query
-        int64_t last = Sk - 1 - kb - 4 * h;
-        if (causal && q - kb - 4 * h < last) last = q - kb - 4 * h;
-        const int thr = (int)last;
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (8 * (r >> 2) + (r & 3) > thr) s[r] = -INFINITY;
-      }
-      float mloc = s[0];
-#pragma unroll
-      for (int r = 1; r < 16; ++r) mloc = fmaxf(mloc, s[r]);
-      mloc = xhalf_max(mloc);
-      // O^T and l are rescaled only when some lane's maximum rose by more than kLazy
-      if (__any(mloc > m + kLazy)) {
-        const float mn = fmaxf(m, mloc), alpha = fexp2(m - (mn == -INFINITY ? 0.f : mn));
-        l *= alpha;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
-        m = mn;
-      }
-      const float mref = m == -INFINITY ? 0.f : m;  // (no key seen yet: p = 0)
-      float p[16], ps = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p[r] = fexp2(s[r] - mref);
-        ps += p[r];
-      }
-      l += xhalf_sum(ps);
-      FxP<Fx<T>::PT> pt;
-      pt.split(p);
-      fx_acc<T, DP, true>(acc, vs + OV::TR0 * OV::PB + kt * 32 * RSB, OV::PB, pt, lane);
-    }
+    fx_turn<T, TWO>(acc, sum);
+    p0 = pend;
   }
+  fx_whole<T, TWO>(acc, sum, fx_sign<T, TWO>(kend - 1));
   if constexpr (sizeof(T) == 4) {
     if (__syncthreads_or(seen.bad() || fx_bad_scale(scale) || fx_bad(acc))) {
       float* f = reinterpret_cast<float*>(sm);
@@ -1906,7 +1960,7 @@ __device__ __forceinline__ void fx_store(T* __restrict__ out, int rs, int64_t ro
   }
 }
 
-template <typename T, int DP, int OCC>
+template <typename T, int DP, int OCC, bool TWO>
 __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
     const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
     const T* __restrict__ O0, const T* __restrict__ dO0, const float* __restrict__ LSE0,
@@ -1963,43 +2017,51 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  f32x16 sum[TWO ? NDB : 1] = {};
   const int64_t kend = causal ? (qb * 128 + 128 < Sk ? qb * 128 + 128 : Sk) : Sk;
   OK ok;
   OV ov;
   ok.load(K, 0, Sk, rs, D, vec);
   ov.load(V, 0, Sk, rs, D, vec);
-  for (int64_t k0 = 0; k0 < kend; k0 += BN) {
-    __syncthreads();
-    ok.store(ks, k0, Sk, D, seen);
-    ov.store(vs, k0, Sk, D, seen);
-    if (k0 + BN < kend) {
-      ok.load(K, k0 + BN, Sk, rs, D, vec);
-      ov.load(V, k0 + BN, Sk, rs, D, vec);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kt = 0; kt < BN / 32; ++kt) {
-      const int64_t kb = k0 + kt * 32;
-      if (kb >= kend || (causal && kb > qw + 31)) break;
-      const f32x16 s = fx_rows<T, DP>(ks + kt * 32 * RSB, OK::PB, own, l32, h);
-      const f32x16 dp = fx_rows<T, DP>(vs + kt * 32 * RSB, OV::PB, od, l32, h);
-      int thr = 1 << 30;
-      if (kb + 32 > Sk || (causal && kb + 31 > qw)) {
-        int64_t last = Sk - 1 - kb - 4 * h;
-        if (causal && q - kb - 4 * h < last) last = q - kb - 4 * h;
-        thr = (int)last;
+  for (int64_t p0 = 0; p0 < kend;) {
+    const float sg = fx_sign<T, TWO>(p0);
+    const int64_t pend = fx_part_end<T, TWO>(p0, kend);
+    for (int64_t k0 = p0; k0 < pend; k0 += BN) {
+      __syncthreads();
+      ok.store(ks, k0, Sk, D, sg * fx_by<T>(), seen);
+      ov.store(vs, k0, Sk, D, sg * fx_by<T>(), seen);
+      if (k0 + BN < kend) {
+        ok.load(K, k0 + BN, Sk, rs, D, vec);
+        ov.load(V, k0 + BN, Sk, rs, D, vec);
       }
-      float ds[16];
+      __syncthreads();
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = 8 * (r >> 2) + (r & 3) > thr ? 0.f : fexp2(fmaf(s[r], sl2, -lq));
-        ds[r] = p * (dp[r] - dsum) * sds;
+      for (int kt = 0; kt < BN / 32; ++kt) {
+        const int64_t kb = k0 + kt * 32;
+        if (kb >= kend || (causal && kb > qw + 31)) break;
+        const f32x16 s = fx_rows<T, DP>(ks + kt * 32 * RSB, OK::PB, own, l32, h);
+        const f32x16 dp = fx_rows<T, DP>(vs + kt * 32 * RSB, OV::PB, od, l32, h);
+        int thr = 1 << 30;
+        if (kb + 32 > Sk || (causal && kb + 31 > qw)) {
+          int64_t last = Sk - 1 - kb - 4 * h;
+          if (causal && q - kb - 4 * h < last) last = q - kb - 4 * h;
+          thr = (int)last;
+        }
+        float ds[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float p = 8 * (r >> 2) + (r & 3) > thr ? 0.f : fexp2(fmaf(s[r], sg * sl2, -lq));
+          ds[r] = p * (sg * dp[r] - dsum) * sds;
+        }
+        FxP<Fx<T>::PT> pt;
+        pt.split(ds);
+        fx_acc<T, DP, false>(acc, ks + OK::TR0 * OK::PB + kt * 32 * RSB, OK::PB, pt, lane);
       }
-      FxP<Fx<T>::PT> pt;
-      pt.split(ds);
-      fx_acc<T, DP, false>(acc, ks + OK::TR0 * OK::PB + kt * 32 * RSB, OK::PB, pt, lane);
     }
+    fx_turn<T, TWO>(acc, sum);
+    p0 = pend;
   }
+  fx_whole<T, TWO>(acc, sum, fx_sign<T, TWO>(kend - 1));
   if constexpr (sizeof(T) == 4) {
     if (__syncthreads_or(seen.bad() || fx_bad_scale(scale) || fx_bad(acc))) {
       float* f = reinterpret_cast<float*>(sm);
@@ -2011,7 +2073,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
   fx_store<T, DP>(dQ, rs, qw, Sq, D, acc, fx_un<T>(), accumulate, l32, h);
 }
 
-template <typename T, int DP, int OCC>
+template <typename T, int DP, int OCC, bool TWO>
 __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
     const T* __restrict__ dO0, const float* __restrict__ LSE0, const float* __restrict__ Dv0,
@@ -2048,6 +2110,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.f;
+  f32x16 sk[TWO ? NDB : 1] = {}, sv[TWO ? NDB : 1] = {};
   const int64_t qstart = causal ? kblk : 0;
   OQ oq, od;
   float lv = 0.f, dd = 0.f;
@@ -2061,48 +2124,59 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     oq.load(Q, qstart, Sq, rs, D, vec);
     od.load(dO, qstart, Sq, ro, D, vec);
   }
-  for (int64_t q0 = qstart; q0 < Sq; q0 += BN) {
-    __syncthreads();
-    oq.store(qs, q0, Sq, D, seen);
-    od.store(dos, q0, Sq, D, seen);
-    if (threadIdx.x < BN) {  // (+inf past Sq: P = 0 there)
-      ls[threadIdx.x] = q0 + threadIdx.x < Sq ? lv * kLog2e : INFINITY;
-      dsm[threadIdx.x] = q0 + threadIdx.x < Sq ? dd / fx_un<T>() : 0.f;
-    }
-    if (q0 + BN < Sq) {
-      rows(q0 + BN);
-      oq.load(Q, q0 + BN, Sq, rs, D, vec);
-      od.load(dO, q0 + BN, Sq, ro, D, vec);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < BN / 32; ++t) {
-      const int64_t qb0 = q0 + t * 32;
-      if (qb0 >= Sq) break;
-      if (causal && qb0 + 31 < kw) continue;  // wholly before this wave's keys
-      const f32x16 s = fx_rows<T, DP>(qs + t * 32 * RSB, OQ::PB, kf, l32, h);
-      const f32x16 dp = fx_rows<T, DP>(dos + t * 32 * RSB, OQ::PB, vf, l32, h);
-      const bool diag = causal && kw + 31 > qb0;
-      const int mb = diag ? (int)(key - qb0) - 4 * h : -1;  // rows below it are masked
-      float p[16], ds[16];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 a = *reinterpret_cast<const float4*>(ls + t * 32 + 8 * g + 4 * h);
-        const float4 b = *reinterpret_cast<const float4*>(dsm + t * 32 + 8 * g + 4 * h);
-        const float la[4] = {a.x, a.y, a.z, a.w}, db[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * g + i;
-          p[r] = 8 * g + i < mb ? 0.f : fexp2(fmaf(s[r], sl2, -la[i]));
-          ds[r] = p[r] * (dp[r] - db[i]) * sds;
-        }
+  for (int64_t p0 = qstart; p0 < Sq;) {
+    const float sg = fx_sign<T, TWO>(p0);
+    const int64_t pend = fx_part_end<T, TWO>(p0, Sq);
+    for (int64_t q0 = p0; q0 < pend; q0 += BN) {
+      __syncthreads();
+      oq.store(qs, q0, Sq, D, sg * fx_by<T>(), seen);
+      od.store(dos, q0, Sq, D, sg * fx_by<T>(), seen);
+      if (threadIdx.x < BN) {  // (+inf past Sq: P = 0 there)
+        ls[threadIdx.x] = q0 + threadIdx.x < Sq ? lv * kLog2e : INFINITY;
+        dsm[threadIdx.x] = q0 + threadIdx.x < Sq ? dd / fx_un<T>() : 0.f;
       }
-      FxP<Fx<T>::PT> pt;
-      pt.split(p);
-      fx_acc<T, DP, false>(dv, dos + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
-      pt.split(ds);
-      fx_acc<T, DP, false>(dk, qs + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
+      if (q0 + BN < Sq) {
+        rows(q0 + BN);
+        oq.load(Q, q0 + BN, Sq, rs, D, vec);
+        od.load(dO, q0 + BN, Sq, ro, D, vec);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < BN / 32; ++t) {
+        const int64_t qb0 = q0 + t * 32;
+        if (qb0 >= Sq) break;
+        if (causal && qb0 + 31 < kw) continue;  // wholly before this wave's keys
+        const f32x16 s = fx_rows<T, DP>(qs + t * 32 * RSB, OQ::PB, kf, l32, h);
+        const f32x16 dp = fx_rows<T, DP>(dos + t * 32 * RSB, OQ::PB, vf, l32, h);
+        const bool diag = causal && kw + 31 > qb0;
+        const int mb = diag ? (int)(key - qb0) - 4 * h : -1;  // rows below it are masked
+        float p[16], ds[16];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 a = *reinterpret_cast<const float4*>(ls + t * 32 + 8 * g + 4 * h);
+          const float4 b = *reinterpret_cast<const float4*>(dsm + t * 32 + 8 * g + 4 * h);
+          const float la[4] = {a.x, a.y, a.z, a.w}, db[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int r = 4 * g + i;
+            p[r] = 8 * g + i < mb ? 0.f : fexp2(fmaf(s[r], sg * sl2, -la[i]));
+            ds[r] = p[r] * (sg * dp[r] - db[i]) * sds;
+          }
+        }
+        FxP<Fx<T>::PT> pt;
+        pt.split(p);
+        fx_acc<T, DP, false>(dv, dos + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
+        pt.split(ds);
+        fx_acc<T, DP, false>(dk, qs + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
+      }
     }
+    fx_turn<T, TWO>(dk, sk);
+    fx_turn<T, TWO>(dv, sv);
+    p0 = pend;
+  }
+  if (qstart < Sq) {
+    fx_whole<T, TWO>(dk, sk, fx_sign<T, TWO>(Sq - 1));
+    fx_whole<T, TWO>(dv, sv, fx_sign<T, TWO>(Sq - 1));
   }
   if constexpr (sizeof(T) == 4) {
     if (__syncthreads_or(seen.bad() || fx_bad_scale(scale) || fx_bad(dk) || fx_bad(dv))) {
@@ -2121,6 +2195,9 @@ template <typename T, int DP> struct FxOcc {
   static constexpr int FWD = sizeof(T) == 4 && DP > 64 ? 1 : 2;
   static constexpr int DQ = sizeof(T) == 4 && DP > 64 ? 1 : 2;
   static constexpr int DKDV = sizeof(T) == 4 ? (DP > 32 ? 1 : 2) : (DP > 64 ? 1 : 2);
+  // fp32: whether they hold the second accumulator, too
+  static constexpr bool FWD2 = sizeof(T) == 4, DQ2 = sizeof(T) == 4 && (DP == 32 || DP == 96),
+                        DKDV2 = sizeof(T) == 4 && DP <= 64;
 };
 
 template <typename T, int DP>
@@ -2128,7 +2205,7 @@ int fwd_split_t(const void* q, const void* k, const void* v, void* o, float* lse
                 int64_t Sq, int64_t Sk, int D, float scale, int causal, int vec, FaLay lay,
                 hipStream_t s) {
   dim3 grid((unsigned)((Sq + 127) / 128), (unsigned)BH);
-  k_fa_fwd_split<T, DP, FxOcc<T, DP>::FWD><<<grid, kThreads, 0, s>>>(
+  k_fa_fwd_split<T, DP, FxOcc<T, DP>::FWD, FxOcc<T, DP>::FWD2><<<grid, kThreads, 0, s>>>(
       (const T*)q, (const T*)k, (const T*)v, (T*)o, lse, Sq, Sk, D, scale, causal, vec, lay);
   return tg_check_launch("tg_flash_attn_fwd");
 }
@@ -2138,11 +2215,11 @@ int bwd_split_t(const void* q, const void* k, const void* v, const void* o, cons
                 int D, float scale, int causal, int acc, float* dvec, int vec, FaLay lay,
                 hipStream_t s) {
   dim3 gq((unsigned)((Sq + 127) / 128), (unsigned)BH);
-  k_fa_bwd_dq_split<T, DP, FxOcc<T, DP>::DQ><<<gq, kThreads, 0, s>>>(
+  k_fa_bwd_dq_split<T, DP, FxOcc<T, DP>::DQ, FxOcc<T, DP>::DQ2><<<gq, kThreads, 0, s>>>(
       (const T*)q, (const T*)k, (const T*)v, (const T*)o, (const T*)dout, lse, dvec, (T*)dq, Sq, Sk,
       D, scale, causal, acc, vec, lay);
   dim3 gkv((unsigned)((Sk + 127) / 128), (unsigned)BH);
-  k_fa_bwd_dkdv_split<T, DP, FxOcc<T, DP>::DKDV><<<gkv, kThreads, 0, s>>>(
+  k_fa_bwd_dkdv_split<T, DP, FxOcc<T, DP>::DKDV, FxOcc<T, DP>::DKDV2><<<gkv, kThreads, 0, s>>>(
       (const T*)q, (const T*)k, (const T*)v, (const T*)dout, lse, dvec, (T*)dk, (T*)dv, Sq, Sk, D,
       scale, causal, acc, vec, lay);
   return tg_check_launch("tg_flash_attn_bwd");

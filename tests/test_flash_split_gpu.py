@@ -131,3 +131,41 @@ def test_split_attention_fp32_subnormal_columns(cuda, D, S, causal):
         _close(t, w, torch.float32, n, 2.0)
         a, b = t[..., c].double() * 1e41, w[..., c] * 1e41
         assert float((a - b).norm() / b.norm()) < 2e-2, n
+
+
+@pytest.mark.parametrize("D", [32, 64, 80, 128])
+@pytest.mark.parametrize("S,causal,offset", [(2048, False, False), (4096, False, False),
+                                             (4096, False, True), (2011, True, False)])
+def test_split_attention_fp32_column_sums(cuda, D, S, causal, offset):
+    """Entries that err to either side at random (up to 1.2e-6 of their size here, as on the
+    fp32 matrix cores) leave 1/sqrt(S) of that in a column sum relative to S entries; held to
+    twice it.  Sums that err downwards leave 1e-7 at S = 2048 and 2e-7 at 4096."""
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v, do = (torch.randn(1, 3, S, D, generator=g, device="cuda") for _ in range(4))
+    if offset:
+        v += 3
+    sc = D ** -0.5
+    o, lse = L().flash_attn_fwd(q, k, v, sc, causal)
+    grads = [torch.empty_like(q) for _ in range(3)]
+    L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, causal, False)
+    want = _ref(q, k, v, do, sc, causal)
+    for t, w, n in zip([o] + grads[:2], want, ("o", "dq", "dk")):
+        if offset and n != "o":  # (dP - D cancels: the entries themselves are further off)
+            continue
+        d = (t.double() - w).sum(2)
+        e = float(d.norm() / (w.norm(dim=2) * S ** 0.5).norm())
+        assert e < 2 * 1.2e-6 / S ** 0.5, f"{n}: {e:.2e}"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_split_attention_fp32_probabilities_add_up(cuda, D):
+    """With dO = 1, the column sums of dV are the sums of the probabilities: S, up to v_exp_f32's
+    error, which a stale maximum in the forward (arguments of either sign) adds to."""
+    S = 4096
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v = (torch.randn(1, 3, S, D, generator=g, device="cuda") for _ in range(3))
+    do = torch.ones_like(q)
+    o, lse = L().flash_attn_fwd(q, k, v, D ** -0.5, False)
+    grads = [torch.empty_like(q) for _ in range(3)]
+    L().flash_attn_bwd(q, k, v, o, do, lse, *grads, D ** -0.5, False, False)
+    assert abs(float(grads[2].double().sum(2).mean()) / S - 1) < 2.5e-7
