@@ -1213,7 +1213,7 @@ __device__ __forceinline__ void fa_fwd_gen(float* Ks, float* Vs, const T* __rest
 // [z*DO, z*DO + DO) of dQ (S and dP are recomputed per column range).
 template <typename T, int DP, int DO>
 __device__ __forceinline__ void fa_bwd_dq_gen(
-    float* Ks, float* Vs, const T* __restrict__ Q, const T* __restrict__ K,
+    int z, float* Ks, float* Vs, const T* __restrict__ Q, const T* __restrict__ K,
     const T* __restrict__ V, const T* __restrict__ O, const T* __restrict__ dO,
     const float* __restrict__ LSE, float* __restrict__ Dv, T* __restrict__ dQ, int64_t Sq,
     int64_t Sk, int D, float scale, int causal, int accumulate, FaLay lay) {
@@ -1231,7 +1231,7 @@ __device__ __forceinline__ void fa_bwd_dq_gen(
   const int rs = lay.rsa, ro = lay.rso;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h = lane >> 5, l32 = lane & 31;
-  const int d0 = blockIdx.z * DO;
+  const int d0 = z * DO;
   const int64_t qb = causal ? (int64_t)gridDim.x - 1 - tile : tile;
   const int64_t q = qb * 128 + wave * 32 + l32;
   const bool qv = q < Sq;
@@ -1247,7 +1247,7 @@ __device__ __forceinline__ void fa_bwd_dq_gen(
       if (qv && d < D) dsum += gld(O, q * ro + d) * dor[4 * t + e];
     }
   dsum += __shfl_xor(dsum, 32, 64);
-  if (qv && h == 0 && blockIdx.z == 0) Dv[q] = dsum;
+  if (qv && h == 0 && z == 0) Dv[q] = dsum;
   const float lq = qv ? LSE[q] * kLog2e : 0.f;
   const float sl2 = scale * kLog2e;
   f32x16 acc[NDB];
@@ -1291,8 +1291,8 @@ __device__ __forceinline__ void fa_bwd_dq_gen(
 // [z*DO, z*DO + DO) of dK and dV.
 template <typename T, int DP, int DO>
 __device__ __forceinline__ void fa_bwd_dkdv_gen(
-    float* Qs, float* dOs, float* ls, float* ds, const T* __restrict__ Q, const T* __restrict__ K,
-    const T* __restrict__ V, const T* __restrict__ dO, const float* __restrict__ LSE,
+    int z, float* Qs, float* dOs, float* ls, float* ds, const T* __restrict__ Q,
+    const T* __restrict__ K, const T* __restrict__ V, const T* __restrict__ dO, const float* __restrict__ LSE,
     const float* __restrict__ Dv, T* __restrict__ dK, T* __restrict__ dV, int64_t Sq, int64_t Sk,
     int D, float scale, int causal, int accumulate, FaLay lay) {
   constexpr int NS = DP / 2, NDB = DO / 32;
@@ -1309,7 +1309,7 @@ __device__ __forceinline__ void fa_bwd_dkdv_gen(
   const int rs = lay.rsa, ro = lay.rso;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h = lane >> 5, l32 = lane & 31;
-  const int d0 = blockIdx.z * DO;
+  const int d0 = z * DO;
   // causal: the first key blocks see the most queries, so they are dispatched first
   const int64_t kb = tile;
   const int64_t key = kb * 128 + wave * 32 + l32;
@@ -1383,7 +1383,7 @@ __global__ __launch_bounds__(kThreads) void k_fa_bwd_dq_gen(
     int causal, int accumulate, FaLay lay) {
   __shared__ __attribute__((aligned(16))) char sm[gen_lds<DP>()];
   float* f = reinterpret_cast<float*>(sm);
-  fa_bwd_dq_gen<T, DP, DO>(f, f + gen_lds<DP>() / 8, Q, K, V, O, dO, LSE, Dv, dQ, Sq, Sk, D, scale,
+  fa_bwd_dq_gen<T, DP, DO>(blockIdx.z, f, f + gen_lds<DP>() / 8, Q, K, V, O, dO, LSE, Dv, dQ, Sq, Sk, D, scale,
                            causal, accumulate, lay);
 }
 
@@ -1396,7 +1396,7 @@ __global__ __launch_bounds__(kThreads) void k_fa_bwd_dkdv_gen(
   __shared__ __attribute__((aligned(16))) char sm[gen_lds<DP>()];
   __shared__ float ls[32], ds[32];
   float* f = reinterpret_cast<float*>(sm);
-  fa_bwd_dkdv_gen<T, DP, DO>(f, f + gen_lds<DP>() / 8, ls, ds, Q, K, V, dO, LSE, Dv, dK, dV, Sq, Sk,
+  fa_bwd_dkdv_gen<T, DP, DO>(blockIdx.z, f, f + gen_lds<DP>() / 8, ls, ds, Q, K, V, dO, LSE, Dv, dK, dV, Sq, Sk,
                              D, scale, causal, accumulate, lay);
 }
 
@@ -1447,8 +1447,8 @@ int bwd_gen_t(const void* q, const void* k, const void* v, const void* o, const 
 // bf16 MFMAs instead of 64 fp32 ones of twice the time, the backward 168 instead of 224.
 // fp32 data are multiplied by 2^24 before they are split (and sums by its inverses), so that
 // every term of any fp32 number is a normal bf16 number; dS is formed 2^24 times too large
-// for the same reason.  Values of 2^36 and more (their products could overflow then), Inf
-// and NaN, and results past 2^80, make the workgroup run the generic kernel's body instead:
+// for the same reason.  Values of 2^36 and more (their products could overflow then) and
+// non-finite sums, of either width, make the workgroup run the generic kernel's body instead:
 // B*H 64, S 1024, d 64, causal, with such a value in every head: forward 250 us, backward
 // 740 to 790, instead of 69 and 230 (the generic kernels alone 234 and 600).
 //
@@ -1535,12 +1535,16 @@ __device__ __forceinline__ void fx_whole(f32x16 (&acc)[N], f32x16 (&sum)[M], flo
   }
 }
 
-// Whether a scale factor leaves the scaled intermediates their range, and a result is one.
+// Whether a scale factor leaves the scaled intermediates no range.
 __device__ __forceinline__ bool fx_bad_scale(float scale) {
   return !(fabsf(scale) >= 0x1p-60f && fabsf(scale) <= 0x1p40f);
 }
-template <int N> __device__ __forceinline__ bool fx_bad(const f32x16 (&acc)[N]) {
-  bool bad = false;
+// Whether the workgroup has to run the generic body: non-finite sums (of 16-bit data, too:
+// an infinity times the low terms of P or dS, or split into terms, is NaN where the product
+// itself is infinite), and fp32 data or a scale outside the range.
+template <typename T, int N>
+__device__ __forceinline__ bool fx_redo(const f32x16 (&acc)[N], const FxSeen& seen, float scale) {
+  bool bad = sizeof(T) == 4 && (seen.bad() || fx_bad_scale(scale));
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll
@@ -1806,7 +1810,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
   using OK = FxOp<T, DP, true, false>;
   using OV = FxOp<T, DP, false, true>;
   constexpr int BN = Fx<T>::BN, RSB = OK::RSB, NDB = DP / 32;
-  constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = sizeof(T) == 4 ? gen_lds<DP>() : 0;
+  constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = gen_lds<DP>();
   __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
   char *ks = sm, *vs = sm + OK::BYTES;
   int64_t tile, bh;
@@ -1902,13 +1906,11 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
     p0 = pend;
   }
   fx_whole<T, TWO>(acc, sum, fx_sign<T, TWO>(kend - 1));
-  if constexpr (sizeof(T) == 4) {
-    if (__syncthreads_or(seen.bad() || fx_bad_scale(scale) || fx_bad(acc))) {
-      float* f = reinterpret_cast<float*>(sm);
-      fa_fwd_gen<T, DP>(f, f + gen_lds<DP>() / 8, Q0, K0, V0, O0, LSE0, Sq, Sk, D, scale, causal,
-                        lay);
-      return;
-    }
+  if (__syncthreads_or(fx_redo<T>(acc, seen, scale))) {
+    float* f = reinterpret_cast<float*>(sm);
+    fa_fwd_gen<T, DP>(f, f + gen_lds<DP>() / 8, Q0, K0, V0, O0, LSE0, Sq, Sk, D, scale, causal,
+                      lay);
+    return;
   }
   if (q < Sq) {
     const float inv = l > 0.f ? 1.f / l / fx_by<T>() : 0.f;
@@ -1969,7 +1971,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
   using OK = FxOp<T, DP, true, true>;
   using OV = FxOp<T, DP, true, false>;
   constexpr int BN = Fx<T>::BN, RSB = OK::RSB, NDB = DP / 32;
-  constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = sizeof(T) == 4 ? gen_lds<DP>() : 0;
+  constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = gen_lds<DP>();
   __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
   char *ks = sm, *vs = sm + OK::BYTES;
   int64_t tile, bh;
@@ -2062,13 +2064,13 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
     p0 = pend;
   }
   fx_whole<T, TWO>(acc, sum, fx_sign<T, TWO>(kend - 1));
-  if constexpr (sizeof(T) == 4) {
-    if (__syncthreads_or(seen.bad() || fx_bad_scale(scale) || fx_bad(acc))) {
-      float* f = reinterpret_cast<float*>(sm);
-      fa_bwd_dq_gen<T, DP, DP>(f, f + gen_lds<DP>() / 8, Q0, K0, V0, O0, dO0, LSE0, Dv0, dQ0, Sq, Sk,
-                               D, scale, causal, accumulate, lay);
-      return;
-    }
+  if (__syncthreads_or(fx_redo<T>(acc, seen, scale))) {
+    float* f = reinterpret_cast<float*>(sm);
+#pragma unroll 1
+    for (int z = 0; z < DP / 32; ++z)  // (32 columns at a time: fewer registers than the loop's)
+      fa_bwd_dq_gen<T, DP, 32>(z, f, f + gen_lds<DP>() / 8, Q0, K0, V0, O0, dO0, LSE0, Dv0, dQ0, Sq,
+                               Sk, D, scale, causal, accumulate, lay);
+    return;
   }
   fx_store<T, DP>(dQ, rs, qw, Sq, D, acc, fx_un<T>(), accumulate, l32, h);
 }
@@ -2081,7 +2083,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     int causal, int accumulate, int vec, FaLay lay) {
   using OQ = FxOp<T, DP, true, true>;
   constexpr int BN = Fx<T>::BN, RSB = OQ::RSB, NDB = DP / 32;
-  constexpr int BYTES = 2 * OQ::BYTES, GEN = sizeof(T) == 4 ? gen_lds<DP>() : 0;
+  constexpr int BYTES = 2 * OQ::BYTES, GEN = gen_lds<DP>();
   __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
   __shared__ __attribute__((aligned(16))) float ls[BN], dsm[BN];
   char *qs = sm, *dos = sm + OQ::BYTES;
@@ -2178,13 +2180,13 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     fx_whole<T, TWO>(dk, sk, fx_sign<T, TWO>(Sq - 1));
     fx_whole<T, TWO>(dv, sv, fx_sign<T, TWO>(Sq - 1));
   }
-  if constexpr (sizeof(T) == 4) {
-    if (__syncthreads_or(seen.bad() || fx_bad_scale(scale) || fx_bad(dk) || fx_bad(dv))) {
-      float* f = reinterpret_cast<float*>(sm);
-      fa_bwd_dkdv_gen<T, DP, DP>(f, f + gen_lds<DP>() / 8, ls, dsm, Q0, K0, V0, dO0, LSE0, Dv0, dK0,
-                                 dV0, Sq, Sk, D, scale, causal, accumulate, lay);
-      return;
-    }
+  if (__syncthreads_or(fx_redo<T>(dk, seen, scale) || fx_redo<T>(dv, seen, scale))) {
+    float* f = reinterpret_cast<float*>(sm);
+#pragma unroll 1
+    for (int z = 0; z < DP / 32; ++z)
+      fa_bwd_dkdv_gen<T, DP, 32>(z, f, f + gen_lds<DP>() / 8, ls, dsm, Q0, K0, V0, dO0, LSE0, Dv0,
+                                 dK0, dV0, Sq, Sk, D, scale, causal, accumulate, lay);
+    return;
   }
   fx_store<T, DP>(dK, rs, kw, Sk, D, dk, fx_un<T>(), accumulate, l32, h);
   fx_store<T, DP>(dV, rs, kw, Sk, D, dv, 1.f / fx_by<T>(), accumulate, l32, h);

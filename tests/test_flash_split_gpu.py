@@ -169,3 +169,37 @@ def test_split_attention_fp32_probabilities_add_up(cuda, D):
     grads = [torch.empty_like(q) for _ in range(3)]
     L().flash_attn_bwd(q, k, v, o, do, lse, *grads, D ** -0.5, False, False)
     assert abs(float(grads[2].double().sum(2).mean()) / S - 1) < 2.5e-7
+
+
+@pytest.mark.parametrize("dt", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("D", [32, 80, 128])
+@pytest.mark.parametrize("where", ["v", "do", "q"])
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan")])
+def test_split_attention_non_finite(cuda, D, dt, where, value):
+    """Infinities stay infinities, of their sign, and NaN spreads no further than by the
+    formulas.  Misaligned (by one element): head dim 128 would run on the tuned kernels."""
+    dt = DT[dt]
+    g = torch.Generator(device="cuda").manual_seed(D)
+    S = 150
+
+    def mk():
+        buf = torch.randn(1 * 2 * S * D + 1, generator=g, device="cuda").to(dt)
+        return buf[1:].view(1, 2, S, D)
+    q, k, v, do = mk(), mk(), mk(), mk()
+    {"q": q, "v": v, "do": do}[where][0, 0, 11, 2] = value
+    sc = 0.5 * D ** -0.5
+    o, lse = L().flash_attn_fwd(q, k, v, sc, False)
+    grads = [mk() for _ in range(3)]
+    L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, False, False)
+    want = _ref(q, k, v, do, sc, False)
+    for t, w, n in zip([o] + grads, want, ("o", "dq", "dk", "dv")):
+        assert torch.equal(torch.isfinite(t), torch.isfinite(w)), n
+        # (dS = P (dP - D) is Inf - Inf or not by the order of D's sum, P of a row of infinite
+        # scores Inf or NaN by the form of its lse)
+        if n == "o" or (n == "dv" and where != "q"):
+            assert torch.equal(torch.isnan(t), torch.isnan(w)), n
+            inf = torch.isinf(w)
+            assert torch.equal(t[inf].double(), w[inf]), n
+        ok = torch.isfinite(w)
+        if bool(ok.any()):
+            _close(t[ok], w[ok], dt, n, 2.0)
