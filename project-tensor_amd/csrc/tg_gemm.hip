@@ -537,6 +537,21 @@ __device__ __forceinline__ float epi_val(float v, float x, float beta, float c) 
   return v;
 }
 
+// Write-back of C without a fused epilogue: its rows start at any element (an odd N, a view),
+// which global memory takes; the type says so.
+typedef unsigned c_u32x4 __attribute__((ext_vector_type(4), aligned(2), may_alias));
+template <typename TC> __device__ __forceinline__ tg_vec16<TC> c_load16(const TC* p) {
+  tg_vec16<TC> r;
+  const c_u32x4 u = *reinterpret_cast<const c_u32x4*>(p);
+  __builtin_memcpy(&r, &u, 16);
+  return r;
+}
+template <typename TC> __device__ __forceinline__ void c_store16(TC* p, const void* v) {
+  c_u32x4 u;
+  __builtin_memcpy(&u, v, 16);
+  *reinterpret_cast<c_u32x4*>(p) = u;
+}
+
 // TAIL: K may end inside a k-tile (its own instantiation: the extra path costs the others
 // about 1 %).
 // EXT: the caller names the tile (row tile xtm, column tile xtn); otherwise it follows
@@ -801,14 +816,14 @@ __device__ __forceinline__ void v3_tile(
               tg_store16(pc, o);
             }
           } else if (beta != 0.f) {
-            tg_vec16<TC> o, c = tg_load16(pc);
+            tg_vec16<TC> o, c = c_load16(pc);
             *reinterpret_cast<uint4*>(&o) = v;
 #pragma unroll
             for (int e = 0; e < tg_vec16<TC>::N; ++e)
               o.v[e] = tg_from_float<TC>(tg_to_float(o.v[e]) + beta * tg_to_float(c.v[e]));
-            tg_store16(pc, o);
+            c_store16(pc, &o);
           } else {
-            *reinterpret_cast<uint4*>(pc) = v;
+            c_store16(pc, &v);
           }
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);

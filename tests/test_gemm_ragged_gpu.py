@@ -118,3 +118,29 @@ def test_epilogue_ragged_equals_separate(cuda, M, N, K):
         want = torch.empty_like(ref)
         L().act_bwd("gelu", r, L().matmul2d(a, w, trans_b=True), want, False)
         assert torch.equal(d, want)
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("odt", ["same", "fp32"])
+@pytest.mark.parametrize("M,N,K,off", [(256, 257, 128, 1), (300, 1025, 72, 0), (512, 515, 264, 3),
+                                       (1024, 2049, 64, 7), (129, 131, 40, 5)])
+def test_gemm_rows_of_c_at_any_element(cuda, M, N, K, off, odt, dt):
+    """Full tiles written to (and, accumulating, read from) rows of C that start at any
+    element; nothing past C's ends is touched.  Operands of -1, 0 and 1: every sum is a whole
+    number below 2^8, exact in each type."""
+    dt = DT[dt]
+    odt = dt if odt == "same" else torch.float32
+    g = torch.Generator(device="cuda").manual_seed(N)
+    a, b = (torch.randint(-1, 2, (r, K), generator=g, device="cuda").to(dt) for r in (M, N))
+    want = a.float() @ b.float().t().contiguous()
+    assert float(want.abs().max()) < 250
+    for beta in (0.0, 1.0):
+        buf = torch.full((M * N + off + 64,), 2.0, device="cuda", dtype=odt)
+        c = buf[off:off + M * N].view(M, N)
+        L().gemm(a, b, c, False, True, 1.0, beta, M, N, K, K, K, N)
+        assert torch.equal(c.float(), want + 2 * beta)
+        assert bool((buf[:off] == 2).all()) and bool((buf[off + M * N:] == 2).all())
+        # B as [K, N], odd rows: copied with aligned ones
+        d = torch.full((M, N), 2.0, device="cuda", dtype=odt)
+        L().matmul2d(a, b.t().contiguous(), d, beta=beta)
+        assert torch.equal(d.float(), want + 2 * beta)
