@@ -774,16 +774,45 @@ __device__ __forceinline__ void v3_tile(
                 ch * (16 / (int)sizeof(TC)));
           }
         }
-        // accumulator registers r in [half*16*HR/32, ...): rows half*HR .. half*HR+HR-1
-#pragma unroll
-        for (int j = 0; j < SN; ++j)
-#pragma unroll
-          for (int rr = 0; rr < HR / 2; ++rr) {
-            const int r = half * (HR / 2) + rr;
-            const int row = (r >> 2) * 8 + lh * 4 + (r & 3) - half * HR;
-            *reinterpret_cast<TC*>(slab + row * RS + (j * 32 + l32) * (int)sizeof(TC)) =
-                tg_from_float<TC>(alpha * acc[i][j][r] + bv[j]);
+        // 16-bit C that is added to goes to the slab first, so that the sum is formed in fp32
+        // and rounded once, as in the edge tiles
+        constexpr bool CADD = EPI == EPI_NONE && sizeof(TC) == 2;
+        const bool cadd = CADD && beta != 0.f;
+        if (cadd) {
+#pragma unroll 2
+          for (int q = 0; q < NQ; ++q) {  // (a few at a time: all at once spill accumulators)
+            const int u = q * 64 + lane, row = u / CPR, ch = u % CPR;
+            const tg_vec16<TC> c = c_load16(C + (m0 + wm + i * 32 + half * HR + row) * ldc + n0 +
+                                            wn + ch * (16 / (int)sizeof(TC)));
+            *reinterpret_cast<uint4*>(slab + row * RS + ch * 16) =
+                *reinterpret_cast<const uint4*>(&c);
           }
+          __builtin_amdgcn_s_waitcnt(0xc07f);
+          __builtin_amdgcn_wave_barrier();
+        }
+        // accumulator registers r in [half*16*HR/32, ...): rows half*HR .. half*HR+HR-1
+        auto slab_at = [&](int j, int rr) {
+          const int r = half * (HR / 2) + rr;
+          const int row = (r >> 2) * 8 + lh * 4 + (r & 3) - half * HR;
+          return reinterpret_cast<TC*>(slab + row * RS + (j * 32 + l32) * (int)sizeof(TC));
+        };
+        if (cadd) {
+#pragma unroll
+          for (int j = 0; j < SN; ++j)
+#pragma unroll
+            for (int rr = 0; rr < HR / 2; ++rr) {
+              TC* p = slab_at(j, rr);
+              const float v = alpha * acc[i][j][half * (HR / 2) + rr] + bv[j];
+              *p = tg_from_float<TC>(v + beta * tg_to_float(*p));
+            }
+        } else {
+#pragma unroll
+          for (int j = 0; j < SN; ++j)
+#pragma unroll
+            for (int rr = 0; rr < HR / 2; ++rr)
+              *slab_at(j, rr) =
+                  tg_from_float<TC>(alpha * acc[i][j][half * (HR / 2) + rr] + bv[j]);
+        }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's slab is written
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -815,7 +844,7 @@ __device__ __forceinline__ void v3_tile(
               }
               tg_store16(pc, o);
             }
-          } else if (beta != 0.f) {
+          } else if (!CADD && beta != 0.f) {
             tg_vec16<TC> o, c = c_load16(pc);
             *reinterpret_cast<uint4*>(&o) = v;
 #pragma unroll

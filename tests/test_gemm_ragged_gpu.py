@@ -144,3 +144,23 @@ def test_gemm_rows_of_c_at_any_element(cuda, M, N, K, off, odt, dt):
         d = torch.full((M, N), 2.0, device="cuda", dtype=odt)
         L().matmul2d(a, b.t().contiguous(), d, beta=beta)
         assert torch.equal(d.float(), want + 2 * beta)
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (300, 257, 72), (512, 1024, 128),
+                                   (1030, 515, 264), (4096, 4096, 64)])
+def test_gemm_16bit_accumulation_rounds_once(cuda, M, N, K, dt):
+    """C += A B in 16 bits adds in fp32 and rounds the sum, in full and in edge tiles of each
+    block shape: rounding the product first would leave up to another half unit in the last
+    place, of the product, where C cancels it."""
+    dt = DT[dt]
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = _mk(g, M, K, dt).contiguous(), _mk(g, N, K, dt).contiguous()
+    ab = a.double() @ b.double().t()
+    c0 = (-ab + 0.25 * torch.randn(M, N, generator=g, device="cuda")).to(dt)
+    c = c0.clone()
+    L().gemm(a, b, c, False, True, 1.0, 1.0, M, N, K, K, K, N)
+    want = ab + c0.double()
+    tol = (K // 16 + 40) * 2.0 ** -23 * (a.double().abs() @ b.double().abs().t() + c0.double().abs())
+    err = (c.double() - want).abs()
+    assert bool((err <= tol + 1.01 * EPS[dt] * want.abs()).all()), float(err.max())
