@@ -33,6 +33,7 @@
 #include "tg_common.h"
 
 #include <initializer_list>
+#include <type_traits>
 
 namespace {
 
@@ -1439,9 +1440,9 @@ int bwd_gen_t(const void* q, const void* k, const void* v, const void* o, const 
 // an fp32 operand is split exactly into three bf16 terms h + m + l (each the bf16 rounding
 // of what is left), and so are P and dS; of the nine term products the six of weight >=
 // 2^-16 are formed (as in tg_gemm_rs.hip).  fp16 / bf16 data multiply S = Q K^T and
-// dP = dO V^T as they are; in the products with P or dS, those are two bf16 terms (16
-// bits, far below the rounding of the 16-bit results) against bf16 data as it is or fp16
-// data as two exact bf16 terms.
+// dP = dO V^T as they are; in the products with P or dS, those are three bf16 terms, too,
+// against bf16 data as it is or fp16 data as two exact bf16 terms; P, whose range is known,
+// against fp16 data is two fp16 terms (22 bits) instead.
 // What bounded the generic kernels was the fp32 matrix cores' rate (1/16 of the 16-bit
 // one) and element-wise staging.  Per 32 x 32 sub-tile at d = 64 the fp32 forward takes 48
 // bf16 MFMAs instead of 64 fp32 ones of twice the time, the backward 168 instead of 224.
@@ -1461,19 +1462,19 @@ typedef __bf16 bfv2 __attribute__((ext_vector_type(2)));
 typedef unsigned short usv2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_e __attribute__((ext_vector_type(4), aligned(4)));  // any dword
 
-// ROWP: planes of a row operand (S, dP); TRP: planes of a transposed operand (with P or
-// dS); SAME: the same planes; PT: terms of P and dS.
+// ROWP: planes of a row operand (S, dP); TRP: planes of a transposed operand (with dS, and
+// with P where that is FxP); SAME: the same planes.
 template <typename T> struct Fx;
 template <> struct Fx<float> {
-  static constexpr int ROWP = 3, TRP = 3, PT = 3, BN = 32;
+  static constexpr int ROWP = 3, TRP = 3, BN = 32;
   static constexpr bool SAME = true;
 };
 template <> struct Fx<tg_bf16> {
-  static constexpr int ROWP = 1, TRP = 1, PT = 2, BN = 64;
+  static constexpr int ROWP = 1, TRP = 1, BN = 64;
   static constexpr bool SAME = true;
 };
 template <> struct Fx<tg_half> {
-  static constexpr int ROWP = 1, TRP = 2, PT = 2, BN = 64;
+  static constexpr int ROWP = 1, TRP = 2, BN = 64;
   static constexpr bool SAME = false;
 };
 // Row fragments: fp32 data as bf16 terms, 16-bit data as it is.
@@ -1633,12 +1634,14 @@ template <typename T> struct FxRaw {
   }
 };
 
+// What a staged operand is multiplied with as a transposed operand.
+enum { FX_NONE = 0, FX_P, FX_DS };
 // A staged operand: BN rows x DP, ROW and/or TR planes.
-template <typename T, int DP, bool ROW, bool TR>
+template <typename T, int DP, bool ROW, int TR>
 struct FxOp {
   static constexpr int BN = Fx<T>::BN, CH = DP / 8, RSB = (CH | 1) * 16;
   static constexpr int PB = BN * RSB;  // bytes of a plane
-  static constexpr bool SEP = TR && !Fx<T>::SAME;                   // own TR planes
+  static constexpr bool SEP = TR == FX_DS && !Fx<T>::SAME;          // own TR planes
   static constexpr bool RP = ROW || !SEP;                           // row planes are stored
   static constexpr int TR0 = SEP ? (ROW ? Fx<T>::ROWP : 0) : 0;     // first TR plane
   static constexpr int NPL = (RP ? Fx<T>::ROWP : 0) + (SEP ? Fx<T>::TRP : 0);
@@ -1743,46 +1746,75 @@ __device__ __forceinline__ f32x16 fx_rows(const char* t, int PB, const FxOwn<T, 
   return c;
 }
 
-// The 16 values of a lane's C-tile column as PT bf16 terms, two 8-element k-steps each.
-template <int PT> struct FxP {
-  bfv8 t[PT][2];
-  __device__ __forceinline__ void split(const float (&v)[16]) {
+// The 16 values of a lane's C-tile column as three bf16 terms, two 8-element k-steps each.
+// (With two terms of P and dS, 16 bits, o and dV of fp16 data were 1.5e-4 of their error
+// further from float64 than with fp32 P, and those of bf16 data 2e-6 of it; so, no further.)
+struct FxP {
+  typedef bfv8 frag;
+  static constexpr int NT = 3;
+  frag t[NT][2];
+  __device__ __forceinline__ void split(const float (&v)[16], float = 1.f) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      uint4 q[PT];
+      uint4 q[NT];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        unsigned x[PT];
-        split2<PT>(v[8 * s + 2 * e], v[8 * s + 2 * e + 1], x);
+        unsigned x[NT];
+        split2<NT>(v[8 * s + 2 * e], v[8 * s + 2 * e + 1], x);
 #pragma unroll
-        for (int i = 0; i < PT; ++i) reinterpret_cast<unsigned*>(&q[i])[e] = x[i];
+        for (int i = 0; i < NT; ++i) reinterpret_cast<unsigned*>(&q[i])[e] = x[i];
       }
 #pragma unroll
-      for (int i = 0; i < PT; ++i) t[i][s] = __builtin_bit_cast(bfv8, q[i]);
+      for (int i = 0; i < NT; ++i) t[i][s] = __builtin_bit_cast(frag, q[i]);
     }
   }
 };
+// P against fp16 data: times `by` as two fp16 terms (two products instead of five).  P of
+// 2^-8 and more keeps 22 bits then, any smaller one 2^-31 (forward: P up to 2^8, by 2^7; dV:
+// P up to 1, by 2^14).
+struct FxPHalf {
+  typedef Vec8<tg_half>::type frag;
+  static constexpr int NT = 2;
+  frag t[NT][2];
+  __device__ __forceinline__ void split(const float (&v)[16], float by) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = v[8 * s + e] * by;
+        const _Float16 hi = (_Float16)x;
+        t[0][s][e] = hi;
+        t[1][s][e] = (_Float16)(x - (float)hi);
+      }
+  }
+};
+template <typename T> struct FxProb { typedef FxP type; };
+template <> struct FxProb<tg_half> { typedef FxPHalf type; };
+// The factors of P (fp16 data) in the forward and in dV.
+template <typename T> constexpr float fx_pf() { return std::is_same<T, tg_half>::value ? 0x1p7f : 1.f; }
+template <typename T> constexpr float fx_pb() { return std::is_same<T, tg_half>::value ? 0x1p14f : 1.f; }
 
 // acc[dt] += products of P (32 staged rows of this sub-tile on the k axis) with the
 // staged operand's columns dt*32 .. +31; TRA: the staged operand is the A operand (the
 // result has the head dim on its rows), else P is.
-template <typename T, int DP, bool TRA>
+template <typename T, int DP, bool TRA, typename P>
 __device__ __forceinline__ void fx_acc(f32x16 (&acc)[DP / 32], const char* t, int PB,
-                                       const FxP<Fx<T>::PT>& p, int lane) {
-  constexpr int RSB = (DP / 8 | 1) * 16, NP = Fx<T>::TRP;
+                                       const P& p, int lane) {
+  constexpr int RSB = (DP / 8 | 1) * 16, NP = P::NT == 3 ? Fx<T>::TRP : 1;
+  typedef typename P::frag frag;
   const int h = lane >> 5, s = lane & 15, nh = (lane >> 4) & 1;
   const char* b0 = t + (4 * h + (s >> 2)) * RSB + (16 * nh + 4 * (s & 3)) * 2;
 #pragma unroll
   for (int sg = 0; sg < 2; ++sg)
 #pragma unroll
     for (int dt = 0; dt < DP / 32; ++dt) {
-      bfv8 x[NP];
+      frag x[NP];
 #pragma unroll
       for (int i = 0; i < NP; ++i) {
         const char* b = b0 + i * PB + sg * 16 * RSB + dt * 64;
         union {
           v4i16 q[2];
-          bfv8 v;
+          frag v;
         } u;
         u.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TG_LDS v4i16*)b);
         u.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TG_LDS v4i16*)(b + 8 * RSB));
@@ -1793,12 +1825,12 @@ __device__ __forceinline__ void fx_acc(f32x16 (&acc)[DP / 32], const char* t, in
       };
       mul(0, 0);
       mul(0, 1);
-      if constexpr (NP >= 2) mul(1, 0);
-      if constexpr (NP == 3) {
+      if constexpr (NP >= 2) {
+        mul(1, 0);
         mul(1, 1);
-        mul(0, 2);
-        mul(2, 0);
       }
+      if constexpr (P::NT == 3) mul(0, 2);
+      if constexpr (NP == 3) mul(2, 0);
     }
 }
 
@@ -1807,8 +1839,8 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
     const T* __restrict__ Q0, const T* __restrict__ K0, const T* __restrict__ V0,
     T* __restrict__ O0, float* __restrict__ LSE0, int64_t Sq, int64_t Sk, int D, float scale,
     int causal, int vec, FaLay lay) {
-  using OK = FxOp<T, DP, true, false>;
-  using OV = FxOp<T, DP, false, true>;
+  using OK = FxOp<T, DP, true, FX_NONE>;
+  using OV = FxOp<T, DP, false, FX_P>;
   constexpr int BN = Fx<T>::BN, RSB = OK::RSB, NDB = DP / 32;
   constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = gen_lds<DP>();
   __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
@@ -1897,8 +1929,8 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
           ps += p[r];
         }
         l += xhalf_sum(ps);
-        FxP<Fx<T>::PT> pt;
-        pt.split(p);
+        typename FxProb<T>::type pt;
+        pt.split(p, fx_pf<T>());
         fx_acc<T, DP, true>(acc, vs + OV::TR0 * OV::PB + kt * 32 * RSB, OV::PB, pt, lane);
       }
     }
@@ -1913,7 +1945,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_fwd_split(
     return;
   }
   if (q < Sq) {
-    const float inv = l > 0.f ? 1.f / l / fx_by<T>() : 0.f;
+    const float inv = l > 0.f ? 1.f / l / (fx_by<T>() * fx_pf<T>()) : 0.f;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -1968,8 +2000,8 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
     const T* __restrict__ O0, const T* __restrict__ dO0, const float* __restrict__ LSE0,
     float* __restrict__ Dv0, T* __restrict__ dQ0, int64_t Sq, int64_t Sk, int D, float scale,
     int causal, int accumulate, int vec, FaLay lay) {
-  using OK = FxOp<T, DP, true, true>;
-  using OV = FxOp<T, DP, true, false>;
+  using OK = FxOp<T, DP, true, FX_DS>;
+  using OV = FxOp<T, DP, true, FX_NONE>;
   constexpr int BN = Fx<T>::BN, RSB = OK::RSB, NDB = DP / 32;
   constexpr int BYTES = OK::BYTES + OV::BYTES, GEN = gen_lds<DP>();
   __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
@@ -2055,7 +2087,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dq_split(
           const float p = 8 * (r >> 2) + (r & 3) > thr ? 0.f : fexp2(fmaf(s[r], sg * sl2, -lq));
           ds[r] = p * (sg * dp[r] - dsum) * sds;
         }
-        FxP<Fx<T>::PT> pt;
+        FxP pt;
         pt.split(ds);
         fx_acc<T, DP, false>(acc, ks + OK::TR0 * OK::PB + kt * 32 * RSB, OK::PB, pt, lane);
       }
@@ -2081,9 +2113,10 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     const T* __restrict__ dO0, const float* __restrict__ LSE0, const float* __restrict__ Dv0,
     T* __restrict__ dK0, T* __restrict__ dV0, int64_t Sq, int64_t Sk, int D, float scale,
     int causal, int accumulate, int vec, FaLay lay) {
-  using OQ = FxOp<T, DP, true, true>;
+  using OQ = FxOp<T, DP, true, FX_DS>;
+  using OD = FxOp<T, DP, true, FX_P>;
   constexpr int BN = Fx<T>::BN, RSB = OQ::RSB, NDB = DP / 32;
-  constexpr int BYTES = 2 * OQ::BYTES, GEN = gen_lds<DP>();
+  constexpr int BYTES = OQ::BYTES + OD::BYTES, GEN = gen_lds<DP>();
   __shared__ __attribute__((aligned(16))) char sm[BYTES > GEN ? BYTES : GEN];
   __shared__ __attribute__((aligned(16))) float ls[BN], dsm[BN];
   char *qs = sm, *dos = sm + OQ::BYTES;
@@ -2114,7 +2147,8 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.f;
   f32x16 sk[TWO ? NDB : 1] = {}, sv[TWO ? NDB : 1] = {};
   const int64_t qstart = causal ? kblk : 0;
-  OQ oq, od;
+  OQ oq;
+  OD od;
   float lv = 0.f, dd = 0.f;
   auto rows = [&](int64_t q0) {
     const int64_t qq = q0 + (threadIdx.x % BN), qc = qq < Sq ? qq : Sq - 1;
@@ -2149,7 +2183,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
         if (qb0 >= Sq) break;
         if (causal && qb0 + 31 < kw) continue;  // wholly before this wave's keys
         const f32x16 s = fx_rows<T, DP>(qs + t * 32 * RSB, OQ::PB, kf, l32, h);
-        const f32x16 dp = fx_rows<T, DP>(dos + t * 32 * RSB, OQ::PB, vf, l32, h);
+        const f32x16 dp = fx_rows<T, DP>(dos + t * 32 * RSB, OD::PB, vf, l32, h);
         const bool diag = causal && kw + 31 > qb0;
         const int mb = diag ? (int)(key - qb0) - 4 * h : -1;  // rows below it are masked
         float p[16], ds[16];
@@ -2165,11 +2199,12 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
             ds[r] = p[r] * (sg * dp[r] - db[i]) * sds;
           }
         }
-        FxP<Fx<T>::PT> pt;
-        pt.split(p);
-        fx_acc<T, DP, false>(dv, dos + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
-        pt.split(ds);
-        fx_acc<T, DP, false>(dk, qs + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, pt, lane);
+        typename FxProb<T>::type pt;
+        pt.split(p, fx_pb<T>());
+        fx_acc<T, DP, false>(dv, dos + OD::TR0 * OD::PB + t * 32 * RSB, OD::PB, pt, lane);
+        FxP dt;
+        dt.split(ds);
+        fx_acc<T, DP, false>(dk, qs + OQ::TR0 * OQ::PB + t * 32 * RSB, OQ::PB, dt, lane);
       }
     }
     fx_turn<T, TWO>(dk, sk);
@@ -2189,7 +2224,7 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
     return;
   }
   fx_store<T, DP>(dK, rs, kw, Sk, D, dk, fx_un<T>(), accumulate, l32, h);
-  fx_store<T, DP>(dV, rs, kw, Sk, D, dv, 1.f / fx_by<T>(), accumulate, l32, h);
+  fx_store<T, DP>(dV, rs, kw, Sk, D, dv, 1.f / (fx_by<T>() * fx_pb<T>()), accumulate, l32, h);
 }
 
 template <typename T, int DP> struct FxOcc {

@@ -203,3 +203,27 @@ def test_split_attention_non_finite(cuda, D, dt, where, value):
         ok = torch.isfinite(w)
         if bool(ok.any()):
             _close(t[ok], w[ok], dt, n, 2.0)
+
+
+@pytest.mark.parametrize("dt", ["fp16", "bf16"])
+@pytest.mark.parametrize("D", [32, 80, 96, 100])
+@pytest.mark.parametrize("S,causal", [(200, False), (1024, True), (3001, False)])
+def test_split_attention_16bit_keeps_fp32_probabilities(cuda, D, S, causal, dt):
+    """o and dV (formed with P) are the rounded float64 results but for a small share: an error
+    of e moves an element's rounding to 11 bits (8 bits) with probability e / 2^-11 (2^-8) or
+    so.  Here e is 2^-21 of the scores and exponentials in fp32, and 2^-25 for each of the S / 16
+    steps of the sum, adding up at random; held to six times that.  P in 16 bits moves 2 %
+    (0.2 to 0.3 %)."""
+    dt = DT[dt]
+    g = torch.Generator(device="cuda").manual_seed(D + S)
+    q, k, v, do = (torch.randn(2, 4, S, D, generator=g, device="cuda").to(dt) for _ in range(4))
+    sc = D ** -0.5
+    o, lse = L().flash_attn_fwd(q, k, v, sc, causal)
+    grads = [torch.empty_like(q) for _ in range(3)]
+    L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, causal, False)
+    want = _ref(q, k, v, do, sc, causal)
+    most = 6 * (2.0 ** -21 + 2.0 ** -25 * (S / 16) ** 0.5) * 2.0 ** (
+        11 if dt == torch.float16 else 8)
+    for t, w, n in ((o, want[0], "o"), (grads[2], want[3], "dv")):
+        share = float((t != w.to(dt)).double().mean())
+        assert share < most, f"{n}: {share:.2e}"
