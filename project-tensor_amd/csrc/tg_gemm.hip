@@ -397,11 +397,12 @@ struct V3Dma {
       off[k] = (uint32_t)(e * (int64_t)sizeof(T));
     }
   }
-  // Copy the tile whose origin is soff bytes past base (both uniform): a raw buffer
-  // load into LDS takes the lane offset in a VGPR and the tile offset in an SGPR, so
-  // the copy costs no vector ALU work.  The resource spans [base, base + 2 GiB) (word
-  // 3: 32-bit untyped access, no swizzle; the gfx9 raw-buffer format).
-  __device__ __forceinline__ void copy(const T* base, uint32_t soff, char* lds) const {
+  // Copy the tile whose origin is `base` (uniform): a raw buffer load into LDS takes the
+  // lane offset in a VGPR and the origin in the resource's SGPRs, so the copy costs no
+  // vector ALU work, and only one tile has to lie within the 2 GiB from its origin that
+  // lane offsets reach (word 3: 32-bit untyped access, no swizzle; the gfx9 raw-buffer
+  // format).
+  __device__ __forceinline__ void copy(const T* base, char* lds) const {
     // The buffer-resource type is compiled in the device pass only: the host pass of
     // this compiler drops the launch stubs of kernel instantiations whose bodies hold it.
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -411,13 +412,12 @@ struct V3Dma {
 #pragma unroll
     for (int k = 0; k < NPW; ++k)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TG_LDS_G void*)(lds + (wave + k * NW) * 1024),
-                                               16, off[k], soff, 0, 0);
+                                               16, off[k], 0, 0, 0);
 #endif
   }
   // Copy of the last, partial tile: lanes whose k is not among the kleft left write zeros
   // themselves.
-  __device__ __forceinline__ void copy_tail(const T* base, uint32_t soff, char* lds,
-                                            int64_t kleft) const {
+  __device__ __forceinline__ void copy_tail(const T* base, char* lds, int64_t kleft) const {
 #if defined(__HIP_DEVICE_COMPILE__)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -428,20 +428,20 @@ struct V3Dma {
       const int r = u / CH, c = (u % CH) ^ v3_key<CH>(r);
       char* dst = lds + (wave + k * NW) * 1024;
       if ((KROWS ? r : c * 8) < kleft)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TG_LDS_G void*)dst, 16, off[k], soff, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TG_LDS_G void*)dst, 16, off[k], 0, 0, 0);
       else
         *reinterpret_cast<uint4*>(dst + lane * 16) = make_uint4(0, 0, 0, 0);
     }
 #endif
   }
   // Instruction k of copy() alone, so a caller can spread a tile's copy over its MFMAs.
-  __device__ __forceinline__ void copy1(const T* base, uint32_t soff, char* lds, int k) const {
+  __device__ __forceinline__ void copy1(const T* base, char* lds, int k) const {
 #if defined(__HIP_DEVICE_COMPILE__)
     const int wave = threadIdx.x >> 6;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T*>(base), (short)0, 0x7fffffff, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TG_LDS_G void*)(lds + (wave + k * NW) * 1024),
-                                             16, off[k], soff, 0, 0);
+                                             16, off[k], 0, 0, 0);
 #endif
   }
 };
@@ -607,18 +607,26 @@ __device__ __forceinline__ void v3_tile(
   db.init(ldb, n0, BKC ? N : (N + 7) / 8 * 8);
   const T* a_org = A + (AKC ? m0 * lda : m0);
   const T* b_org = B + (BKC ? n0 * ldb : n0);
-  auto dma = [&](int64_t k0, char* as, char* bs) {
-    da.copy(a_org, (uint32_t)((AKC ? k0 : k0 * lda) * (int64_t)sizeof(T)), as);
-    db.copy(b_org, (uint32_t)((BKC ? k0 : k0 * ldb) * (int64_t)sizeof(T)), bs);
+  // (tiles are copied in order: the origins of the next one; a product with k0 for each tile
+  // costs 1.3 % of 8192x1024x4096)
+  const int64_t a_step = AKC ? V3_BK : V3_BK * lda, b_step = BKC ? V3_BK : V3_BK * ldb;
+  auto next = [&] {
+    a_org += a_step;
+    b_org += b_step;
+  };
+  auto dma = [&](char* as, char* bs) {
+    da.copy(a_org, as);
+    db.copy(b_org, bs);
+    next();
   };
   // The next tile's copy, instruction q of ANPW + BNPW (A's first), issued between the
   // MFMAs of the current tile by the pipelined path below (has_next false: nothing).
   constexpr int ANPW = decltype(da)::NPW, BNPW = decltype(db)::NPW;
-  auto dma1 = [&](int64_t k0, char* as, char* bs, int q) {
-    if (q < ANPW) da.copy1(a_org, (uint32_t)((AKC ? k0 : k0 * lda) * (int64_t)sizeof(T)), as, q);
-    else db.copy1(b_org, (uint32_t)((BKC ? k0 : k0 * ldb) * (int64_t)sizeof(T)), bs, q - ANPW);
+  auto dma1 = [&](char* as, char* bs, int q) {
+    if (q < ANPW) da.copy1(a_org, as, q);
+    else db.copy1(b_org, bs, q - ANPW);
   };
-  auto mul = [&](const char* as, const char* bs, bool has_next, int64_t kn, char* an, char* bn) {
+  auto mul = [&](const char* as, const char* bs, bool has_next, char* an, char* bn) {
     if constexpr (OCC == 1) {
       // One wave per SIMD: software pipeline.  The fragment reads of k-step ks+1 are
       // issued between the MFMAs of k-step ks (sched_barrier keeps the order), so only
@@ -655,7 +663,7 @@ __device__ __forceinline__ void v3_tile(
               ++nr;
             }
             const int mf = (ks * SM + i) * SN + j;
-            if (has_next && mf % QSTEP == QSTEP - 1 && mf / QSTEP < NQ) dma1(kn, an, bn, mf / QSTEP);
+            if (has_next && mf % QSTEP == QSTEP - 1 && mf / QSTEP < NQ) dma1(an, bn, mf / QSTEP);
             __builtin_amdgcn_sched_barrier(0);
           }
         if (ks + 1 < V3_BK / 16)
@@ -663,8 +671,9 @@ __device__ __forceinline__ void v3_tile(
           for (; nr < SM + SN; ++nr) rd(cur ^ 1, ks + 1, nr);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if (has_next) next();
     } else {
-      if (has_next) dma(kn, an, bn);
+      if (has_next) dma(an, bn);
 #pragma unroll
       for (int ks = 0; ks < V3_BK / 16; ++ks) {
         typename Vec8<T>::type af[SM], bf[SN];
@@ -687,18 +696,18 @@ __device__ __forceinline__ void v3_tile(
   const int64_t kf = TAIL ? K & ~(int64_t)(V3_BK - 1) : K;
   auto dma_tail = [&](char* as, char* bs) {
     if (!TAIL || kf == K) return;
-    da.copy_tail(a_org, (uint32_t)((AKC ? kf : kf * lda) * (int64_t)sizeof(T)), as, K - kf);
-    db.copy_tail(b_org, (uint32_t)((BKC ? kf : kf * ldb) * (int64_t)sizeof(T)), bs, K - kf);
+    da.copy_tail(a_org, as, K - kf);
+    db.copy_tail(b_org, bs, K - kf);
   };
   bool odd = false;  // the partial tile is in a1, b1
-  if (kf > 0) dma(0, a0, b0);
+  if (kf > 0) dma(a0, b0);
   else dma_tail(a0, b0);
   for (int64_t k0 = 0; k0 < kf; k0 += 2 * V3_BK) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     const bool more1 = k0 + V3_BK < kf;
     if (!more1) dma_tail(a1, b1);
-    mul(a0, b0, more1, k0 + V3_BK, a1, b1);
+    mul(a0, b0, more1, a1, b1);
     if (!more1) {
       odd = true;
       break;
@@ -707,14 +716,14 @@ __device__ __forceinline__ void v3_tile(
     __syncthreads();
     const bool more2 = k0 + 2 * V3_BK < kf;
     if (!more2) dma_tail(a0, b0);
-    mul(a1, b1, more2, k0 + 2 * V3_BK, a0, b0);
+    mul(a1, b1, more2, a0, b0);
     if (!more2) break;
   }
   if constexpr (TAIL) {
     if (kf < K) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      mul(odd ? a1 : a0, odd ? b1 : b0, false, 0, a0, b0);
+      mul(odd ? a1 : a0, odd ? b1 : b0, false, a0, b0);
     }
   }
   if constexpr (BSUM) {
@@ -958,10 +967,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void k_gemm_v3g(
       g.db[bz], dbt, (g.dbacc >> bz) & 1u, nullptr, 0, loc / gx, loc % gx);
 }
 
-// Block shapes of the DMA-staged kernel (waves of 64 x 64 of C): 4 x 2 waves
-// (256 x 128, one block per CU, two waves per SIMD) when the problem has at least
-// one such tile per CU, else 2 x 2 waves (128 x 128, two blocks per CU).
-
 // Whether a 16-bit GEMM runs on the DMA-staged kernel (k_gemm_v3).
 // padded: rows are padded to whole 8-element chunks, readable and zero behind their end.
 bool v3_ok(int elem, int ta, int tb, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
@@ -969,11 +974,12 @@ bool v3_ok(int elem, int ta, int tb, int64_t M, int64_t N, int64_t K, const void
   const int VE = 16 / elem;
   const bool vec = tg_aligned16(A) && tg_aligned16(B) && lda % VE == 0 && ldb % VE == 0 &&
                    sa % VE == 0 && sb % VE == 0;
-  // The DMA addresses each operand through a 2 GiB buffer window that starts at the
-  // block's origin: a k-contiguous operand (A, or B given as [N, K]) spans at most 256
-  // of its rows plus K elements from there, an m/n-contiguous one all K of its rows.
-  const int64_t a_span = (ta ? K * lda : 256 * lda + K) * (int64_t)elem;
-  const int64_t b_span = (tb ? 256 * ldb + K : K * ldb) * (int64_t)elem;
+  // The DMA reaches 2 GiB from a tile's origin: 256 rows of a k-contiguous operand (A, or B
+  // given as [N, K]), 64 of an m/n-contiguous one.  Rows of 2^22 (2^24) elements are left to
+  // the generic kernel.  (The weight gradient of 32768 tokens and 50304 words, whose dY is
+  // 3.3 GB: 24.5 ms there, 4.9 here.)
+  const int64_t a_span = (ta ? 64 * lda + 256 : 256 * lda + V3_BK) * (int64_t)elem;
+  const int64_t b_span = (tb ? 256 * ldb + V3_BK : 64 * ldb + 256) * (int64_t)elem;
   // Whole 8-element chunks along each contiguous dimension: K of a k-contiguous operand,
   // M of a transposed A, N of a plain B.
   const bool chunks = padded || ((ta || K % 8 == 0) && (!tb || K % 8 == 0) && (!ta || M % 8 == 0) &&

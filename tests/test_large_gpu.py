@@ -195,6 +195,46 @@ def test_axpby_paths_round_alike(cuda, dx_, dy_, beta):
     assert torch.equal(part, want[k:])
 
 
+@pytest.mark.parametrize("N", [33_000, 33_001])
+def test_gemm_column_major_operand_past_2gib(cuda, free_after, N):
+    """dW = X^T dY with a dY of 32800 x N fp16 (2.17 GB; odd N: copied with aligned rows, past
+    2 GiB, too): column windows against float64, and bit for bit against the same columns as
+    a small call; and at the rate of a dY below 2 GiB."""
+    K, M = 32_800, 256
+    gen = torch.Generator(device="cuda").manual_seed(29)
+    x = torch.randn(K, M, dtype=torch.float16, device="cuda", generator=gen)
+    g = torch.randn(K, N, dtype=torch.float16, device="cuda", generator=gen) * 0.05
+    dw = L().matmul2d(x, g, trans_a=True, out_dtype=torch.float32)
+    w, xd = 64, x.double()
+    for c in [0, N // 2 - 5, N - w]:
+        part = g[:, c:c + w].contiguous()
+        want = xd.t() @ part.double()
+        mag = xd.abs().t() @ part.double().abs()
+        err = (dw[:, c:c + w].double() - want).abs()
+        assert bool((err <= (K // 16 + 40) * 2.0 ** -23 * mag).all()), f"columns {c}"
+    if N % 8 == 0:  # (without K splits, whose number depends on the sizes)
+        whole = torch.empty(M, N, device="cuda")
+        L().gemm(x, g, whole, True, False, 1.0, 0.0, M, N, K, M, N, N)
+        for c in [0, N - w]:
+            part, small = g[:, c:c + w].contiguous(), torch.empty(M, w, device="cuda")
+            L().gemm(x, part, small, True, False, 1.0, 0.0, M, w, K, M, w, w)
+            assert torch.equal(small, whole[:, c:c + w]), f"columns {c}"
+
+    def us(gg):
+        best = 1e30
+        for _ in range(5):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            L().matmul2d(x[:gg.shape[0]], gg, trans_a=True, out_dtype=torch.float32)
+            t1.record()
+            t1.synchronize()
+            best = min(best, t0.elapsed_time(t1) * 1e3)
+        return best
+    past, below = us(g), us(g[:32_000])  # 2.11e9 bytes
+    print(f"[{K}x{M}]^T x [{K}x{N}]: {past:.0f} us, {below:.0f} with 32000 rows", flush=True)
+    assert past < 1.5 * below, (past, below)
+
+
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_gemm_row_major_operand_past_2gib(cuda, free_after, trans_b):
     """An fp16 A of 1,050,000 x 1024 (2.15 GB, past the 2 GiB a buffer window covers)
