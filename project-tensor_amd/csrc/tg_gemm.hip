@@ -1378,6 +1378,13 @@ struct PackPlan {
   int64_t ra, ca, rb, cb;  // stored rows and columns
   size_t a, b;
 };
+// Whether the copies of such a plan bring the product to the DMA-staged kernel: not where
+// the other operand stays misaligned, or rows are too long.
+bool pack_serves(const PackPlan& p, int ta, int tb, int64_t M, int64_t N, int64_t K,
+                 const void* A, int64_t lda, const void* B, int64_t ldb) {
+  return v3_ok(2, ta, tb, M, N, K, p.a ? nullptr : A, p.a ? (p.ca + 7) / 8 * 8 : lda, 0,
+               p.b ? nullptr : B, p.b ? (p.cb + 7) / 8 * 8 : ldb, 0, true);
+}
 PackPlan pack_plan(int dtype_ab, int ta, int tb, int64_t M, int64_t N, int64_t K) {
   PackPlan p{ta ? K : M, ta ? M : K, tb ? N : K, tb ? K : N, 0, 0};
   const double mnk = (double)M * (double)N * (double)K;
@@ -1390,6 +1397,7 @@ PackPlan pack_plan(int dtype_ab, int ta, int tb, int64_t M, int64_t N, int64_t K
     return p;
   if (p.ca % 8) p.a = al256((size_t)(p.ra * ((p.ca + 7) / 8)) * 16);
   if (p.cb % 8) p.b = al256((size_t)(p.rb * ((p.cb + 7) / 8)) * 16);
+  if (!pack_serves(p, ta, tb, M, N, K, nullptr, p.ca, nullptr, p.cb)) p.a = p.b = 0;
   return p;
 }
 
@@ -1467,8 +1475,8 @@ TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int
                         void* workspace, size_t workspace_bytes, void* stream) {
   const char* who = "tg_matmul";
   const SplitPlan p = M > 0 && N > 0 && K > 0 ? split_plan(dtype_ab, M, N, K) : SplitPlan{};
-  const PackPlan pk = M > 0 && N > 0 && K > 0 ? pack_plan(dtype_ab, trans_a, trans_b, M, N, K)
-                                              : PackPlan{};
+  PackPlan pk = M > 0 && N > 0 && K > 0 ? pack_plan(dtype_ab, trans_a, trans_b, M, N, K)
+                                        : PackPlan{};
   const size_t need = p.bytes + pk.a + pk.b;
   if (need == 0 || workspace_bytes < need)
     return gemm_dispatch(who, dtype_ab, dtype_c, trans_a, trans_b, M, N, K, alpha, A, lda, 0, B,
@@ -1481,6 +1489,7 @@ TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int
              "%s: unsupported dtype combination ab=%d c=%d", who, dtype_ab, dtype_c);
   hipStream_t s = tg_stream(stream);
   char* ws = static_cast<char*>(workspace);
+  if (!pack_serves(pk, trans_a, trans_b, M, N, K, A, lda, B, ldb)) pk.a = pk.b = 0;
   const bool padded = pk.a || pk.b;
   int rc = pack_operands(pk, A, lda, B, ldb, ws + p.bytes, s);
   if (rc != TG_OK) return rc;
@@ -1541,6 +1550,7 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
   hipStream_t s = tg_stream(stream);
   const int64_t S = p.sp.S, kc = p.sp.kc, sc = split_stride(M * N);
   const void* G0 = G;
+  if (!pack_serves(p.pk, 1, 0, M, N, K, X, ldx, G, ldg)) p.pk.a = p.pk.b = 0;
   const bool padded = p.pk.a || p.pk.b;
   int rc = TG_OK;
   if (K > 0)

@@ -164,3 +164,34 @@ def test_gemm_16bit_accumulation_rounds_once(cuda, M, N, K, dt):
     tol = (K // 16 + 40) * 2.0 ** -23 * (a.double().abs() @ b.double().abs().t() + c0.double().abs())
     err = (c.double() - want).abs()
     assert bool((err <= tol + 1.01 * EPS[dt] * want.abs()).all()), float(err.max())
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_ragged_copies_only_where_they_serve(cuda, dt):
+    """Odd rows are copied with aligned ones for the DMA-staged kernel only: not where the
+    other operand is misaligned (the workspace stays as it was), and no workspace is asked
+    for where rows are too long for it."""
+    code, f32 = L().dtype_code(torch.empty(0, dtype=dt)), L().dtype_code(torch.empty(0))
+    lib, s = L().load(), L().stream_handle()
+    M, N, K = 520, 1025, 1000
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for off in (0, 1):
+        a, b = _mk(g, M, K, dt, 0, off), _mk(g, K, N, dt)
+        nb = lib.tg_matmul_workspace(code, 0, 0, M, N, K)
+        assert nb == (K * 1032 * 2 + 255) // 256 * 256
+        ws = torch.full((nb,), 0x5a, device="cuda", dtype=torch.uint8)
+        c = torch.empty(M, N, device="cuda")
+        assert lib.tg_matmul(code, f32, 0, 0, M, N, K, 1.0, a.data_ptr(), K, b.data_ptr(), N, None,
+                             0.0, c.data_ptr(), N, ws.data_ptr(), nb, s) == 0
+        _bound(c, a, b, f"off {off}")
+        assert bool((ws == 0x5a).all()) == (off == 1)
+        x, gr = _mk(g, K, M, dt, 0, off), b
+        nb = lib.tg_gemm_wgrad_workspace(code, M, N, K, 0)
+        ws = torch.full((nb,), 0x5a, device="cuda", dtype=torch.uint8)
+        assert lib.tg_gemm_wgrad(code, M, N, K, x.data_ptr(), M, gr.data_ptr(), N, f32,
+                                 c.data_ptr(), N, 0, 0, None, 0, ws.data_ptr(), nb, s) == 0
+        _bound(c, x.t(), gr, f"wgrad off {off}")
+        assert bool((ws == 0x5a).all()) == (off == 1)
+    # k-contiguous rows of 2^23 elements
+    even, odd = (lib.tg_matmul_workspace(code, 0, 1, 64, 64, 2 ** 23 + i) for i in (0, 1))
+    assert even == odd
