@@ -107,9 +107,12 @@ def test_split_attention_fp32_extremes(cuda, D, kind):
     _close(o[ok], want[0][ok], torch.float32, "o", 200.0 if kind == "large_scores" else 2.0)
     grads = [torch.empty_like(q) for _ in range(3)]
     L().flash_attn_bwd(q, k, v, o, do, lse, *grads, sc, False, False)
-    if kind in ("tiny", "negative_scale"):
-        for t, w, n in zip(grads, want[1:], ("dq", "dk", "dv")):
-            _close(t, w, torch.float32, n, 10.0)
+    # (large_scores: scores of up to 10^3 are off by 2^-24 of themselves and more, and P by
+    # as much relative to itself)
+    for t, w, n in zip(grads, want[1:], ("dq", "dk", "dv")):
+        ok = torch.isfinite(w.float())
+        assert torch.equal(torch.isfinite(t), ok), n
+        _close(t[ok], w[ok], torch.float32, n, 200.0 if kind == "large_scores" else 10.0)
 
 
 @pytest.mark.parametrize("D", [24, 64, 128])

@@ -1,6 +1,6 @@
 """16-bit products at ragged sizes and alignments: k past the last tile (masked DMA), any
-M and N, odd leading dimensions (the register-staged kernel), K splits whose last chunk is
-short, and the fused and grouped forms at such sizes, against float64 products of the same
+M and N, odd rows (copied with aligned ones where a workspace holds them, else the
+register-staged kernel), K splits whose last chunk is short, and the fused and grouped forms at such sizes, against float64 products of the same
 16-bit operands."""
 import pytest
 import torch
@@ -93,8 +93,13 @@ def test_wgrad_ragged_tokens(cuda, K, M, N):
     _bound(ws[1], x.t(), gr * 0.5, "wgrad_group")
 
 
-@pytest.mark.parametrize("M,N,K", [(357, 512, 128), (1917, 3232, 808), (61, 136, 72), (257, 264, 1000)])
+@pytest.mark.parametrize("M,N,K", [(357, 512, 128), (1917, 3232, 808), (61, 136, 72),
+                                   (257, 264, 1000), (1917, 3232, 832), (61, 136, 64),
+                                   (257, 264, 1024), (9, 72, 192), (300, 56, 128)])
 def test_epilogue_ragged_equals_separate(cuda, M, N, K):
+    """Fused where K is a multiple of 64 and N one of 8 from 64 on, at any M; refused (False,
+    nothing run) elsewhere."""
+    fused = K % 64 == 0 and N >= 64
     dt = torch.bfloat16
     g = torch.Generator(device="cuda").manual_seed(N)
     a, b = _mk(g, M, K, dt).contiguous(), (_mk(g, K, N, dt).contiguous() * 0.05)
@@ -105,16 +110,19 @@ def test_epilogue_ragged_equals_separate(cuda, M, N, K):
     _bound(ref, torch.cat([a.double(), torch.ones(M, 1, device="cuda").double()], 1),
            torch.cat([b.double(), bias.double()[None]], 0), "bias")
     out, act = torch.empty_like(ref), torch.empty_like(ref)
-    if L().gemm_epilogue("gelu_fwd", a, b, act, out, bias):
+    assert L().gemm_epilogue("gelu_fwd", a, b, act, out, bias) is fused
+    if fused:
         assert torch.equal(out, ref)
         assert torch.equal(act, L().act_fwd("gelu", ref))
     out = torch.empty_like(ref)
-    if L().gemm_epilogue("residual", a, b, r, out, bias):
+    assert L().gemm_epilogue("residual", a, b, r, out, bias) is fused
+    if fused:
         assert torch.equal(out, ref + r)
     # GELU backward: A [M, K] @ W^T with W [N, K]
     w = _mk(g, N, K, dt).contiguous()
     d = torch.empty_like(ref)
-    if L().gemm_epilogue("gelu_bwd", a, w, r, d):
+    assert L().gemm_epilogue("gelu_bwd", a, w, r, d) is fused
+    if fused:
         want = torch.empty_like(ref)
         L().act_bwd("gelu", r, L().matmul2d(a, w, trans_b=True), want, False)
         assert torch.equal(d, want)
