@@ -4,7 +4,9 @@
 //
 // fp32 products.  Every fp32 operand element is split into three bf16 terms,
 //   x = h + m + l,  h = bf16(x), m = bf16(x - h), l = bf16(x - h - m),
-// round-to-nearest each.  24 significand bits fall into 8 + 8 + 8, so the split is exact.
+// round-to-nearest each (Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", ARITH 2019).  24 significand bits
+// fall into 8 + 8 + 8, so the split is exact.
 // Of the nine products of two split operands the six with weight >= 2^-16 are kept,
 //   hh + hm + mh + mm + hl + lh,
 // accumulated in fp32; the three that are dropped (a term is at most 2^-8 of the one before
@@ -398,7 +400,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
 // and B).
 constexpr int kSmallWaves = 16;
 template <bool TA, bool TB>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_gemm_f32_small(
+__global__ __launch_bounds__(64 * kSmallWaves) void k_gemm_rs_small(
     int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha, const float* __restrict__ A,
     int64_t lda, int64_t sa, const float* __restrict__ B, int64_t ldb, int64_t sb, float beta,
     float* __restrict__ C, int64_t ldc, int64_t sc, const float* __restrict__ bias) {
@@ -541,7 +543,7 @@ int tg_gemm_rs(const TgRsPlan& p, int ta, int tb, int64_t M, int64_t N, int64_t 
 #undef TG_RSL
   const dim3 gs((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)batch);
 #define TG_SM(TA_, TB_)                                                                      \
-  k_gemm_f32_small<TA_, TB_><<<gs, 64 * kSmallWaves, 0, s>>>(M, N, kc, ktot, alpha, A, lda, sa, B, \
+  k_gemm_rs_small<TA_, TB_><<<gs, 64 * kSmallWaves, 0, s>>>(M, N, kc, ktot, alpha, A, lda, sa, B, \
                                                              ldb, sb, beta, C, ldc, sc, bias)
   if (!ta && !tb) TG_SM(false, false);
   else if (!ta) TG_SM(false, true);
