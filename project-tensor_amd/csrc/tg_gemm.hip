@@ -1350,24 +1350,29 @@ __global__ __launch_bounds__(kPackBlock) void k_pack_rows(PackArg pa, PackArg pb
   const unsigned short* s = static_cast<const unsigned short*>(p.src) + r * p.ld + c;
   unsigned o[4];
   if (c >= 8 && c + 16 <= p.cols) {
-    const uintptr_t u = reinterpret_cast<uintptr_t>(s);
-    const uint4* v = reinterpret_cast<const uint4*>(u & ~(uintptr_t)15);
+    const unsigned mis = reinterpret_cast<uintptr_t>(s) & 15;
+    const uint4* v = reinterpret_cast<const uint4*>(s - mis / 2);
     const uint4 a = v[0], b = v[1];
-    unsigned x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    const bool two = u & 8, one = u & 4, half = u & 2;
-#pragma unroll
-    for (int e = 0; e < 6; ++e) x[e] = two ? x[e + 2] : x[e];
-#pragma unroll
-    for (int e = 0; e < 5; ++e) x[e] = one ? x[e + 1] : x[e];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = half ? (x[e] >> 16) | (x[e + 1] << 16) : x[e];
+    // (in scalars: an array of the eight words, shifted by selects, went to LDS with its
+    // loads one by one; 12913x192x256, A transposed, 28.5 us with that copy, 17.1 so)
+    const bool two = mis & 8, one = mis & 4, half = mis & 2;
+    const unsigned w0 = two ? a.z : a.x, w1 = two ? a.w : a.y, w2 = two ? b.x : a.z;
+    const unsigned w3 = two ? b.y : a.w, w4 = two ? b.z : b.x, w5 = two ? b.w : b.y;
+    const unsigned x0 = one ? w1 : w0, x1 = one ? w2 : w1, x2 = one ? w3 : w2;
+    const unsigned x3 = one ? w4 : w3, x4 = one ? w5 : w4;
+    o[0] = half ? __builtin_amdgcn_alignbit(x1, x0, 16) : x0;
+    o[1] = half ? __builtin_amdgcn_alignbit(x2, x1, 16) : x1;
+    o[2] = half ? __builtin_amdgcn_alignbit(x3, x2, 16) : x2;
+    o[3] = half ? __builtin_amdgcn_alignbit(x4, x3, 16) : x3;
   } else {
+    // (all loads go out at once, past the row's end of its last element)
     const int64_t n = p.cols - c;
+    unsigned x[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const unsigned lo = 2 * e < n ? s[2 * e] : 0, hi = 2 * e + 1 < n ? s[2 * e + 1] : 0;
-      o[e] = lo | (hi << 16);
-    }
+    for (int e = 0; e < 8; ++e) x[e] = s[e < n ? e : n - 1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = (2 * e < n ? x[2 * e] : 0) | (2 * e + 1 < n ? x[2 * e + 1] << 16 : 0);
   }
   p.dst[q] = make_uint4(o[0], o[1], o[2], o[3]);
 }

@@ -203,3 +203,20 @@ def test_ragged_copies_only_where_they_serve(cuda, dt):
     # k-contiguous rows of 2^23 elements
     even, odd = (lib.tg_matmul_workspace(code, 0, 1, 64, 64, 2 ** 23 + i) for i in (0, 1))
     assert even == odd
+
+
+@pytest.mark.parametrize("cols", [3, 9, 15, 17, 23, 25, 31, 39, 1001])
+def test_ragged_rows_are_copied_exactly(cuda, cols):
+    """Odd rows at every offset from 16 bytes: first, inner and last chunks of a row.  Operands
+    of whole numbers, so each sum is exact; the last column ends the buffer."""
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    M, K = 3000, 200
+    a = torch.randint(-2, 3, (M, K), generator=g, device="cuda").half()
+    for off in range(8):
+        buf = torch.randint(-2, 3, (K * cols + off,), generator=g, device="cuda").half()
+        b = buf[off:].view(K, cols)
+        c = L().matmul2d(a, b, out_dtype=torch.float32)
+        assert torch.equal(c, a.float() @ b.float().clone())
+        w = torch.empty(cols, M, device="cuda")
+        L().wgrad(b, a.t().contiguous(), w, False)
+        assert torch.equal(w, c.t())
