@@ -988,48 +988,67 @@ bool v3_ok(int elem, int ta, int tb, int64_t M, int64_t N, int64_t K, const void
          b_span < (int64_t{1} << 31);
 }
 
-// Block shape and K split of a 16-bit product: the fastest by the times (us) measured per
-// 64-deep k-tile with every CU busy: 256x256 blocks (4x2 waves of 64x128) 1.85,
-// 256x128 (4x2 of 64x64) 1.02, both one block per CU; 128x128 (2x2 of 64x64) 1.08 with
-// two blocks on every CU, 0.9 with two on a few, 0.7 with one; a block's start and store
-// take 4-6.  A K split (chunks of a multiple of 64) adds its finishing launch: 4 us and its
-// traffic at 6 TB/s (whole and in two: 2048x1024x4096 41 and 31 us, 3072x768x3072 33 and 30,
-// 4096x1024x4096 45 and 47, so whole).
+// Times (us) of a 16-bit product by block shape, from those measured per 64-deep k-tile with
+// every CU busy: t[2] 256x256 blocks (4x2 waves of 64x128) 1.85 and 6 for a block's start and
+// store (few k-tiles: 1.15 and 12, the stores of the whole chip at once), t[1] 256x128 (4x2 of
+// 64x64) 1.02 and 5, both one block per CU; t[0] 128x128 (2x2 of 64x64) 1.08 with two blocks on
+// every CU, 0.9 with two on a few, 0.7 with one, and 4.
 // (256x256 as 2x2 waves of 128x128, one wave per SIMD, measured 3-8 % slower: nothing
 // overlaps a wave's LDS waits and barrier.)
-struct V3Plan {
-  int shape;      // 2: 256x256, 1: 256x128, 0: 128x128
-  int64_t S, kc;
-};
-V3Plan v3_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool can_split) {
-  V3Plan best{0, 1, K};
-  if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
-  const double ncu = (double)tg_num_cus();
+void v3_times(double (&t)[4], int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const double ncu = (double)tg_num_cus(), kt = (double)((K + 63) / 64);
   const auto tiles = [&](int64_t bm, int64_t bn) {
     return (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
   };
+  t[2] = std::ceil(tiles(256, 256) / ncu) * std::max(kt * 1.85 + 6.0, kt * 1.15 + 12.0);
+  t[1] = std::ceil(tiles(256, 128) / ncu) * (kt * 1.02 + 5.0);
+  const double b = tiles(128, 128), pairs = std::floor(b / (2 * ncu));
+  const double rest = b - pairs * 2 * ncu;
+  const double tk = rest > ncu ? 0.9 + 0.18 * (rest - ncu) / ncu : 0.7;
+  t[0] = pairs * (kt * 1.08 + 4.0) + (rest > 0 ? kt * tk + 4.0 : 0.0);
+  // t[3] 128x64 (2x2 of 64x32): 0.96 and 2 with three blocks on every CU, 0.65 with two, 0.3 with
+  // one, and 3.7 (by t[0] and so: 512x512x1024 12.0 and 8.4 us, 392x608x376 10.6 and 7.2)
+  const double b3 = tiles(128, 64), full = std::floor(b3 / (3 * ncu)), r3 = b3 / ncu - 3 * full;
+  const double c3 = r3 > 1 ? 0.3 + 0.33 * (r3 - 1) : 0.3;
+  t[3] = full * (kt * 0.96 + 2.1) + (r3 > 0 ? kt * c3 + 3.7 : 0.0);
+}
+
+// The K split of a 16-bit product: batch entry s of S multiplies k in [s*kc, min(K, (s+1)*kc)).
+// The fastest by these times; a split (chunks of a multiple of 64) adds its finishing launch: 4
+// us and its traffic at 6 TB/s (whole and in two: 2048x1024x4096 41 and 31 us, 3072x768x3072 33
+// and 30, 4096x1024x4096 45 and 47, so whole).
+struct V3Plan {
+  int64_t S, kc;
+};
+V3Plan v3_plan(int64_t M, int64_t N, int64_t K) {
+  V3Plan best{1, K};
   double tbest = 1e30;
   // (K below 2048 stays whole, so such a product's rows do not depend on how many there are)
-  for (int64_t S = 1; S <= (can_split && K >= 2048 ? 32 : 1); S *= 2) {
+  for (int64_t S = 1; S <= (K >= 2048 ? 32 : 1); S *= 2) {
     const int64_t kc = S == 1 ? K : ((K + S - 1) / S + 63) / 64 * 64;
     if (S > 1 && (kc < 256 || (K + kc - 1) / kc != S)) continue;
     // (a split's partial sums stay within 256 MiB)
     if (S > 1 && (double)S * (double)M * (double)N * 4.0 > 268435456.0) break;
-    const double kt = (double)((kc + 63) / 64);
     const double fin = S > 1 ? 4.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 6e6 : 0.0;
-    double t[3];
-    t[2] = std::ceil(tiles(256, 256) * S / ncu) * (kt * 1.85 + 6.0);
-    t[1] = std::ceil(tiles(256, 128) * S / ncu) * (kt * 1.02 + 5.0);
-    const double b = tiles(128, 128) * S, pairs = std::floor(b / (2 * ncu));
-    const double rest = b - pairs * 2 * ncu;
-    const double tk = rest > ncu ? 0.9 + 0.18 * (rest - ncu) / ncu : 0.7;
-    t[0] = pairs * (kt * 1.08 + 4.0) + (rest > 0 ? kt * tk + 4.0 : 0.0);
-    for (int i = 2; i >= 0; --i)
-      if (t[i] + fin < tbest) {
-        tbest = t[i] + fin;
-        best = V3Plan{i, S, kc};
-      }
+    double t[4];
+    v3_times(t, M, N, kc, S);
+    const double ts = std::min(std::min(t[0], t[1]), t[2]) + fin;
+    if (ts < tbest) {
+      tbest = ts;
+      best = V3Plan{S, kc};
+    }
   }
+  return best;
+}
+
+// The block shape (index of t) of `batch` products.  nt: both operands contiguous along k, the
+// orientation that has 128x64 blocks.
+int v3_shape(bool nt, int64_t M, int64_t N, int64_t K, int64_t batch) {
+  double t[4];
+  v3_times(t, M, N, K, batch);
+  int best = 2;
+  for (int i : {1, 0, 3})
+    if (t[i] < t[best] && (i < 3 || nt)) best = i;
   return best;
 }
 
@@ -1098,7 +1117,7 @@ int launch(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const v
     return TG_ERR_UNSUPPORTED;
   }
   if (v3_ok((int)sizeof(T), ta, tb, M, N, K, A, lda, sa, B, ldb, sb, padded)) {
-    const int shape = v3_plan(M, N, K, batch, false).shape;
+    const int shape = v3_shape(!ta && tb, M, N, K, batch);
     // some batch entry's K ends inside a k-tile
     const bool ragged = K % V3_BK || (ktot != INT64_MAX && ktot % V3_BK);
 #define TG_G3_RUN(TA_, TB_, WGM, WGN, SM, SN, OCC, TAIL)                                     \
@@ -1128,6 +1147,7 @@ int launch(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const v
     else TG_G3_SHAPE(TA_, TB_, 2, 2, 2, 2, 2);                   \
   } while (0)
     if (!ta && !tb) TG_G3(false, false);
+    else if (!ta && tb && shape == 3) TG_G3_SHAPE(false, true, 2, 2, 2, 1, 2);
     else if (!ta && tb) TG_G3(false, true);
     else if (ta && !tb) TG_G3(true, false);
     else TG_G3(true, true);
@@ -1444,7 +1464,7 @@ SplitPlan split_plan(int dtype_ab, int64_t M, int64_t N, int64_t K) {
     p.rs = tg_gemm_rs_plan(M, N, K, 1, true);
     p.S = p.rs.S, p.kc = p.rs.kc;
   } else if (dtype_ab != TG_F64) {
-    const V3Plan v = v3_plan(M, N, K, 1, true);
+    const V3Plan v = v3_plan(M, N, K);
     p.S = v.S, p.kc = v.kc;
   }
   if (p.S > 1) p.bytes = al256((size_t)(p.S * split_stride(M * N)) * sizeof(float));
