@@ -1249,7 +1249,7 @@ int gemm_dispatch(const char* who, int dtype_ab, int dtype_c, int trans_a, int t
       return launch_f32(trans_a, trans_b, M, N, K, alpha, (const float*)A, lda, stride_a,
                         (const float*)B, ldb, stride_b, beta, (float*)C, ldc, stride_c, batch, s,
                         bias);
-    return tg_gemm_rs(tg_gemm_rs_plan(M, N, K, batch, false), trans_a, trans_b, M, N, K, alpha,
+    return tg_gemm_rs(tg_gemm_rs_plan(trans_a && !trans_b, M, N, K, batch, false), trans_a, trans_b, M, N, K, alpha,
                       (const float*)A, lda, stride_a, (const float*)B, ldb, stride_b, beta,
                       (float*)C, ldc, stride_c, batch, bias, s);
   }
@@ -1456,12 +1456,12 @@ struct SplitPlan {
   size_t bytes;
 };
 
-SplitPlan split_plan(int dtype_ab, int64_t M, int64_t N, int64_t K) {
+SplitPlan split_plan(int dtype_ab, bool tn, int64_t M, int64_t N, int64_t K) {
   SplitPlan p{};
   p.S = 1, p.kc = K;
   if (dtype_ab == TG_F32) {
     if (!tg_gemm_rs_serves(M, N, K, 1)) return p;
-    p.rs = tg_gemm_rs_plan(M, N, K, 1, true);
+    p.rs = tg_gemm_rs_plan(tn, M, N, K, 1, true);
     p.S = p.rs.S, p.kc = p.rs.kc;
   } else if (dtype_ab != TG_F64) {
     const V3Plan v = v3_plan(M, N, K);
@@ -1478,7 +1478,7 @@ struct WgradPlan {
 };
 
 WgradPlan wgrad_plan(int dtype_ab, int64_t M, int64_t N, int64_t K, bool has_b) {
-  WgradPlan p{split_plan(dtype_ab, M, N, K), 0, 0, pack_plan(dtype_ab, 1, 0, M, N, K)};
+  WgradPlan p{split_plan(dtype_ab, true, M, N, K), 0, 0, pack_plan(dtype_ab, 1, 0, M, N, K)};
   if (has_b) {
     p.bparts = al256((size_t)(p.sp.S * N) * sizeof(float));
     p.red = al256(tg_reduce_rows_workspace(K, N));
@@ -1491,7 +1491,7 @@ TG_EXPORT size_t tg_matmul_workspace(int dtype_ab, int trans_a, int trans_b, int
                                      int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const PackPlan pk = pack_plan(dtype_ab, trans_a, trans_b, M, N, K);
-  return split_plan(dtype_ab, M, N, K).bytes + pk.a + pk.b;
+  return split_plan(dtype_ab, trans_a && !trans_b, M, N, K).bytes + pk.a + pk.b;
 }
 
 TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int64_t M, int64_t N,
@@ -1499,7 +1499,9 @@ TG_EXPORT int tg_matmul(int dtype_ab, int dtype_c, int trans_a, int trans_b, int
                         int64_t ldb, const float* bias, float beta, void* C, int64_t ldc,
                         void* workspace, size_t workspace_bytes, void* stream) {
   const char* who = "tg_matmul";
-  const SplitPlan p = M > 0 && N > 0 && K > 0 ? split_plan(dtype_ab, M, N, K) : SplitPlan{};
+  const SplitPlan p = M > 0 && N > 0 && K > 0
+                          ? split_plan(dtype_ab, trans_a && !trans_b, M, N, K)
+                          : SplitPlan{};
   PackPlan pk = M > 0 && N > 0 && K > 0 ? pack_plan(dtype_ab, trans_a, trans_b, M, N, K)
                                         : PackPlan{};
   const size_t need = p.bytes + pk.a + pk.b;
@@ -1570,7 +1572,7 @@ TG_EXPORT int tg_gemm_wgrad(int dtype_ab, int64_t M, int64_t N, int64_t K, const
   void* red = ws + p.sp.bytes + p.bparts;
   if (ldw != N && p.sp.S > 1) {  // the split finish writes a dense dW
     p.sp.S = 1, p.sp.kc = K;
-    p.sp.rs = tg_gemm_rs_plan(M, N, K, 1, false);
+    p.sp.rs = tg_gemm_rs_plan(true, M, N, K, 1, false);
   }
   hipStream_t s = tg_stream(stream);
   const int64_t S = p.sp.S, kc = p.sp.kc, sc = split_stride(M * N);

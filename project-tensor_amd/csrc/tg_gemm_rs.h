@@ -21,8 +21,9 @@ inline bool tg_gemm_rs_serves(int64_t M, int64_t N, int64_t K, int64_t batch) {
 }
 
 // The fastest of the kernels for `batch` products of M x N x K, K split only where
-// can_split.
-TgRsPlan tg_gemm_rs_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool can_split);
+// can_split.  tn: A transposed, B plain.
+TgRsPlan tg_gemm_rs_plan(bool tn, int64_t M, int64_t N, int64_t K, int64_t batch,
+                         bool can_split);
 
 // C[z] = alpha * op(A[z]) @ op(B[z]) + beta * C[z] (+ bias) in fp32, any extents, leading
 // dimensions and alignment (element alignment is enough).  Without a split (p.S = 1) z

@@ -398,13 +398,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 2) void k_gemm_rs(
 // between wavefronts), then the partial tiles added in LDS in a fixed order.  Of every
 // 8 k, lane half h multiplies k + 4h .. k + 4h + 3 in four MFMAs (the same pairing for A
 // and B).
-constexpr int kSmallWaves = 16;
-template <bool TA, bool TB>
-__global__ __launch_bounds__(64 * kSmallWaves) void k_gemm_rs_small(
+// NW: 16, or 4 where lanes read along the rows of both operands (A transposed, B plain):
+// workgroups are smaller and more of them run, so a tile's sums and stores cost less.
+template <bool TA, bool TB, int NW>
+__global__ __launch_bounds__(64 * NW) void k_gemm_rs_small(
     int64_t M, int64_t N, int64_t K, int64_t ktot, float alpha, const float* __restrict__ A,
     int64_t lda, int64_t sa, const float* __restrict__ B, int64_t ldb, int64_t sb, float beta,
     float* __restrict__ C, int64_t ldc, int64_t sc, const float* __restrict__ bias) {
-  constexpr int NW = kSmallWaves;
   const int64_t bz = blockIdx.z;
   A += bz * sa;
   B += bz * sb;
@@ -438,8 +438,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void k_gemm_rs_small(
 #pragma unroll
   for (int r = 0; r < 16; ++r) red[wave][r][lane] = acc[r];
   __syncthreads();
-  {  // wave w finishes accumulator register w
-    const int r = wave;
+  for (int r = wave; r < 16; r += NW) {  // wave w finishes accumulator registers w, w + NW, ..
     float v = red[0][r][lane];
 #pragma unroll
     for (int w = 1; w < NW; ++w) v += red[w][r][lane];
@@ -478,7 +477,7 @@ int rs_launch(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t ktot, flo
   return tg_check_launch("tg_gemm");
 }
 
-enum { RS_256x128 = 0, RS_128x128, RS_64x64, RS_SMALL };
+enum { RS_256x128 = 0, RS_128x128, RS_64x64, RS_SMALL, RS_SMALL4 };
 
 }  // namespace
 
@@ -487,12 +486,14 @@ enum { RS_256x128 = 0, RS_128x128, RS_64x64, RS_SMALL };
 // 1.75 us (one block per CU each), 64x64 1.13 / 1.4 / 1.95 us with one / two / three
 // blocks per CU; a block's start and store take 3-4 us.  The small kernel takes 0.9 us
 // per 128 k plus 2.1 us for each block per CU (its operands come straight from the
-// caches).  A K split adds the finishing launch: 10 us, half of it
+// caches); with 4 waves, A transposed, 3 us and per k 0.012 plus 0.0063 for each tile per CU
+// (1722x370x427: 16 us, 64x64 blocks 26; 1114x632x784 26 and 40).  A K split adds the finishing launch: 10 us, half of it
 // the host's, and its traffic at 3.5 TB/s.
 // (Measured against the previous kernels, us: 8192x4096x1024 727 -> 402, 1024x4096x8192
 // with A transposed 1086 -> 399, 832x1664x8932 1210 -> 224, 1000^3 117 -> 37,
 // 448x256x32000 867 -> 72, 33x257x784 20 -> 15.)
-TgRsPlan tg_gemm_rs_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool can_split) {
+TgRsPlan tg_gemm_rs_plan(bool tn, int64_t M, int64_t N, int64_t K, int64_t batch,
+                         bool can_split) {
   TgRsPlan best{RS_256x128, 1, K};
   if (M <= 0 || N <= 0 || K <= 0 || batch <= 0) return best;
   const double ncu = (double)tg_num_cus();
@@ -508,15 +509,20 @@ TgRsPlan tg_gemm_rs_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool ca
     const double fin = S > 1 ? 10.0 + (double)(S + 1) * (double)M * (double)N * 4.0 / 3.5e6 : 0.0;
     // (a split's partial sums stay within 256 MiB)
     if (S > 1 && (double)S * (double)M * (double)N * 4.0 > 268435456.0) break;
-    double t[4];
+    double t[5];
     t[RS_256x128] = rounds(tiles(256, 128) * S) * (kt * 3.2 + 4.0);
     t[RS_128x128] = rounds(tiles(128, 128) * S) * (kt * 1.75 + 3.5);
     const double b64 = tiles(64, 64) * S, full = std::floor(b64 / (3 * ncu));
     const double rest = rounds(b64 - full * 3 * ncu);
     t[RS_64x64] = full * (kt * 1.95 + 3.0) +
                   (rest > 0 ? kt * (rest > 2 ? 1.95 : rest > 1 ? 1.4 : 1.13) + 3.0 : 0.0);
-    t[RS_SMALL] = (M + 31) / 32 > 65535 ? 1e30 : (double)((kc + 127) / 128) * (0.9 + 2.1 * tiles(32, 32) * S / ncu) + 3.0;
-    for (int i = 0; i < 4; ++i)
+    t[RS_SMALL] = t[RS_SMALL4] = 1e30;
+    if ((M + 31) / 32 <= 65535) {
+      const double per_cu = tiles(32, 32) * S / ncu;
+      t[RS_SMALL] = (double)((kc + 127) / 128) * (0.9 + 2.1 * per_cu) + 3.0;
+      if (tn && S == 1) t[RS_SMALL4] = (double)kc * (0.012 + 0.0063 * std::max(per_cu, 1.0)) + 3.0;
+    }
+    for (int i = 0; i < 5; ++i)
       if (t[i] + fin < tbest) {
         tbest = t[i] + fin;
         best = TgRsPlan{i, S, kc};
@@ -542,13 +548,14 @@ int tg_gemm_rs(const TgRsPlan& p, int ta, int tb, int64_t M, int64_t N, int64_t 
   }
 #undef TG_RSL
   const dim3 gs((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)batch);
-#define TG_SM(TA_, TB_)                                                                      \
-  k_gemm_rs_small<TA_, TB_><<<gs, 64 * kSmallWaves, 0, s>>>(M, N, kc, ktot, alpha, A, lda, sa, B, \
-                                                             ldb, sb, beta, C, ldc, sc, bias)
-  if (!ta && !tb) TG_SM(false, false);
-  else if (!ta) TG_SM(false, true);
-  else if (!tb) TG_SM(true, false);
-  else TG_SM(true, true);
+#define TG_SM(TA_, TB_, NW_)                                                                   \
+  k_gemm_rs_small<TA_, TB_, NW_><<<gs, 64 * NW_, 0, s>>>(M, N, kc, ktot, alpha, A, lda, sa, B, ldb, \
+                                                         sb, beta, C, ldc, sc, bias)
+  if (p.shape == RS_SMALL4) TG_SM(true, false, 4);
+  else if (!ta && !tb) TG_SM(false, false, 16);
+  else if (!ta) TG_SM(false, true, 16);
+  else if (!tb) TG_SM(true, false, 16);
+  else TG_SM(true, true, 16);
 #undef TG_SM
   return tg_check_launch("tg_gemm");
 }

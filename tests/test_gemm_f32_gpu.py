@@ -56,6 +56,13 @@ def test_matmul_f32(cuda, M, N, K, ta, tb):
         assert torch.allclose(y, c + bias, rtol=1e-6, atol=1e-6 * float(c.abs().max()) + 1e-6)
 
 
+@pytest.mark.parametrize("M,N,K", [(1722, 370, 427), (2049, 33, 65), (2081, 31, 7), (2064, 64, 32),
+                                   (1114, 632, 785)])
+def test_matmul_f32_transposed_small_output(cuda, M, N, K):
+    """A^T B of few 32 x 32 tiles: four wavefronts a tile, at its edges and k remainders."""
+    test_matmul_f32(cuda, M, N, K, True, False)
+
+
 @pytest.mark.parametrize("K,M,N", [(4561, 64, 64), (130, 33, 257), (8932, 130, 70), (77, 5, 3)])
 def test_wgrad_f32(cuda, K, M, N):
     g = torch.Generator(device="cuda").manual_seed(K)
