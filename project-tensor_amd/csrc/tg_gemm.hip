@@ -1346,11 +1346,11 @@ size_t al256(size_t n) { return (n + 255) & ~size_t{255}; }
 // ---- rows of other lengths: copies with aligned, zero-padded rows ----
 // The DMA-staged kernel needs rows of whole 16-byte chunks.  A 16-bit operand whose rows
 // are not (an odd vocabulary or hidden size) is copied into the workspace with its rows
-// padded by zeros; the copy streams once through memory (4096 x 50257: 180 us) where the
+// padded by zeros; the copy streams once through memory (2048 x 50257: 108 us) where the
 // element-wise staging of k_gemm costs the product most of its rate (4096 x 1024 x 50257:
-// 2440 us there).  Products too short for that stay on k_gemm: below 2^20 multiply-adds, or
-// with K < 192 below 2^31 (1429 x 1000 x 161: 18 us there, 21 with copies; 64 x 85 x 233: 20
-// and 15).
+// 2440 us there).  Products too short for that stay on k_gemm, which is one launch instead of two
+// (12 us of the host): below 2^20 multiply-adds, or with K < 96 below 2^28 (1310x497x19, A
+// transposed, 10 us there and 12 with copies; 9804x910x51 24 and 17; 73x153x117 14 and 12).
 struct PackArg {
   const void* src;
   uint4* dst;
@@ -1414,7 +1414,7 @@ PackPlan pack_plan(int dtype_ab, int ta, int tb, int64_t M, int64_t N, int64_t K
   PackPlan p{ta ? K : M, ta ? M : K, tb ? N : K, tb ? K : N, 0, 0};
   const double mnk = (double)M * (double)N * (double)K;
   if ((dtype_ab != TG_F16 && dtype_ab != TG_BF16) ||
-      mnk < (K < 192 ? 2147483648.0 : 1048576.0))
+      mnk < (K < 96 ? 268435456.0 : 1048576.0))
     return p;
   const double most = 4294967296.0 - kPackBlock;  // chunks that 32-bit indices count
   if ((double)p.ra * (double)((p.ca + 7) / 8) > most ||
