@@ -1011,6 +1011,9 @@ void v3_times(double (&t)[4], int64_t M, int64_t N, int64_t K, int64_t batch) {
   const double b3 = tiles(128, 64), full = std::floor(b3 / (3 * ncu)), r3 = b3 / ncu - 3 * full;
   const double c3 = r3 > 1 ? 0.3 + 0.33 * (r3 - 1) : 0.3;
   t[3] = full * (kt * 0.96 + 2.1) + (r3 > 0 ? kt * c3 + 3.7 : 0.0);
+  // (the instances for a partial k-tile hold a third more registers: 1917x3232x808 24.6 us by t[0]
+  // and 26.6 so, 2048x2048x616 12.0 and 13.4)
+  if (K % V3_BK) t[3] *= 1.15;
 }
 
 // The K split of a 16-bit product: batch entry s of S multiplies k in [s*kc, min(K, (s+1)*kc)).
