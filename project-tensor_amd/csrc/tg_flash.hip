@@ -2228,7 +2228,9 @@ __global__ __launch_bounds__(kThreads, OCC) void k_fa_bwd_dkdv_split(
 }
 
 template <typename T, int DP> struct FxOcc {
-  // workgroups per CU that the registers allow without spills
+  // workgroups per CU that the registers allow without spills; with 16-bit data also where a
+  // second one spills some (d 64 dK/dV, d above 96 dQ): one is slower (bf16 d 100, B*H 64, S 1024,
+  // causal, backward 429 us with two and 642 with one; d 64 236 and 236)
   static constexpr int FWD = sizeof(T) == 4 && DP > 64 ? 1 : 2;
   static constexpr int DQ = sizeof(T) == 4 && DP > 64 ? 1 : 2;
   static constexpr int DKDV = sizeof(T) == 4 ? (DP > 32 ? 1 : 2) : (DP > 64 ? 1 : 2);
